@@ -283,8 +283,8 @@ struct md_engine {
     bool vv_force_stale = false;   // the force array (velocity Verlet's first half kick) predates a PME change
     int pme_S = 0;                 // slot count the buffers were made for
     double pme_eself = 0, pme_qsum2 = 0;   // self term; (sum q)^2 for the background term
+    bool pme_small_q = true;       // every |q| < 2^18
     int pme_nconv = 0, pme_ngather = 0;
-    DBuf<unsigned long long> pme_qacc;
     DBuf<float> pme_qgrid;
     DBuf<float2> pme_sgrid, pme_tab;
     DBuf<float4> pme_frec;
@@ -684,7 +684,6 @@ int pme_prepare(md_engine* e) {
     const size_t n = (size_t)K[0] * K[1] * K[2], nh = (size_t)K[0] * K[1] * (K[2] / 2 + 1);
     e->pme_nconv = (int)std::min<size_t>((nh + 255) / 256, 2048);
     e->pme_ngather = (e->S + 63) / 64;   // 4 lanes per slot, 256 lanes per workgroup
-    CHECK(e->pme_qacc.alloc(n));
     CHECK(e->pme_qgrid.alloc(n));
     CHECK(e->pme_sgrid.alloc(nh));
     CHECK(e->pme_tab.alloc((size_t)K[0] + K[1] + K[2]));
@@ -710,7 +709,9 @@ int pme_prepare(md_engine* e) {
     HIPCHECK(hipMemcpy(e->pme_tab.p, tab.data(), tab.size() * sizeof(float2), hipMemcpyHostToDevice));
     // self and neutralizing-background terms
     double s1 = 0.0, s2 = 0.0;
+    e->pme_small_q = true;
     for (int i = 0; i < e->N; i++) {
+        if (!(std::fabs(e->charge_h[i]) < 262144.0f)) e->pme_small_q = false;
         s1 += e->charge_h[i];
         s2 += (double)e->charge_h[i] * e->charge_h[i];
     }
@@ -740,7 +741,7 @@ int pme_prepare(md_engine* e) {
 PmeArgs pme_args(md_engine* e, int mode) {
     PmeArgs g{};
     g.pos[0] = e->pos[0].p; g.pos[1] = e->pos[1].p; g.ids = e->ids.p; g.slot_of = e->slot_of.p; g.excl = e->excl.p;
-    g.st = e->rst.p; g.qacc = e->pme_qacc.p; g.qgrid = e->pme_qgrid.p; g.sgrid = e->pme_sgrid.p; g.tab = e->pme_tab.p;
+    g.st = e->rst.p; g.cell_rank = e->cell_rank.p; g.cell_start = e->cell_start.p; g.qgrid = e->pme_qgrid.p; g.sgrid = e->pme_sgrid.p; g.tab = e->pme_tab.p;
     g.frec = e->pme_frec.p; g.part = e->pme_part.p; g.out = e->pme_out.p;
     g.K0 = e->pme_K[0]; g.K1 = e->pme_K[1]; g.K2 = e->pme_K[2]; g.order = e->pme_order;
     g.nslot = e->S; g.mode = mode; g.has_excl = e->has_excl ? 1 : 0;
@@ -752,6 +753,11 @@ PmeArgs pme_args(md_engine* e, int mode) {
     g.qfac = e->ff.qfac;
     g.pi2_b2 = (float)(pi * pi / (beta * beta));
     g.e_self = e->pme_eself; g.qsum2 = e->pme_qsum2;
+    g.margin = 0.5f * e->ff.skin * 1.0001f + 2e-3f;
+    g.small_q = e->pme_small_q ? 1 : 0;
+    g.baro = e->in.barostat != MD_BARO_NONE ? 1 : 0;
+    g.rl = std::sqrt(e->rl2);
+    g.rc = e->ff.rc;
     return g;
 }
 

@@ -234,10 +234,10 @@ struct StepArgs {
 };
 
 // Smooth particle-mesh Ewald for one replica (pme.hip), a chain of kernels and
-// two FFTs before each step kernel: spread the charges onto the grid (fixed
-// point, so the sum does not depend on the order of the atomic adds), convert,
-// transform, multiply by the influence function (energy and virial on the
-// way), transform back, gather the forces.
+// two FFTs before each step kernel: spread the charges onto the grid (in fixed
+// point, so the sum does not depend on the order of the adds), transform,
+// multiply by the influence function (energy and virial on the way), transform
+// back, gather the forces.
 #define MD_PME_MAX_ORDER 8
 #define MD_PME_QUNIT 4294967296.0   // fixed-point units per charge unit in the spread grid
 struct PmeArgs {
@@ -246,7 +246,8 @@ struct PmeArgs {
     const int* slot_of;         // [N]
     const int4* excl;           // [N] excluded partners (-1 empty)
     const RepState* st;         // the replica (one)
-    unsigned long long* qacc;   // [K0 K1 K2] charge grid in fixed point, zero between steps
+    const int* cell_rank;       // the cells of the last list build: linear cell -> curve rank,
+    const int* cell_start;      // and first slot by rank (the atoms of a cell are consecutive slots)
     float* qgrid;               // [K0 K1 K2] charges (transform input); dE/dQ (inverse output)
     float2* sgrid;              // [K0 K1 (K2/2 + 1)] the transform
     const float2* tab;          // [K0 + K1 + K2] per axis and index: (signed frequency m, |b(m)|^2)
@@ -266,6 +267,10 @@ struct PmeArgs {
     float pi2_b2;               // pi^2 / beta^2
     double e_self;              // -qfac beta / sqrt(pi) sum q^2
     double qsum2;               // (sum q)^2: the neutralizing-background term -qfac pi qsum2 / (2 V beta^2)
+    float margin;               // most an atom can have moved since the list build (skin / 2, rounded up)
+    int small_q;                // every |q| < 2^18: a weighted charge's fixed point fits 52 bits
+    int baro;                   // pressure coupling: the box (and the margin) follow the scale since the build
+    float rl, rc;
 };
 
 // Progress of a run for the host: one small copy per check instead of one per

@@ -8,11 +8,9 @@
 // the long-range energy and virial to the replica's first tile):
 //   k_pme_spread  the order-p B-spline weights of each atom's scaled coordinates
 //                 u = K (x / L + 1/2) (in FP64, so the weights carry only FP32
-//                 rounding), p^3 64-bit fixed-point atomic adds of q th_x th_y th_z
-//                 into the charge grid by a wavefront per atom: integer sums, so the
-//                 grid does not depend on the order of the adds and runs repeat bit
-//                 for bit
-//   k_pme_fix     fixed point -> float, clearing the fixed-point grid for the next step
+//                 rounding), q th_x th_y th_z summed per brick of the grid in LDS in
+//                 64-bit fixed point: integer sums, so the grid does not depend on the
+//                 order of the adds and runs repeat bit for bit
 //   R2C FFT       (hipFFT, on the engine's stream, its work area allocated up front)
 //   k_pme_conv    multiply by the influence function C(m) = qfac exp(-pi^2 m^2/b^2)
 //                 B(m) / (pi V m^2), summing the energy 1/2 C |S|^2 and the traced
@@ -107,75 +105,227 @@ __device__ __forceinline__ PmeBox pme_box(const PmeArgs& a) {
     return b;
 }
 
-// Lane l of a wavefront first computes the stencil of slot (wavefront's base + l);
-// then the wavefront walks its 64 atoms, its lanes taking the atom's P^3 grid
-// points with the z index fastest, so each atomic instruction touches P^2 runs of
-// P consecutive grid words instead of 64 scattered ones (atomics are combined
-// per cache line on the way to L2).
-template <int P>
-__global__ __launch_bounds__(PT) void k_pme_spread(const PmeArgs a) {
-    const RepState s = a.st[0];
-    if (!pme_go(s, a.mode)) return;   // grid-uniform
-    const int lane = threadIdx.x & 63;
-    const int slot = blockIdx.x * PT + threadIdx.x;
-    float q = 0.0f;
-    int k0 = 0, k1 = 0, k2 = 0;
-    float t0[P], t1[P], t2[P];
-#pragma unroll
-    for (int c = 0; c < P; c++) t0[c] = t1[c] = t2[c] = 0.0f;
-    if (slot < a.nslot && a.ids[slot] >= 0) {
-        const PmeBox bx = pme_box(a);
-        const float4 x = a.pos[cur_buf(s)][slot];
-        q = x.w;
-        float w0, w1, w2;
-        grid_coord(x.x, bx.hl[0], bx.kl[0], a.ik0, a.K0, k0, w0);
-        grid_coord(x.y, bx.hl[1], bx.kl[1], a.ik1, a.K1, k1, w1);
-        grid_coord(x.z, bx.hl[2], bx.kl[2], a.ik2, a.K2, k2, w2);
-        bspline<P, false>(w0, t0, nullptr);
-        bspline<P, false>(w1, t1, nullptr);
-        bspline<P, false>(w2, t2, nullptr);
-#pragma unroll
-        for (int c = 0; c < P; c++) t0[c] *= q;   // the charge rides on the x weights
+// Charge spreading, one workgroup per brick of SB0 x SB1 x SB2 grid points summed in
+// LDS.  The bricks tile the grid, so every grid point is written once, as float:
+// no clearing, no device-scope atomics and no separate conversion pass.
+//  1. The cells of the last list build that can hold an atom touching the brick
+//     (its points grown by the spline's support and by a.margin, the most an atom
+//     can have moved since the build) are tabulated, their atoms tested, and those
+//     in reach collected in LDS (in any order: the sums are integers).
+//  2. The collected atoms' weights are computed, a lane per atom.
+//  3. A lane per (atom, x point, y point) adds its run of P z points that lie in
+//     the brick, in 64-bit fixed point: the same sums bit for bit whatever the order.
+// The z rows in LDS are padded by one word against bank conflicts.
+// Bound by latency at 96^3 (the chain state -> cells -> atoms -> weights -> adds, once
+// per brick) and by the LDS adds and their addresses at 128^3.  A wavefront per atom
+// with one 8-byte global atomic per stencil point, then a conversion pass, took 30 + 5.5
+// us for 32,768 ions on 96^3 and 161 + 7.4 us for 196,608 water atoms on 128^3 (the
+// device's atomic units); this takes 11.4 and 28.6 us for the same grids bit for bit.
+// Brick and workgroup were swept: 8 x 8 x 16 with 256 threads gives 12.0 and 31.1,
+// 16 x 8 x 32 with 512 threads 12.1 and 24.8 but 15.6 instead of 10.5 us for 6,591 atoms
+// on 45^3 (27 bricks), 8 x 8 x 8 with 256 threads 15.8 and 39.6.
+constexpr int SB0 = 16, SB1 = 8, SB2 = 16, SBZ = SB2 + 1, ST = 512;   // ST threads per brick
+constexpr int SU = 4;                 // candidates a thread tests at once (their loads in flight together)
+constexpr int SLIST = (SU + 1) * ST;  // collected atoms: up to ST - 1 pending and SU ST new ones
+
+// fixed point (units of 2^-32) of f, rounded to nearest even.  small: |f| < 2^19, where
+// the rounding falls out of one FP64 fma (the integer is the low 52 bits).
+__device__ __forceinline__ long long to_fixed(float f, bool small) {
+    if (small) {
+        const double magic = 6755399441055744.0;   // 1.5 * 2^52
+        return __double_as_longlong(fma((double)f, MD_PME_QUNIT, magic)) - __double_as_longlong(magic);
     }
-    unsigned long long todo = __ballot(q != 0.0f);
-    while (todo) {
-        const int t = __builtin_ctzll(todo);   // wavefront-uniform
-        todo &= todo - 1;
-        const int b0 = __builtin_amdgcn_readlane(k0, t), b1 = __builtin_amdgcn_readlane(k1, t),
-                  b2 = __builtin_amdgcn_readlane(k2, t);
-        float u0[P], u1[P], u2[P];
-#pragma unroll
-        for (int c = 0; c < P; c++) {
-            u0[c] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(t0[c]), t));
-            u1[c] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(t1[c]), t));
-            u2[c] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(t2[c]), t));
-        }
-#pragma unroll
-        for (int p0 = 0; p0 < P * P * P; p0 += 64) {
-            const int p = p0 + lane;
-            if (P * P * P % 64 != 0 && p >= P * P * P) break;
-            const int i = p / (P * P), j = (p / P) % P, c = p % P;
-            float wx = u0[0], wy = u1[0], wz = u2[0];
-#pragma unroll
-            for (int m = 1; m < P; m++) {
-                wx = i == m ? u0[m] : wx;
-                wy = j == m ? u1[m] : wy;
-                wz = c == m ? u2[m] : wz;
-            }
-            const size_t idx = ((size_t)wrapk(b0 - i, a.K0) * a.K1 + wrapk(b1 - j, a.K1)) * a.K2 + wrapk(b2 - c, a.K2);
-            const long long v = __double2ll_rn((double)(wx * wy * wz) * MD_PME_QUNIT);
-            atomicAdd(a.qacc + idx, (unsigned long long)v);
-        }
-    }
+    return __double2ll_rn((double)f * MD_PME_QUNIT);
 }
 
-__global__ __launch_bounds__(PT) void k_pme_fix(const PmeArgs a) {
-    if (!pme_go(a.st[0], a.mode)) return;
-    const size_t n = (size_t)a.K0 * a.K1 * a.K2;
-    for (size_t i = (size_t)blockIdx.x * PT + threadIdx.x; i < n; i += (size_t)gridDim.x * PT) {
-        const long long v = (long long)a.qacc[i];
-        a.qacc[i] = 0ull;
-        a.qgrid[i] = (float)((double)v * (1.0 / MD_PME_QUNIT));
+// cells of one axis that can hold an atom whose stencil meets grid points [g0, g0 + b)
+struct CellSpan {
+    int lo, n, nc;
+    __device__ int at(int k) const { const int c = lo + k; return c >= nc ? c - nc : c; }
+};
+__device__ __forceinline__ CellSpan cell_span(int g0, int b, int P, float h, float margin, float cinv, int nc) {
+    const float lo = (float)g0 * h - margin, hi = (float)(g0 + b + P - 1) * h + margin;
+    CellSpan c;
+    c.nc = nc;
+    const int l = (int)floorf(lo * cinv), r = (int)floorf(hi * cinv);
+    if (r - l + 1 >= nc) {
+        c.lo = 0;
+        c.n = nc;
+    } else {
+        c.lo = l < 0 ? l + nc : (l >= nc ? l - nc : l);
+        c.n = r - l + 1;
+    }
+    return c;
+}
+
+template <int P>
+__global__ __launch_bounds__(ST) void k_pme_spread(const PmeArgs a) {
+    __shared__ unsigned long long s_acc[SB0 * SB1 * SBZ];
+    __shared__ int s_at[SLIST];                          // slots of the collected atoms
+    __shared__ float s_w[3][ST][P];                  // weights of the atoms being added
+    __shared__ uint32_t s_k[ST];                         // their grid indices relative to the brick, 10 bits each
+    __shared__ int s_start[ST], s_pref[ST + 1], s_wsum[ST / 64], s_cnt;
+    const RepState s = a.st[0];
+    const RepParam p = a.rep[0];      // in the state's round trip
+    loads_issued();
+    if (!pme_go(s, a.mode)) return;   // grid-uniform
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const PmeBox bx = pme_box(a);
+    const float4* __restrict__ pin = a.pos[cur_buf(s)];
+    const int nb1 = (a.K1 + SB1 - 1) / SB1, nb2 = (a.K2 + SB2 - 1) / SB2;
+    const int blk = xcd_block(blockIdx.x, gridDim.x);
+    const int g2 = blk % nb2 * SB2, g1 = blk / nb2 % nb1 * SB1, g0 = blk / (nb2 * nb1) * SB0;
+    const int n0 = min(SB0, a.K0 - g0), n1 = min(SB1, a.K1 - g1), n2 = min(SB2, a.K2 - g2);
+    for (int k = tid; k < SB0 * SB1 * SBZ; k += ST) s_acc[k] = 0ull;
+    if (tid == 0) s_cnt = 0;
+    float margin = a.margin;
+    if (a.baro) {
+        // scaled box (pressure coupling): an atom moved by less than (min m r_list - r_c) / 2
+        // from its scaled build position, m = L / Lb, at the scale before the last
+        // rescaling, which at most halves the box
+        const float m = fminf(bx.L[0] / p.Lb[0], fminf(bx.L[1] / p.Lb[1], bx.L[2] / p.Lb[2]));
+        margin = fmaxf(margin, 0.5f * (m * a.rl - 0.5f * a.rc) + 2e-3f);
+    }
+    const CellSpan c0 = cell_span(g0, n0, P, bx.L[0] / (float)a.K0, margin, p.cinv[0], p.nc[0]);
+    const CellSpan c1 = cell_span(g1, n1, P, bx.L[1] / (float)a.K1, margin, p.cinv[1], p.nc[1]);
+    const CellSpan c2 = cell_span(g2, n2, P, bx.L[2] / (float)a.K2, margin, p.cinv[2], p.nc[2]);
+    const int ncell = c0.n * c1.n * c2.n;
+    // FP32 reach test: floor(u) - g mod K below n + P - 1, with 0.01 of slack on both
+    // sides (the points are tested exactly in step 3)
+    const float kf[3] = {(float)a.K0, (float)a.K1, (float)a.K2};
+    const float sc[3] = {(float)bx.kl[0], (float)bx.kl[1], (float)bx.kl[2]};
+    const float gf[3] = {(float)g0, (float)g1, (float)g2};
+    const float rf[3] = {(float)(n0 + P - 1), (float)(n1 + P - 1), (float)(n2 + P - 1)};
+    auto reach = [&](float x, int d) {
+        const float t = fmaf(x, sc[d], 0.5f * kf[d]) - gf[d] + 0.01f;
+        const float r = t - kf[d] * floorf(t / kf[d]);
+        return r < rf[d] + 0.02f;
+    };
+    const bool wr0 = a.K0 < n0 + P - 1, wr1 = a.K1 < n1 + P - 1, wr2 = a.K2 < n2 + P - 1;
+    int pend = 0;   // collected atoms not yet added (workgroup-uniform)
+    // add n (at most ST) collected atoms, from the list's entry base on, to the brick
+    auto add = [&](int base, int n) {
+        if (tid < n) {
+            const float4 x = pin[s_at[base + tid]];
+            int k0, k1, k2;
+            float w0, w1, w2, t0[P], t1[P], t2[P];
+            grid_coord(x.x, bx.hl[0], bx.kl[0], a.ik0, a.K0, k0, w0);
+            grid_coord(x.y, bx.hl[1], bx.kl[1], a.ik1, a.K1, k1, w1);
+            grid_coord(x.z, bx.hl[2], bx.kl[2], a.ik2, a.K2, k2, w2);
+            bspline<P, false>(w0, t0, nullptr);
+            bspline<P, false>(w1, t1, nullptr);
+            bspline<P, false>(w2, t2, nullptr);
+#pragma unroll
+            for (int c = 0; c < P; c++) {
+                s_w[0][tid][c] = t0[c] * x.w;   // the charge rides on the x weights
+                s_w[1][tid][c] = t1[c];
+                s_w[2][tid][c] = t2[c];
+            }
+            const uint32_t r0 = (uint32_t)wrapk(k0 - g0, a.K0), r1 = (uint32_t)wrapk(k1 - g1, a.K1),
+                           r2 = (uint32_t)wrapk(k2 - g2, a.K2);
+            s_k[tid] = r0 | (r1 << 10) | (r2 << 20);
+        }
+        __syncthreads();
+        for (int u = tid; u < n * P * P; u += ST) {
+            const int t = u / (P * P), ij = u % (P * P), i = ij / P, j = ij % P;
+            const uint32_t k = s_k[t];
+            // point v of the brick, or out of range; an axis shorter than the brick and the
+            // spline's support (wrap) meets the brick from both sides
+            auto point = [](uint32_t r, int c, int K, bool wrap) {
+                int v = (int)r - c;
+                if (wrap) v = wrapk(v, K);
+                return (uint32_t)v;
+            };
+            const uint32_t v0 = point(k & 1023u, i, a.K0, wr0), v1 = point((k >> 10) & 1023u, j, a.K1, wr1);
+            if (v0 < (uint32_t)n0 && v1 < (uint32_t)n1) {
+                const float wxy = s_w[0][t][i] * s_w[1][t][j];
+                float wz[P];
+#pragma unroll
+                for (int c = 0; c < P; c++) wz[c] = s_w[2][t][c];
+                unsigned long long* row = s_acc + (v0 * SB1 + v1) * SBZ;
+#pragma unroll
+                for (int c = 0; c < P; c++) {
+                    const uint32_t v2 = point(k >> 20, c, a.K2, wr2);
+                    if (v2 < (uint32_t)n2) atomicAdd(row + v2, (unsigned long long)to_fixed(wxy * wz[c], a.small_q != 0));
+                }
+            }
+        }
+    };
+    for (int b = 0; b < ncell; b += ST) {
+        int cs = 0, cn = 0;
+        if (b + tid < ncell) {
+            const int c = b + tid, w2 = c % c2.n, w1 = c / c2.n % c1.n, w0 = c / (c2.n * c1.n);
+            const int r = a.cell_rank[c0.at(w0) + p.nc[0] * (c1.at(w1) + p.nc[1] * c2.at(w2))];
+            cs = a.cell_start[r];
+            cn = a.cell_start[r + 1] - cs;
+        }
+        int inc = cn;
+        for (int o = 1; o < 64; o <<= 1) {
+            const int t = __shfl_up(inc, o, 64);
+            if (lane >= o) inc += t;
+        }
+        if (lane == 63) s_wsum[wave] = inc;
+        __syncthreads();
+        int off = inc - cn, T = 0;
+#pragma unroll
+        for (int w = 0; w < ST / 64; w++) {
+            if (w < wave) off += s_wsum[w];
+            T += s_wsum[w];
+        }
+        s_start[tid] = cs;
+        s_pref[tid] = off;
+        if (tid == 0) s_pref[ST] = T;
+        __syncthreads();
+        for (int q0 = 0; q0 < T; q0 += SU * ST) {
+            int slot[SU];
+            float4 x[SU];
+#pragma unroll
+            for (int u = 0; u < SU; u++) {
+                const int q = min(q0 + u * ST + tid, T - 1);
+                int lo = 0;   // last cell with pref <= q
+#pragma unroll
+                for (int h = ST / 2; h >= 1; h >>= 1) lo += s_pref[lo + h] <= q ? h : 0;
+                slot[u] = s_start[lo] + (q - s_pref[lo]);
+            }
+#pragma unroll
+            for (int u = 0; u < SU; u++) x[u] = pin[slot[u]];
+#pragma unroll
+            for (int u = 0; u < SU; u++) {
+                const bool hit = q0 + u * ST + tid < T && x[u].w != 0.0f && reach(x[u].x, 0) && reach(x[u].y, 1) &&
+                                 reach(x[u].z, 2);
+                const unsigned long long m = __ballot(hit);
+                if (m == 0) continue;   // wavefront-uniform
+                int at = 0;
+                if (lane == 0) at = atomicAdd(&s_cnt, (int)__popcll(m));
+                at = __builtin_amdgcn_readfirstlane(at);
+                if (hit) s_at[at + (int)__popcll(m & ((1ull << lane) - 1ull))] = slot[u];
+            }
+            __syncthreads();
+            pend = s_cnt;
+            int base = 0;
+            while (pend >= ST) {   // workgroup-uniform
+                add(base, ST);
+                __syncthreads();
+                base += ST;
+                pend -= ST;
+            }
+            if (base > 0) {   // the atoms past the added ones move to the front
+                const int k = tid < pend ? s_at[base + tid] : 0;
+                __syncthreads();
+                if (tid < pend) s_at[tid] = k;
+                if (tid == 0) s_cnt = pend;
+            }
+            __syncthreads();
+        }
+    }
+    if (pend > 0) add(0, pend);
+    __syncthreads();
+    for (int k = tid; k < SB0 * SB1 * SB2; k += ST) {
+        const int z = k % SB2, y = k / SB2 % SB1, x = k / (SB2 * SB1);
+        if (x < n0 && y < n1 && z < n2) {
+            const long long v = (long long)s_acc[(x * SB1 + y) * SBZ + z];
+            a.qgrid[((size_t)(g0 + x) * a.K1 + g1 + y) * a.K2 + g2 + z] = (float)((double)v * (1.0 / MD_PME_QUNIT));
+        }
     }
 }
 
@@ -374,7 +524,8 @@ __global__ __launch_bounds__(PT) void k_pme_sum(const PmeArgs a) {
 
 template <int P>
 void launch_spread(const PmeArgs& a, hipStream_t st) {
-    hipLaunchKernelGGL(k_pme_spread<P>, dim3((a.nslot + PT - 1) / PT), dim3(PT), 0, st, a);
+    const int nb = ((a.K0 + SB0 - 1) / SB0) * ((a.K1 + SB1 - 1) / SB1) * ((a.K2 + SB2 - 1) / SB2);
+    hipLaunchKernelGGL(k_pme_spread<P>, dim3(nb), dim3(ST), 0, st, a);
 }
 
 template <int P>
@@ -392,9 +543,6 @@ extern "C" int md_launch_pme(const PmeArgs& a, hipfftHandle r2c, hipfftHandle c2
     case 8: launch_spread<8>(a, st); break;
     default: return 1;
     }
-    const size_t n = (size_t)a.K0 * a.K1 * a.K2;
-    const int nfix = (int)std::min<size_t>((n + PT - 1) / PT, 4096);
-    hipLaunchKernelGGL(k_pme_fix, dim3(nfix), dim3(PT), 0, st, a);
     if (hipGetLastError() != hipSuccess) return 1;
     if (hipfftExecR2C(r2c, a.qgrid, reinterpret_cast<hipfftComplex*>(a.sgrid)) != HIPFFT_SUCCESS) return 2;
     hipLaunchKernelGGL(k_pme_conv, dim3(a.nconv), dim3(PT), 0, st, a);

@@ -93,6 +93,43 @@ def test_forces_nacl(E, orc, grid, order):
     check_forces(E, orc, s)
 
 
+@pytest.mark.parametrize("cell_div", [1, 2, 3])
+@pytest.mark.parametrize("grid,order", [((4, 4, 4), 4), ((8, 16, 17), 4), ((9, 33, 15), 6), ((8, 8, 48), 8)])
+def test_forces_brick_edges(E, orc, grid, order, cell_div):
+    """The spread kernel's bricks (8 x 8 x 16 grid points) at their edges: a grid of one
+    clipped brick whose stencils wrap onto themselves, exact multiples, one point over
+    and one short, with each cell size of the list the bricks find their atoms by, after
+    steps that move the atoms away from their cells (600 to 5,000 atoms per brick, so the
+    collected atoms are added in several passes)."""
+    s = nacl_pme(grid=grid, order=order)
+    say("pme forces brick edges", s.pme, "cell_div", cell_div)
+    e = E.Engine.from_system(s)
+    e.set_launch(cell_div=cell_div)
+    e.run(5, stats=False)
+    so = s.copy()
+    so.pos = e.download()[0]
+    F, _, _ = e.compute_forces()
+    Fo, _, _ = orc.forces(so)
+    e.close()
+    assert rel_rms(F, Fo) < FORCE_TOL
+
+
+def test_forces_large_charges(E, orc):
+    """Charges beyond 2^18 e take the spread's full-range fixed point: the forces of NaCl with
+    charges of 3e5 e (the pair law scaled back by qfac) equal the oracle's."""
+    s = nacl_pme(nsites=12)
+    s.charge = (s.charge * np.float32(3.0e5)).astype(np.float32)
+    s.ff = dataclasses.replace(s.ff, qfac=s.ff.qfac / 9.0e10)
+    say("pme forces large charges", s.pme)
+    e = E.Engine.from_system(s)
+    so = s.copy()
+    so.pos = e.download()[0]
+    F, _, _ = e.compute_forces()
+    Fo, _, _ = orc.forces(so)
+    e.close()
+    assert rel_rms(F, Fo) < FORCE_TOL
+
+
 def test_forces_orthorhombic_box(E, orc):
     """Box edges 49.6, 45.1 and 42.9 A (the rock-salt lattice stretched per axis)
     on a 50 x 45 x 44 grid: every per-axis scale (grid coordinates, reciprocal
