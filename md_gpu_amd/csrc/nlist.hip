@@ -15,22 +15,24 @@
 //   k_nl_permute  deterministic order inside a cell (by eighth of the cell, then
 //                 original index); gathers pos/vel/force/id/type into scratch in the
 //                 new order, positions wrapped into the box
-//   k_nl_tbuild   one workgroup per 64-slot tile: the image cells within r_list of
-//                 the tile's bounding box are listed in LDS, their members streamed
-//                 through an LDS ring and tested against the tile's atoms with the
-//                 canonical FP32 predicate.  Candidates that some atom of the tile
-//                 hits form the tile's neighbor set (in candidate order); each atom's
-//                 row holds 16-bit indices into that set, in candidate order, so rows
-//                 are deterministic.  Each tile stores its longest row and set size.
+//   k_nl_tbuild   one workgroup per 64-slot tile: the members of the image cells within
+//                 r_list of the tile's bounding box are streamed through LDS and tested
+//                 against the tile's atoms with the canonical FP32 predicate.  Candidates
+//                 that some atom of the tile hits form the tile's neighbor set (in
+//                 candidate order); each atom's row holds 16-bit indices into that set, in
+//                 candidate order, so rows are deterministic.  Each tile stores its longest
+//                 row and set size.
 //   k_nl_commit   per rebuilt replica: new list epoch (or the next step kernel opens it).
 // Bytes per atom per rebuild (algorithmic): read pos/vel/force/id/type 56 B,
 // write them twice (scratch + copy back) 112 B, plus the rows 2*K B and the
 // tile sets (4 B per set entry, about 4*K/16 B per atom).
+#include <type_traits>
+
 #include "md_device.h"
 
 namespace {
 
-constexpr int kTab = 1024;    // region cells per table batch
+constexpr int kTab = 512;     // region cells per table batch
 
 __device__ __forceinline__ int cell_coord(float x, float halfL, float cinv, int nc) {
     int k = (int)floorf((x + halfL) * cinv);
@@ -101,6 +103,13 @@ __device__ int block_scan(int v, int* s_w, int& total) {
     __syncthreads();
     return off + inc - v;
 }
+
+// old with lane n's value replaced by the wavefront-uniform v (no builtin: the LLVM intrinsic by name)
+extern "C" __device__ int md_writelane(int v, int n, int old) __asm("llvm.amdgcn.writelane.i32");
+__device__ __forceinline__ int writelane(int v, int n, int old) { return md_writelane(v, n, old); }
+
+// second hash of an original index into the tile build's 16,384-bit exclusion filter
+__device__ __forceinline__ uint32_t excl_hash(int id) { return ((uint32_t)id * 2654435761u) >> 18; }
 
 }  // namespace
 
@@ -249,36 +258,47 @@ __global__ __launch_bounds__(256) void k_nl_permute(BuildArgs a) {
     a.slot_of[myid] = f;
 }
 
-// Tile neighbor-set build: one workgroup of NW wavefronts (4 or 8) per 64-slot
-// tile, 64 / NW atoms per wavefront (held as wavefront-uniform values).  The set
-// and rows do not depend on NW: four wavefronts (more workgroups resident per CU
-// to overlap the latency-bound candidate streaming) build the same lists as eight.
-//  1. The image cells within r_list of the tile's bounding box are listed in LDS
-//     (region order, two-pass block scan), in batches of kTab region cells.
-//  2. Their members are streamed 64 NW per chunk (a thread per candidate); those
-//     whose image lies r_list or farther from the box are dropped, the rest are
-//     appended to an LDS ring in candidate order (stable block compaction).
-//  3. Every 64 ring entries, each wavefront tests the 64 candidates (a lane each)
-//     against its 8 atoms with the canonical predicate; a candidate that hits any
-//     atom of the tile gets the next local index of the tile's set (the OR of the
-//     wavefronts' hit masks goes through LDS, one barrier per 64 candidates), and
-//     each atom's hits are appended to its row at count + (hits in lower lanes).
+// Tile neighbor-set build: one workgroup of 8 wavefronts per 64-slot tile, 8 atoms (a
+// group of consecutive slots, so a compact one) per wavefront, their positions held as
+// wavefront-uniform values.
+//  1. The image cells within r_list of the tile's bounding box (region order, kTab cells a
+//     round, a thread per cell) write their members' slots to LDS, 512 per chunk.
+//  2. A thread per candidate finds the groups whose bounding box its image is within r_list of.
+//  3. Each wavefront lists the chunk's candidates in reach of its group (in candidate
+//     order) and tests them, 64 at a time (a lane each), against its 8 atoms with the
+//     canonical predicate; the hit masks stay in registers (a lane per atom and 64
+//     candidates).  A candidate that hits any atom of the tile gets the next local index
+//     of the tile's set, and each atom's hits are appended to its row, first in LDS, then
+//     64 entries at a time to memory in one contiguous store.
 // So set and rows follow candidate order and do not depend on scheduling.
-template <bool EXCL, int NW>
-__global__ __launch_bounds__(64 * NW, (NW == 4 && !EXCL) ? 5 : 1) void k_nl_tbuild(BuildArgs a) {
-    constexpr int NT = 64 * NW, AW = 64 / NW, RING = 1024, PER = kTab / NT;
-    __shared__ int s_tstart[kTab];        // first slot of the cell
-    __shared__ int s_tpref[kTab + 1];     // first candidate index of each table row; [ntab] = total
-    __shared__ int s_tcode[kTab];         // image shift code of the cell
-    __shared__ float4 s_cx[RING];         // ring: candidate position (unshifted), w = bits of the set entry
-    __shared__ int s_cid[EXCL ? RING : 1];   // original index of the candidate (exclusions)
+//
+// Bound by VALU issue (72 % busy; 7 instructions per atom and 64 candidates for the test, 7
+// for the append, 4 to keep the mask in between), the rest barriers and load latency; at
+// 32,768 ions two tiles per CU leave it latency-bound.  A full build (us): 196,608 water
+// atoms 397 (660 before), 32,768 ions 77 (89), 512 Ar-Xe replicas 912 (1,065), 64 replicas
+// 151 (211).  Before, every wavefront tested every candidate of the tile (a barrier per 64
+// of them), tested self and exclusions per atom and stored hits to memory 2 bytes at a
+// time; a group's own candidates are under half of the tile's.  Groups by bounding sphere
+// instead of box: 480 us (water).  80 registers keep three workgroups per CU (unbounded,
+// 114: one workgroup fewer, 542 us); 64 spill (500 us).
+template <bool EXCL>
+__global__ __launch_bounds__(512, 6) void k_nl_tbuild(BuildArgs a) {
+    constexpr int NW = 8, NT = 64 * NW, AW = 64 / NW;
+    __shared__ uint32_t s_cand[NT];       // the next chunk's candidates: slot | image shift code << 24
+    __shared__ float4 s_cx[NT];           // the chunk: candidate position (unshifted), w = bits of the set entry
+    __shared__ int s_cid[EXCL ? NT : 1];  // original index of the candidate (exclusions), bit 31: may be excluded
+    __shared__ uint2 s_gm[NW][NW];        // [wavefront of the candidates][group]: those in reach of the group
+    __shared__ uint8_t s_hit[NT];         // the candidate hit some atom of the tile
+    __shared__ uint16_t s_li[NT];         // row entry of a candidate of the set
+    __shared__ uint16_t s_list[NW][NT];   // per wavefront the chunk's candidates in reach of its group
+    __shared__ uint16_t s_row[64][128];   // per atom the row entries not yet stored (ring by entry mod 128)
+    __shared__ uint32_t s_bloom[EXCL ? 512 : 1];   // excluded partners of the tile's atoms (16,384 bits, two hashes)
     __shared__ float4 s_shv[27];          // -k L per shift code (canonical displacement (xi - xj) + s)
     __shared__ float4 s_ax[64];           // the tile's atoms (x, y, z, bits of the id)
+    __shared__ float4 s_glo[NW], s_ghi[NW];   // per group: bounding box
     __shared__ int4 s_ex[EXCL ? 64 : 1];
-    __shared__ unsigned long long s_any[2][NW];
     __shared__ float s_bb[6];
-    __shared__ int s_w[NW];
-    __shared__ int s_wmax[NW];
+    __shared__ int s_w[NW], s_cw[NW], s_wmax[NW];
     __shared__ int s_cnt[64];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int tile = blockIdx.x;
@@ -300,29 +320,51 @@ __global__ __launch_bounds__(64 * NW, (NW == 4 && !EXCL) ? 5 : 1) void k_nl_tbui
     const RepParam& p = a.rep[r];
     const int cb = cur_buf(st);
     const float L0 = p.L[0], L1 = p.L[1], L2 = p.L[2];
+    const float rl2 = a.rl2;
+    const float rlp = sqrtf(rl2) * 1.0001f + 1e-4f;
+    // reach of a group's bounding box: r_list grown by what rounding of the coordinates, the
+    // image shift and the test can lose
+    const float reach2 = (rlp + 1e-3f + 1e-6f * (L0 + L1 + L2)) * (rlp + 1e-3f + 1e-6f * (L0 + L1 + L2));
     if (tid < 27) {
         const int kx = tid % 3 - 1, ky = (tid / 3) % 3 - 1, kz = tid / 9 - 1;
         s_shv[tid] = make_float4(-(float)kx * L0, -(float)ky * L1, -(float)kz * L2, 0.0f);
+    }
+    if (EXCL) {
+        s_bloom[tid] = 0u;   // NT = 512 words
+        __syncthreads();
     }
     if (tid < 64) {
         const bool act = id_pre >= 0;
         s_ax[tid] = make_float4(act ? x_pre.x : MD_FAR, act ? x_pre.y : MD_FAR, act ? x_pre.z : MD_FAR,
                                 __int_as_float(id_pre));
-        if (EXCL) s_ex[tid] = act ? a.excl[id_pre] : make_int4(-1, -1, -1, -1);
-        // tile bounding box over the active atoms
+        if (EXCL) {
+            const int4 ex = act ? a.excl[id_pre] : make_int4(-1, -1, -1, -1);
+            s_ex[tid] = ex;
+            for (const int q : {ex.x, ex.y, ex.z, ex.w})
+                if (q >= 0) {
+                    atomicOr(&s_bloom[(q >> 5) & 511], 1u << (q & 31));
+                    atomicOr(&s_bloom[excl_hash(q) >> 5], 1u << (excl_hash(q) & 31));
+                }
+        }
+        // bounding boxes over the active atoms, of the groups (8 lanes), then of the tile
         float lx = act ? x_pre.x : 3.0e38f, ly = act ? x_pre.y : 3.0e38f, lz = act ? x_pre.z : 3.0e38f;
         float hx = act ? x_pre.x : -3.0e38f, hy = act ? x_pre.y : -3.0e38f, hz = act ? x_pre.z : -3.0e38f;
-        for (int o = 32; o >= 1; o >>= 1) {
+        auto grow = [&](int o) {
             lx = fminf(lx, __shfl_xor(lx, o, 64)); ly = fminf(ly, __shfl_xor(ly, o, 64)); lz = fminf(lz, __shfl_xor(lz, o, 64));
             hx = fmaxf(hx, __shfl_xor(hx, o, 64)); hy = fmaxf(hy, __shfl_xor(hy, o, 64)); hz = fmaxf(hz, __shfl_xor(hz, o, 64));
+        };
+        for (int o = 1; o <= 4; o <<= 1) grow(o);
+        if ((lane & 7) == 0) {
+            s_glo[lane >> 3] = make_float4(lx, ly, lz, 0.0f);
+            s_ghi[lane >> 3] = make_float4(hx, hy, hz, 0.0f);
         }
+        for (int o = 8; o <= 32; o <<= 1) grow(o);
         if (tid == 0) {
             s_bb[0] = lx; s_bb[1] = ly; s_bb[2] = lz;
             s_bb[3] = hx; s_bb[4] = hy; s_bb[5] = hz;
         }
     }
     __syncthreads();
-    const float lx = s_bb[0], ly = s_bb[1], lz = s_bb[2], hx = s_bb[3], hy = s_bb[4], hz = s_bb[5];
     // this wavefront's atoms as wavefront-uniform values; an empty slot sits far
     // outside the box, so no candidate passes the distance test for it
     float axr[AW], ayr[AW], azr[AW];
@@ -337,209 +379,234 @@ __global__ __launch_bounds__(64 * NW, (NW == 4 && !EXCL) ? 5 : 1) void k_nl_tbui
     }
     const int gs = __builtin_ctz(a.row_g);   // row layout: lanes per atom of the step kernel, a power of 2
     const int cap = a.cap, jcap = a.jcap;
-    const float rl2 = a.rl2;
     uint16_t* const wrow = a.nl16 + (size_t)(slot0 + wave * AW) * cap;   // row of the wavefront's first atom
     uint32_t* const jset = a.jset + (size_t)tile * jcap;
-    const unsigned long long below = (1ull << lane) - 1ull;
     int jn = 0;     // size of the tile's set so far (workgroup-uniform)
-    int head = 0, tail = 0, nproc = 0;   // ring positions (taken mod RING), sub-chunks processed
+    // where this lane's entry of a 64-entry stretch of a row goes (lpos16): entry fe of the
+    // stretch to position fp, so the wavefront's stores are contiguous (G = 16: in 8-byte
+    // pieces, the stretch being half a block)
+    const int fe = gs == 2 ? (lane & 32) + ((lane >> 3) & 3) + 4 * (lane & 7)
+                           : gs == 3 ? (lane >> 3) + 8 * (lane & 7) : (lane >> 2) + 16 * (lane & 3);
+    const int fp = gs == 4 ? 8 * (lane >> 2) + (lane & 3) : lane;
 
-    // test ring entries [head, head + n) against this wavefront's atoms; assign set indices
-    auto process = [&](int n) {
-        const int q = (head + lane) & (RING - 1);
-        const bool valid = lane < n;
-        const float4 cx = s_cx[q];
-        const uint32_t info = __float_as_uint(cx.w);
-        const float4 sv = s_shv[valid ? (info >> MD_SLOTBITS) & 31 : MD_SHIFT0];   // ring data past n is stale
-        const int js = (int)(info & MD_SLOTMASK);
-        const int jid = EXCL ? s_cid[q] : 0;
-        unsigned long long m[AW];
-        unsigned long long any = 0;
-        // each condition is balloted on its own and the masks are combined as
-        // scalars: a compare then writes its lane mask directly
-        const unsigned long long vmask = __builtin_amdgcn_ballot_w64(valid);
-#pragma unroll
-        for (int i = 0; i < AW; i++) {
-            // (xi - xj) - k L: the canonical minimum-image displacement for this image
-            const float dx = (axr[i] - cx.x) + sv.x;
-            const float dy = (ayr[i] - cx.y) + sv.y;
-            const float dz = (azr[i] - cx.z) + sv.z;
-            const float rsq = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
-            unsigned long long mi = vmask & __builtin_amdgcn_ballot_w64(rsq < rl2) &
-                                    __builtin_amdgcn_ballot_w64(js != slot0 + wave * AW + i);
-            if (EXCL) {
-                const int4 ex = s_ex[wave * AW + i];
-                mi &= __builtin_amdgcn_ballot_w64(jid != ex.x) & __builtin_amdgcn_ballot_w64(jid != ex.y) &
-                      __builtin_amdgcn_ballot_w64(jid != ex.z) & __builtin_amdgcn_ballot_w64(jid != ex.w);
-            }
-            m[i] = mi;
-            any |= mi;
-        }
-        const int par = nproc & 1;
-        if (lane == 0) s_any[par][wave] = any;
-        __syncthreads();
-        any = 0;
-#pragma unroll
-        for (int w = 0; w < NW; w++) any |= s_any[par][w];
-        const bool mine = (any >> lane) & 1ull;
-        const int li = jn + 1 + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(any >> 32),
-                                                               __builtin_amdgcn_mbcnt_lo((uint32_t)any, 0u));
-        if (wave == 0 && mine && li - 1 < jcap) jset[li - 1] = info;
-        // a set that outgrew its capacity is rebuilt after the host grows it (the run
-        // is rolled back); until then its rows point past it only at the dummy.  Row
-        // entries are byte offsets of the staged entry (li x 16, li <= MD_JMAX).
-        const uint16_t lis = (uint16_t)(li - 1 < jcap ? li << 4 : 0);
-#pragma unroll
-        for (int i = 0; i < AW; i++) {
-            if (m[i]) {
-                const uint32_t e = __builtin_amdgcn_mbcnt_hi((uint32_t)(m[i] >> 32),
-                                                             __builtin_amdgcn_mbcnt_lo((uint32_t)m[i], (uint32_t)cnt[i]));
-                const int nh = __popcll(m[i]);
-                // the hit lanes are the mask itself (no per-lane bit test); the
-                // capacity test per lane only where this batch can cross it
-                if (cnt[i] + nh <= cap) {
-                    if (__builtin_amdgcn_inverse_ballot_w64(m[i])) wrow[(uint32_t)(i * cap) + lpos16_u(e, gs)] = lis;
-                } else {
-                    if (__builtin_amdgcn_inverse_ballot_w64(m[i]) && e < (uint32_t)cap)
-                        wrow[(uint32_t)(i * cap) + lpos16_u(e, gs)] = lis;
-                }
-                cnt[i] += nh;
-            }
-        }
-        jn += __popcll(any);
-        head += n;
-        nproc++;
+    // store entries e0 .. e0 + 63 (e0 a multiple of 64) of atom i's row; past c: the dummy.
+    // Rows longer than the capacity are cut (the host grows it and replays).
+    auto flush = [&](int i, int e0, int c) {
+        if (e0 >= cap) return;   // wavefront-uniform
+        __builtin_amdgcn_wave_barrier();
+        const uint16_t v = e0 + fe < c ? s_row[wave * AW + i][(e0 + fe) & 127] : (uint16_t)0;
+        const int off = gs == 4 ? (e0 & ~127) + ((e0 >> 4) & 4) : e0;
+        wrow[(uint32_t)(i * cap + off) + fp] = v;
+        __builtin_amdgcn_wave_barrier();
     };
 
-    if (lx <= hx) {
-        const float rlp = sqrtf(rl2) * 1.0001f + 1e-4f;
-        const float rlp2 = rlp * rlp;
-        // image-cell region covering the tile box grown by r_list
-        const Axis ax = make_axis(lx, hx, rlp, p.halfL[0], p.cinv[0], p.cedge[0], p.nc[0]);
-        const Axis ay = make_axis(ly, hy, rlp, p.halfL[1], p.cinv[1], p.cedge[1], p.nc[1]);
-        const Axis az = make_axis(lz, hz, rlp, p.halfL[2], p.cinv[2], p.cedge[2], p.nc[2]);
-        const int nreg = ax.nr * ay.nr * az.nr;
-        const int cell_off = p.cell_off, cs_off = p.cs_off, ncx = p.nc[0], ncy = p.nc[1];
-        // region cell c -> its cell's linear index and image shift code; -1 when the
-        // image cell lies r_list or farther from the box
-        auto locate = [=](int c, int& code) -> int {
-            int kx, ky, kz, wx, wy, wz;
-            const int cyz = floor_div(c, ax.nr, ax.inv_nr), cz = floor_div(cyz, ay.nr, ay.inv_nr);
-            const float ddx = ax.gap(ax.lo + (c - cyz * ax.nr), kx, wx);
-            const float ddy = ay.gap(ay.lo + (cyz - cz * ay.nr), ky, wy);
-            const float ddz = az.gap(az.lo + cz, kz, wz);
-            if (ddx * ddx + ddy * ddy + ddz * ddz >= rlp2) return -1;
-            code = shift_code(kx, ky, kz);
-            return wx + ncx * (wy + ncy * wz);
-        };
+    {
+        const int cell_off = p.cell_off, cs_off = p.cs_off;
+        int nreg = 1;
         for (int b0 = 0; b0 < nreg; b0 += kTab) {
-            // ---- table of non-empty image cells within r_list of the box (region order);
-            //      pass 1 counts, pass 2 writes
-            const int c0 = b0 + tid * PER, c1 = min(min(c0 + PER, nreg), b0 + kTab);
-            // the thread's PER region cells: geometry first, then all their rank
-            // loads, then all their bounds loads (two round trips, not 2 PER)
-            int pcell[PER], pcode[PER], prank[PER], pcs[PER], pn[PER];
-#pragma unroll
-            for (int u = 0; u < PER; u++) {
-                pcode[u] = 0;
-                pcell[u] = c0 + u < c1 ? locate(c0 + u, pcode[u]) : -1;
-            }
-#pragma unroll
-            for (int u = 0; u < PER; u++) prank[u] = pcell[u] >= 0 ? a.cell_rank[cell_off + pcell[u]] : 0;
-#pragma unroll
-            for (int u = 0; u < PER; u++) {
-                pcs[u] = 0;
-                pn[u] = 0;
-                if (pcell[u] >= 0) {
-                    pcs[u] = a.cell_start[cs_off + prank[u]];
-                    pn[u] = a.cell_start[cs_off + prank[u] + 1] - pcs[u];
-                }
-            }
-            int n_keep = 0, csum = 0;
-#pragma unroll
-            for (int u = 0; u < PER; u++) {
-                n_keep += pn[u] > 0;
-                csum += pn[u];
-            }
-            int ntab, T;
-            const int off = block_scan<NT>(n_keep, s_w, ntab);
-            const int coff = block_scan<NT>(csum, s_w, T);
-#pragma unroll
-            for (int u = 0, k = off, run = coff; u < PER; u++) {
-                if (pn[u] > 0) {
-                    s_tstart[k] = pcs[u];
-                    s_tpref[k] = run;
-                    s_tcode[k] = pcode[u];
-                    k++;
-                    run += pn[u];
-                }
-            }
-            if (tid == 0) s_tpref[ntab] = T;
-            __syncthreads();
-            // ---- stream the candidates, NT per chunk, into the ring (stable compaction).
-            //      The next chunk's members are located and their loads issued before
-            //      this chunk is tested, so the loads are in flight during the tests.
-            auto find = [&](int q, int& code) -> int {
-                int lo_ = 0, hi_ = ntab - 1;   // last table row with pref <= q
-                while (lo_ < hi_) {
-                    const int mid = (lo_ + hi_ + 1) >> 1;
-                    if (s_tpref[mid] <= q) lo_ = mid; else hi_ = mid - 1;
-                }
-                code = s_tcode[lo_];
-                return s_tstart[lo_] + (q - s_tpref[lo_]);
+            // image-cell region covering the tile box grown by r_list (in the loop, so its
+            // values need no registers during the tests; one round unless the cells are small)
+            auto bb = [&](int k) { return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(s_bb[k]))); };
+            const Axis ax = make_axis(bb(0), bb(3), rlp, p.halfL[0], p.cinv[0], p.cedge[0], p.nc[0]);
+            const Axis ay = make_axis(bb(1), bb(4), rlp, p.halfL[1], p.cinv[1], p.cedge[1], p.nc[1]);
+            const Axis az = make_axis(bb(2), bb(5), rlp, p.halfL[2], p.cinv[2], p.cedge[2], p.nc[2]);
+            nreg = bb(0) <= bb(3) ? ax.nr * ay.nr * az.nr : 0;   // no atoms: no region
+            if (nreg == 0) break;
+            const int ncx = p.nc[0], ncy = p.nc[1];
+            const float rlp2 = rlp * rlp;
+            // region cell c -> its cell's linear index and image shift code; -1 when the
+            // image cell lies r_list or farther from the box
+            auto locate = [=](int c, int& code) -> int {
+                int kx, ky, kz, wx, wy, wz;
+                const int cyz = floor_div(c, ax.nr, ax.inv_nr), cz = floor_div(cyz, ay.nr, ay.inv_nr);
+                const float ddx = ax.gap(ax.lo + (c - cyz * ax.nr), kx, wx);
+                const float ddy = ay.gap(ay.lo + (cyz - cz * ay.nr), ky, wy);
+                const float ddz = az.gap(az.lo + cz, kz, wz);
+                if (ddx * ddx + ddy * ddy + ddz * ddz >= rlp2) return -1;
+                code = shift_code(kx, ky, kz);
+                return wx + ncx * (wy + ncy * wz);
             };
-            int nj = -1, ncode = 0, nty = 0, nid = 0;
-            float4 nx = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (tid < T) {
-                nj = find(tid, ncode);
-                nx = a.pos_s[nj];
-                nty = a.typ_s[nj];
-                if (EXCL) nid = a.ids_s[nj];
+            // ---- a region cell per thread: its first slot and image shift (cell), members (n)
+            //      and the index of its first member among the candidates (first)
+            static_assert(kTab == NT, "a region cell per thread");
+            int code = 0, n = 0;
+            uint32_t cell = 0;
+            if (b0 + tid < nreg) {
+                const int c = locate(b0 + tid, code);
+                if (c >= 0) {
+                    const int rank = a.cell_rank[cell_off + c];
+                    const int cs = a.cell_start[cs_off + rank];
+                    n = a.cell_start[cs_off + rank + 1] - cs;
+                    cell = (uint32_t)cs | ((uint32_t)code << MD_SLOTBITS);
+                }
             }
+            int T;
+            const int first = block_scan<NT>(n, s_w, T);
+            // the candidates [q0, q0 + NT) to s_cand, each cell's by its thread
+            auto expand = [&](int q0) {
+                const int e = min(first + n, q0 + NT);
+                for (int q = max(first, q0); q < e; q++) s_cand[q - q0] = cell + (uint32_t)(q - first);
+            };
+            // ---- the candidates, NT per chunk.  The next chunk's loads are issued before
+            //      this chunk is tested, so they are in flight during the tests.
+            uint32_t nj = 0;   // slot | shift code << 24 of the candidate
+            int nty = 0, nid = 0;
+            float4 nx = make_float4(0.f, 0.f, 0.f, 0.f);
+            auto fetch = [&]() {
+                nj = s_cand[tid];
+                const int j = (int)(nj & MD_SLOTMASK);
+                nx = a.pos_s[j];
+                nty = a.typ_s[j];
+                if (EXCL) nid = a.ids_s[j];
+            };
+            expand(0);
+            __syncthreads();
+            if (tid < T) fetch();
             for (int base = 0; base < T; base += NT) {
-                const int j = nj, code = ncode, ty = nty, cid = nid;
                 float4 cx = nx;
-                nj = -1;
-                if (base + NT + tid < T) {
-                    nj = find(base + NT + tid, ncode);
-                    nx = a.pos_s[nj];
-                    nty = a.typ_s[nj];
-                    if (EXCL) nid = a.ids_s[nj];
+                const uint32_t info = nj | ((uint32_t)nty << MD_JBITS);
+                const int cid = nid;
+                // groups in reach: the image within `reach` of the group's bounding box
+                {
+                    const bool valid = base + tid < T;
+                    const float4 sv = s_shv[valid ? nj >> MD_SLOTBITS : MD_SHIFT0];
+                    const float ix = valid ? cx.x - sv.x : MD_FAR, iy = cx.y - sv.y, iz = cx.z - sv.z;
+                    int glo = 0, ghi = 0;   // lane g: the wavefront's mask of group g
+#pragma unroll 2
+                    for (int g = 0; g < NW; g++) {
+                        const float4 lo = s_glo[g], hi = s_ghi[g];
+                        const float gx = fmaxf(0.0f, fmaxf(lo.x - ix, ix - hi.x));
+                        const float gy = fmaxf(0.0f, fmaxf(lo.y - iy, iy - hi.y));
+                        const float gz = fmaxf(0.0f, fmaxf(lo.z - iz, iz - hi.z));
+                        const unsigned long long in =
+                            __builtin_amdgcn_ballot_w64(fmaf(gz, gz, fmaf(gy, gy, gx * gx)) < reach2);
+                        glo = writelane((int)(uint32_t)in, g, glo);
+                        ghi = writelane((int)(uint32_t)(in >> 32), g, ghi);
+                    }
+                    if (lane < NW) s_gm[wave][lane] = make_uint2((uint32_t)glo, (uint32_t)ghi);
                 }
-                bool keep = false;
-                if (j >= 0) {
-                    const float4 sv = s_shv[code];
-                    const float ix = cx.x - sv.x, iy = cx.y - sv.y, iz = cx.z - sv.z;   // image position
-                    const float gx = fmaxf(0.0f, fmaxf(lx - ix, ix - hx));
-                    const float gy = fmaxf(0.0f, fmaxf(ly - iy, iy - hy));
-                    const float gz = fmaxf(0.0f, fmaxf(lz - iz, iz - hz));
-                    keep = gx * gx + gy * gy + gz * gz < rlp2;
-                    cx.w = __uint_as_float((uint32_t)j | ((uint32_t)code << MD_SLOTBITS) | ((uint32_t)ty << MD_JBITS));
+                cx.w = __uint_as_float(info);
+                s_cx[tid] = cx;
+                s_hit[tid] = 0;
+                if (EXCL) {
+                    const bool may = ((s_bloom[(cid >> 5) & 511] >> (cid & 31)) & 1u) &&
+                                     ((s_bloom[excl_hash(cid) >> 5] >> (excl_hash(cid) & 31)) & 1u);
+                    s_cid[tid] = cid | (may ? (int)0x80000000 : 0);
                 }
-                int kept;
-                const int at = block_scan<NT>(keep ? 1 : 0, s_w, kept);
-                if (keep) {
-                    const int k = (tail + at) & (RING - 1);
-                    s_cx[k] = cx;
-                    if (EXCL) s_cid[k] = cid;
+                if (base + NT < T) expand(base + NT);
+                __syncthreads();
+                if (base + NT + tid < T) fetch();
+                // ---- this wavefront's candidates of the chunk
+                int nl = 0;
+                const uint2 gm = s_gm[lane & (NW - 1)][wave];
+#pragma unroll
+                for (int w = 0; w < NW; w++) {
+                    const uint32_t g0 = (uint32_t)__builtin_amdgcn_readlane((int)gm.x, w),
+                                   g1 = (uint32_t)__builtin_amdgcn_readlane((int)gm.y, w);
+                    const unsigned long long in = ((unsigned long long)g1 << 32) | g0;
+                    const uint32_t e = __builtin_amdgcn_mbcnt_hi(g1, __builtin_amdgcn_mbcnt_lo(g0, (uint32_t)nl));
+                    if (__builtin_amdgcn_inverse_ballot_w64(in)) s_list[wave][e] = (uint16_t)(w * 64 + lane);
+                    nl += __popcll(in);
+                }
+                // ---- distance tests: hit masks of batch b and atom i in lane 8 b + i
+                int mlo = 0, mhi = 0;
+                const int nbat = (nl + 63) >> 6;
+                for (int b = 0; b < nbat; b++) {
+                    const int k = b * 64 + lane;
+                    const bool valid = k < nl;
+                    const int t = s_list[wave][valid ? k : 0];
+                    float4 q = s_cx[t];
+                    const uint32_t qi = __float_as_uint(q.w);
+                    const int qc = (int)((qi >> MD_SLOTBITS) & 31u), js = (int)(qi & MD_SLOTMASK);
+                    const int jid = EXCL ? s_cid[t] : 0;
+                    if (!valid) q.x = MD_FAR;   // out of everyone's reach
+                    // Most batches hold no image (every shift zero: the canonical (xi - xj) - 0
+                    // is xi - xj) and neither an atom of the tile nor a possibly excluded one;
+                    // those conditions are only tested for batches that do (wavefront-uniform).
+                    const bool shifted = __builtin_amdgcn_ballot_w64(qc != MD_SHIFT0) != 0;
+                    const bool own = __builtin_amdgcn_ballot_w64((uint32_t)(js - slot0) < 64u || (EXCL && jid < 0)) != 0;
+                    unsigned long long any = 0;
+                    auto test = [&](auto shift_tag, auto own_tag) {
+                        constexpr bool SH = decltype(shift_tag)::value, OWN = decltype(own_tag)::value;
+                        float4 sv = make_float4(0.f, 0.f, 0.f, 0.f);
+                        if (SH) sv = s_shv[qc];
+#pragma unroll
+                        for (int i = 0; i < AW; i++) {
+                            float dx = axr[i] - q.x, dy = ayr[i] - q.y, dz = azr[i] - q.z;
+                            if (SH) {   // (xi - xj) - k L: the canonical minimum-image displacement for this image
+                                dx += sv.x;
+                                dy += sv.y;
+                                dz += sv.z;
+                            }
+                            const float rsq = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
+                            unsigned long long m = __builtin_amdgcn_ballot_w64(rsq < rl2);
+                            if (OWN) {
+                                m &= __builtin_amdgcn_ballot_w64(js != slot0 + wave * AW + i);
+                                if (EXCL) {
+                                    const int qid = jid & 0x7fffffff;
+                                    const int4 ex = s_ex[wave * AW + i];
+                                    m &= __builtin_amdgcn_ballot_w64(qid != ex.x && qid != ex.y && qid != ex.z && qid != ex.w);
+                                }
+                            }
+                            any |= m;
+                            mlo = writelane((int)(uint32_t)m, b * AW + i, mlo);
+                            mhi = writelane((int)(uint32_t)(m >> 32), b * AW + i, mhi);
+                        }
+                    };
+                    if (own) test(std::true_type{}, std::true_type{});
+                    else if (shifted) test(std::true_type{}, std::false_type{});
+                    else test(std::false_type{}, std::false_type{});
+                    if (__builtin_amdgcn_inverse_ballot_w64(any)) s_hit[t] = 1;
                 }
                 __syncthreads();
-                tail += kept;
-                while (tail - head >= 64) process(64);   // at most 63 entries stay pending
+                // ---- the chunk's set entries
+                const unsigned long long hm = __builtin_amdgcn_ballot_w64(s_hit[tid] != 0);
+                if (lane == 0) s_cw[wave] = __popcll(hm);
+                __syncthreads();
+                int li = jn + 1 + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(hm >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)hm, 0u));
+#pragma unroll
+                for (int w = 0; w < NW; w++) {
+                    if (w < wave) li += s_cw[w];
+                    jn += s_cw[w];
+                }
+                // a set that outgrew its capacity is rebuilt after the host grows it (the run
+                // is rolled back); until then its rows point past it only at the dummy.  Row
+                // entries are byte offsets of the staged entry (li x 16, li <= MD_JMAX).
+                if (__builtin_amdgcn_inverse_ballot_w64(hm)) {
+                    if (li - 1 < jcap) jset[li - 1] = info;
+                    s_li[tid] = (uint16_t)(li - 1 < jcap ? li << 4 : 0);
+                }
+                __syncthreads();
+                // ---- the hits to the atoms' rows in LDS (under the hit mask itself); a full
+                //      stretch of 64 entries goes out
+                for (int b = 0; b < nbat; b++) {
+                    const int k = b * 64 + lane;
+                    const uint16_t lis = s_li[s_list[wave][k < nl ? k : 0]];
+#pragma unroll
+                    for (int i = 0; i < AW; i++) {
+                        const uint32_t m0 = (uint32_t)__builtin_amdgcn_readlane(mlo, b * AW + i),
+                                       m1 = (uint32_t)__builtin_amdgcn_readlane(mhi, b * AW + i);
+                        const unsigned long long mi = ((unsigned long long)m1 << 32) | m0;
+                        const uint32_t e = __builtin_amdgcn_mbcnt_hi(m1, __builtin_amdgcn_mbcnt_lo(m0, (uint32_t)cnt[i]));
+                        if (__builtin_amdgcn_inverse_ballot_w64(mi)) s_row[wave * AW + i][e & 127u] = lis;
+                        const int c0 = cnt[i];
+                        cnt[i] += __popcll(mi);
+                        if ((c0 ^ cnt[i]) & 64) flush(i, c0 & ~63, cnt[i]);
+                    }
+                }
             }
         }
-        if (tail > head) process(tail - head);
     }
-    // row lengths, row padding up to the end of the last block (the dummy, local
-    // index 0), longest row of the wavefront
-    const int blk = 8 << gs;
+    // the rows' last entries, padded to the end of the last block (the dummy, local
+    // index 0), row lengths, longest row of the wavefront
     int mx = 0;
 #pragma unroll
     for (int i = 0; i < AW; i++) {
         const int c = cnt[i];
         mx = max(mx, c);
-        const int endb = min((c + blk - 1) / blk * blk, cap);
-        for (int e = c + lane; e < endb; e += 64) wrow[(size_t)i * cap + lpos16(e, blk / 8)] = 0;
+        if (c & 63) flush(i, c & ~63, c);
+        const int e1 = (c + 63) & ~63;
+        if (gs == 4 && (e1 & 64)) flush(i, e1, c);
         if (lane == i) {
             const int cc = __float_as_int(s_ax[wave * AW + i].w) >= 0 ? c : 0;
             a.ncount[slot0 + wave * AW + i] = cc;
@@ -553,6 +620,7 @@ __global__ __launch_bounds__(64 * NW, (NW == 4 && !EXCL) ? 5 : 1) void k_nl_tbui
     if (tid < 64) {
         const int c = s_cnt[tid];
         int rank = 0;
+#pragma unroll 4
         for (int k = 0; k < 64; k++) {
             const int d = s_cnt[k];
             rank += (d > c) || (d == c && k < tid);
@@ -691,13 +759,8 @@ extern "C" hipError_t md_launch_rebuild(const BuildArgs& a, int commit, hipStrea
     hipLaunchKernelGGL(k_nl_scatter, dim3(nb), dim3(256), 0, st, a);
     hipLaunchKernelGGL(k_nl_permute, dim3(nb), dim3(256), 0, st, a);
     const dim3 ntiles(a.nslot / 64);
-    if (a.build_nw == 8) {
-        if (a.has_excl) hipLaunchKernelGGL((k_nl_tbuild<true, 8>), ntiles, dim3(512), 0, st, a);
-        else hipLaunchKernelGGL((k_nl_tbuild<false, 8>), ntiles, dim3(512), 0, st, a);
-    } else {
-        if (a.has_excl) hipLaunchKernelGGL((k_nl_tbuild<true, 4>), ntiles, dim3(256), 0, st, a);
-        else hipLaunchKernelGGL((k_nl_tbuild<false, 4>), ntiles, dim3(256), 0, st, a);
-    }
+    if (a.has_excl) hipLaunchKernelGGL((k_nl_tbuild<true>), ntiles, dim3(512), 0, st, a);
+    else hipLaunchKernelGGL((k_nl_tbuild<false>), ntiles, dim3(512), 0, st, a);
     if (commit) hipLaunchKernelGGL(k_nl_commit, dim3((a.nrep + 3) / 4), dim3(256), 0, st, a);
     return hipGetLastError();
 }

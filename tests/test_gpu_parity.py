@@ -78,6 +78,50 @@ def test_neighbor_sets_bit_exact(E, orc, name, lanes, cell_div, build):
     e.close()
 
 
+def few_atoms(n, seed=5, L=40.0):
+    """n Ar-Xe atoms at random in a box of L A: tiles with empty groups of slots."""
+    rng = np.random.default_rng(seed)
+    s = S.arxe_replicas(nrep=1, nmin=1024, nmax=1025)[0]
+    s.box = np.full(3, L, np.float32)
+    s.pos = rng.uniform(-L / 2, L / 2, (n, 3)).astype(np.float32)
+    s.type, s.charge, s.vel = s.type[:n], s.charge[:n], s.vel[:n]
+    return s
+
+
+def list_edges():
+    """Systems at the list build's edges: one atom in a tile, a partial group, whole tiles;
+    rows of several 64-entry stretches (about 630 neighbors) in a box whose reach is nearly
+    all of it (images on every side)."""
+    dense = perturbed(S.nacl(nsites=12, ff=S.nacl_ff(rc=14.0)), 0.2)
+    return {"atoms2": few_atoms(2), "atoms65": few_atoms(65), "atoms72": few_atoms(72), "atoms1000": few_atoms(1000),
+            "argon256": perturbed(S.argon(ncell=4), 0.2), "dense1728": dense,
+            "water693": perturbed(S.water(nmol=700), 0.05)}
+
+
+EDGES = list_edges()
+
+
+@pytest.mark.parametrize("lanes", [4, 8, 16])
+@pytest.mark.parametrize("cell_div", [1, 3])
+@pytest.mark.parametrize("name", list(EDGES))
+def test_list_build_edges(E, orc, name, lanes, cell_div):
+    """Neighbor sets at the build's edges equal the oracle's for every row layout (64-entry
+    stretches of rows in blocks of 32, 64 and 128 entries) and for one and several rounds of
+    region cells."""
+    s = EDGES[name]
+    say("list edges", name, s.n, "lanes", lanes, "cell_div", cell_div)
+    e = E.Engine.from_system(s)
+    e.set_launch(lanes=lanes, cell_div=cell_div)
+    assert all(v == 0 for v in e.check_lists().values()), e.check_lists()
+    pos, _, _ = e.download()
+    counts, nbrs = e.neighbors()
+    oc, on = orc.nlist(pos, s.box, e.thresholds()[1], s.exclusions())
+    assert np.array_equal(counts, oc)
+    for i in range(s.n):
+        assert np.array_equal(np.sort(nbrs[i, :counts[i]]), on[i, :oc[i]]), f"atom {i}"
+    e.close()
+
+
 @pytest.mark.parametrize("name", ["argon864", "nacl4096_wolf", "water1536"])
 def test_build_wavefronts_same_lists(E, name):
     """The tile build with 4 or 8 wavefronts per tile writes the same sets and rows
