@@ -52,7 +52,10 @@ extern "C" hipError_t md_launch_persist(const PersistArgs& a, int lanes, size_t 
                                         hipEvent_t ev1);
 extern "C" hipError_t md_launch_persist_clear(unsigned* flags, hipStream_t st);
 extern "C" hipError_t md_launch_settle(const SettleArgs& a, hipStream_t st);
-extern "C" int md_launch_pme(const PmeArgs& a, hipfftHandle r2c, hipfftHandle c2r, hipStream_t st);
+extern "C" int md_launch_pme(const PmeArgs& a, const PmeFftArgs* f, hipfftHandle r2c, hipfftHandle c2r, int energy,
+                             hipStream_t st);
+extern "C" int md_pme_fft_plan(int K0, int K1, int K2, size_t lds, PmeFftArgs* f);
+extern "C" hipError_t md_pme_fft_setup(int K0, int K1, int K2, const PmeFftArgs& f);
 extern "C" hipError_t md_launch_report(const RepState* st, int nrep, const int* tmax, int ntiles, const int* err,
                                        RunReport* out, hipStream_t stream);
 
@@ -291,6 +294,9 @@ struct md_engine {
     DBuf<double> pme_part, pme_out;
     DBuf<char> pme_work;
     hipfftHandle pme_r2c = nullptr, pme_c2r = nullptr;
+    bool pme_own = false;          // the transforms run in pme_fft.hip (else hipFFT)
+    PmeFftArgs pme_fft{};
+    DBuf<double2> pme_tw;          // its twiddle tables
     // segment graphs by key (check interval, energy interval, blocks); two
     // executable copies each, launched alternately, so the next replay can be
     // submitted while the previous one still runs
@@ -681,7 +687,8 @@ int pme_prepare(md_engine* e) {
     e->drop_graphs();   // captured segments hold the previous buffers
     e->drop_pme_plans();
     const size_t n = (size_t)K[0] * K[1] * K[2], nh = (size_t)K[0] * K[1] * (K[2] / 2 + 1);
-    e->pme_nconv = (int)std::min<size_t>((nh + 255) / 256, 2048);
+    e->pme_own = md_pme_fft_plan(K[0], K[1], K[2], e->lds_max, &e->pme_fft) != 0;
+    e->pme_nconv = e->pme_own ? e->pme_fft.ncol : (int)std::min<size_t>((nh + 255) / 256, 2048);
     e->pme_ngather = (e->S + 63) / 64;   // 4 lanes per slot, 256 lanes per workgroup
     CHECK(e->pme_qgrid.alloc(n));
     CHECK(e->pme_sgrid.alloc(nh));
@@ -717,6 +724,19 @@ int pme_prepare(md_engine* e) {
     const double beta = e->ff.alpha;
     e->pme_eself = -(double)e->ff.qfac * beta / std::sqrt(pi) * s2;
     e->pme_qsum2 = s1 * s1;
+    if (e->pme_own) {
+        std::vector<double2> tw;
+        for (int d = 0; d < 3; d++)
+            for (int k = 0; k < K[d]; k++)
+                tw.push_back(make_double2(std::cos(2.0 * pi * k / K[d]), std::sin(2.0 * pi * k / K[d])));
+        CHECK(e->pme_tw.alloc(tw.size()));
+        HIPCHECK(hipMemcpy(e->pme_tw.p, tw.data(), tw.size() * sizeof(double2), hipMemcpyHostToDevice));
+        e->pme_fft.tw = e->pme_tw.p;
+        HIPCHECK(md_pme_fft_setup(K[0], K[1], K[2], e->pme_fft));
+        e->pme_S = e->S;
+        e->pme_on = true;
+        return MD_OK;
+    }
     // FFT plans on the engine's stream with one work area allocated here, so a
     // captured segment makes no allocation
     size_t ws1 = 0, ws2 = 0;
@@ -760,8 +780,8 @@ PmeArgs pme_args(md_engine* e, int mode) {
     return g;
 }
 
-int enqueue_pme(md_engine* e, int mode) {
-    const int rc = md_launch_pme(pme_args(e, mode), e->pme_r2c, e->pme_c2r, e->st);
+int enqueue_pme(md_engine* e, int mode, int energy) {
+    const int rc = md_launch_pme(pme_args(e, mode), e->pme_own ? &e->pme_fft : nullptr, e->pme_r2c, e->pme_c2r, energy, e->st);
     if (rc == 2) return fail(MD_E_HIP, "hipFFT execution failed");
     if (rc != 0) return fail(MD_E_HIP, "PME kernel launch failed");
     return MD_OK;
@@ -769,7 +789,7 @@ int enqueue_pme(md_engine* e, int mode) {
 
 int enqueue_stepkernel(md_engine* e, const StepArgs& a, TimedSpan* ts, bool finalize = true) {
     // long-range part first: the step kernel adds its forces and energy
-    if (e->pme_on) CHECK(enqueue_pme(e, a.mode));
+    if (e->pme_on) CHECK(enqueue_pme(e, a.mode, a.mode == MODE_FORCE ? a.force_energy : a.energy_every > 0));
     std::pair<hipEvent_t, hipEvent_t> ev{};
     if (ts) ev = ts->take();   // the launch records the kernel's own start and end
     HIPCHECK(md_launch_step(a, e->lanes, e->coul_kernel, e->st, ev.first, ev.second));

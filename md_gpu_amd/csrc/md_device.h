@@ -33,6 +33,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "md_fft.h"
+
 #define MD_TILE 64
 #define MD_JBITS 29             // bond_list entries: partner | type << 29
 #define MD_JMASK 0x1FFFFFFFu
@@ -271,6 +273,15 @@ struct PmeArgs {
     int small_q;                // every |q| < 2^18: a weighted charge's fixed point fits 52 bits
     int baro;                   // pressure coupling: the box (and the margin) follow the scale since the build
     float rl, rc;
+};
+
+// Transforms of smooth PME in the engine's own kernels (pme_fft.hip).
+struct PmeFftArgs {
+    FftPlan p0, p1, p2;         // factors per axis
+    fft::Div drow, dh, dk2, dk24, dcol;   // (K1 + 1) / 2, K2 / 2 + 1, K2, K2 / 4 (at least 1), columns per workgroup
+    int plane;                  // complex elements of one LDS buffer of an x plane
+    int ncol;                   // workgroups of the x transforms (16 columns each)
+    const double2* tw;          // [K0 + K1 + K2] per axis (cos, sin)(2 pi k / K)
 };
 
 // Progress of a run for the host: one small copy per check instead of one per

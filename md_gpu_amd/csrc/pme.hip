@@ -387,19 +387,23 @@ __global__ __launch_bounds__(PT) void k_pme_conv(const PmeArgs a) {
 // then lane c of the quad reads the stencil points with z offsets c and c + 4
 // and the quad's partial gradients are summed by DPP.  Lane c also takes the
 // atom's c-th excluded partner.
-template <int P>
+template <int P, bool EN>
 __global__ __launch_bounds__(PT) void k_pme_gather(const PmeArgs a) {
     __shared__ float s_t[PT / 4][3][P], s_d[PT / 4][3][P];
     __shared__ int s_k[PT / 4][3];
-    const RepState s = a.st[0];
-    if (!pme_go(s, a.mode)) return;   // grid-uniform
     const int sub = threadIdx.x & 3, la = threadIdx.x >> 2;   // lane in the quad, atom in the workgroup
-    const int slot = blockIdx.x * (PT / 4) + la;
+    const int slot = blockIdx.x * (PT / 4) + la, sl = min(slot, a.nslot - 1);
     double e = 0.0, w = 0.0;
-    const int id = slot < a.nslot ? a.ids[slot] : -1;
-    const float4* __restrict__ pin = a.pos[cur_buf(s)];
-    const float4 x = id >= 0 ? pin[slot] : make_float4(0.f, 0.f, 0.f, 0.f);
+    // the state, the slot's id, its position in both buffers and the box in one round trip
+    const RepState s = a.st[0];
+    const int id0 = a.ids[sl];
+    const float4 xa = a.pos[0][sl], xb = a.pos[1][sl];
     const PmeBox bx = pme_box(a);
+    loads_issued();
+    if (!pme_go(s, a.mode)) return;   // grid-uniform
+    const int id = slot < a.nslot ? id0 : -1;
+    const float4* __restrict__ pin = a.pos[cur_buf(s)];
+    const float4 x = id >= 0 ? (cur_buf(s) ? xb : xa) : make_float4(0.f, 0.f, 0.f, 0.f);
     if (x.w != 0.0f && sub < 3) {   // this lane's axis
         const float xc = sub == 0 ? x.x : (sub == 1 ? x.y : x.z);
         // selected, not indexed by the lane's axis: an indexed private array lives in scratch
@@ -484,10 +488,12 @@ __global__ __launch_bounds__(PT) void k_pme_gather(const PmeArgs a) {
                 fz = fmaf(fr, dzz, fz);
                 // energy and virial in FP64: for neutral molecules these terms nearly
                 // cancel the self term, each far larger than their sum
-                const double rd = sqrt((double)r2), bd = (double)a.beta * rd;
-                const double qqd = (double)a.qfac * (double)x.w * (double)y.w, erfd = erf(bd);
-                e -= 0.5 * qqd * erfd / rd;   // each pair is listed from both atoms
-                w += 0.5 * qqd * (1.1283791670955126 * bd * exp(-bd * bd) - erfd) / rd;
+                if (EN) {
+                    const double rd = sqrt((double)r2), bd = (double)a.beta * rd;
+                    const double qqd = (double)a.qfac * (double)x.w * (double)y.w, erfd = erf(bd);
+                    e -= 0.5 * qqd * erfd / rd;   // each pair is listed from both atoms
+                    w += 0.5 * qqd * (1.1283791670955126 * bd * exp(-bd * bd) - erfd) / rd;
+                }
             }
         }
     }
@@ -495,7 +501,7 @@ __global__ __launch_bounds__(PT) void k_pme_gather(const PmeArgs a) {
     fy = group_sum<4>(fy);
     fz = group_sum<4>(fz);
     if (id >= 0 && sub == 0) a.frec[slot] = make_float4(fx, fy, fz, 0.0f);
-    block_pair_sum(e, w, a.part, a.nconv + blockIdx.x);
+    if (EN) block_pair_sum(e, w, a.part, a.nconv + blockIdx.x);
 }
 
 // Every workgroup's (energy, virial) pair of the influence and gather kernels in
@@ -529,14 +535,21 @@ void launch_spread(const PmeArgs& a, hipStream_t st) {
 }
 
 template <int P>
-void launch_gather(const PmeArgs& a, hipStream_t st) {
-    hipLaunchKernelGGL(k_pme_gather<P>, dim3(a.ngather), dim3(PT), 0, st, a);
+void launch_gather(const PmeArgs& a, int energy, hipStream_t st) {
+    if (energy) hipLaunchKernelGGL((k_pme_gather<P, true>), dim3(a.ngather), dim3(PT), 0, st, a);
+    else hipLaunchKernelGGL((k_pme_gather<P, false>), dim3(a.ngather), dim3(PT), 0, st, a);
 }
 
 }  // namespace
 
-// Queue the chain for one step.  Returns 0, or 1 (HIP launch error) or 2 (hipFFT error).
-extern "C" int md_launch_pme(const PmeArgs& a, hipfftHandle r2c, hipfftHandle c2r, hipStream_t st) {
+extern "C" hipError_t md_launch_pme_fft(const PmeArgs& a, const PmeFftArgs& f, int energy, hipStream_t st);
+
+// Queue the chain for one step.  f: the plans of the engine's own transforms, or null: r2c
+// and c2r.  energy = 0: no step of the run asks for energies or the virial, so their sums are
+// left out (their readers, the step kernel's energy variants, do not run either).
+// Returns 0, or 1 (HIP launch error) or 2 (hipFFT error).
+extern "C" int md_launch_pme(const PmeArgs& a, const PmeFftArgs* f, hipfftHandle r2c, hipfftHandle c2r, int energy,
+                             hipStream_t st) {
     switch (a.order) {
     case 4: launch_spread<4>(a, st); break;
     case 6: launch_spread<6>(a, st); break;
@@ -544,14 +557,18 @@ extern "C" int md_launch_pme(const PmeArgs& a, hipfftHandle r2c, hipfftHandle c2
     default: return 1;
     }
     if (hipGetLastError() != hipSuccess) return 1;
-    if (hipfftExecR2C(r2c, a.qgrid, reinterpret_cast<hipfftComplex*>(a.sgrid)) != HIPFFT_SUCCESS) return 2;
-    hipLaunchKernelGGL(k_pme_conv, dim3(a.nconv), dim3(PT), 0, st, a);
-    if (hipfftExecC2R(c2r, reinterpret_cast<hipfftComplex*>(a.sgrid), a.qgrid) != HIPFFT_SUCCESS) return 2;
-    switch (a.order) {
-    case 4: launch_gather<4>(a, st); break;
-    case 6: launch_gather<6>(a, st); break;
-    default: launch_gather<8>(a, st); break;
+    if (f) {
+        if (md_launch_pme_fft(a, *f, energy, st) != hipSuccess) return 1;
+    } else {
+        if (hipfftExecR2C(r2c, a.qgrid, reinterpret_cast<hipfftComplex*>(a.sgrid)) != HIPFFT_SUCCESS) return 2;
+        hipLaunchKernelGGL(k_pme_conv, dim3(a.nconv), dim3(PT), 0, st, a);
+        if (hipfftExecC2R(c2r, reinterpret_cast<hipfftComplex*>(a.sgrid), a.qgrid) != HIPFFT_SUCCESS) return 2;
     }
-    hipLaunchKernelGGL(k_pme_sum, dim3(1), dim3(PT), 0, st, a);
+    switch (a.order) {
+    case 4: launch_gather<4>(a, energy, st); break;
+    case 6: launch_gather<6>(a, energy, st); break;
+    default: launch_gather<8>(a, energy, st); break;
+    }
+    if (energy) hipLaunchKernelGGL(k_pme_sum, dim3(1), dim3(PT), 0, st, a);
     return hipGetLastError() == hipSuccess ? 0 : 1;
 }

@@ -93,6 +93,26 @@ def test_forces_nacl(E, orc, grid, order):
     check_forces(E, orc, s)
 
 
+@pytest.mark.parametrize("grid", [(5, 9, 15), (16, 6, 10), (48, 50, 45), (27, 25, 81), (96, 8, 4), (128, 120, 100),
+                                  (40, 136, 128), (108, 108, 108), (48, 160, 150)])
+def test_forces_own_transforms(E, orc, grid):
+    """The transforms in the engine's own kernels: odd and even edges on every axis (an odd
+    last edge, a last row without a partner), one to three passes per axis, every radix, the
+    largest planes that fit the LDS and one that does not (hipFFT); energies and virial, and
+    the forces of a step that asks for none (their sums left out)."""
+    s = nacl_pme(nsites=12, grid=grid)
+    say("pme own transforms", s.pme)
+    check_forces(E, orc, s)
+    e = E.Engine.from_system(dataclasses.replace(s, integrator="vverlet", thermostat="none"))
+    e.run(1, stats=False)
+    F1 = e.download()[2]
+    so = s.copy()
+    so.pos = e.download()[0]
+    e.close()
+    Fo, _, _ = orc.forces(so)
+    assert rel_rms(F1, Fo) < FORCE_TOL
+
+
 @pytest.mark.parametrize("cell_div", [1, 2, 3])
 @pytest.mark.parametrize("grid,order", [((4, 4, 4), 4), ((8, 16, 17), 4), ((9, 33, 15), 6), ((8, 8, 48), 8)])
 def test_forces_brick_edges(E, orc, grid, order, cell_div):
