@@ -28,6 +28,7 @@
 #include <hipfft/hipfft.h>
 
 #include "md_device.h"
+#include "state_out.h"
 #include "mdgpu/md_api.h"
 
 extern "C" hipError_t md_launch_rebuild(const BuildArgs& a, int commit, hipStream_t st);
@@ -307,6 +308,8 @@ struct md_engine {
     double t_step_ms = 0, t_reb_ms = 0;
     long long n_step = 0, n_reb = 0;
     std::vector<hipEvent_t> ev_pool;
+
+    HostRing host_ring;   // downloads pass through it
 
     ~md_engine() {
         drop_graphs();
@@ -1357,38 +1360,12 @@ int md_upload_state(md_engine* e, const float* pos, const float* vel) {
 int md_download_state(md_engine* e, float* pos, float* vel, float* force) {
     CHECK(check_ready(e, true));
     HIPCHECK(hipSetDevice(e->dev));
-    std::vector<RepState> rs;
-    CHECK(read_states(e, rs));
-    const int S = e->S;
-    std::vector<int> ids(S);
-    HIPCHECK(hipMemcpy(ids.data(), e->ids.p, S * sizeof(int), hipMemcpyDeviceToHost));
-    std::vector<float4> buf(S), buf2;
-    float* outs[3] = {pos, vel, force};
-    for (int k = 0; k < 3; k++) {
-        if (!outs[k]) continue;
-        if (k == 0) {   // positions: each replica's current buffer
-            buf2.resize(S);
-            HIPCHECK(hipMemcpy(buf.data(), e->pos[0].p, S * sizeof(float4), hipMemcpyDeviceToHost));
-            HIPCHECK(hipMemcpy(buf2.data(), e->pos[1].p, S * sizeof(float4), hipMemcpyDeviceToHost));
-        } else {
-            HIPCHECK(hipMemcpy(buf.data(), k == 1 ? e->vel.p : e->force.p, S * sizeof(float4), hipMemcpyDeviceToHost));
-        }
-        for (int s = 0; s < S; s++) {
-            int i = ids[s];
-            if (i < 0) continue;
-            const int r = e->tile_rep_h[s / MD_TILE];
-            float4 v = (k == 0 && cur_buf(rs[r]) == 1) ? buf2[s] : buf[s];
-            if (k == 0) {   // positions run unwrapped between list builds: wrap as the build does
-                const RepParam& p = e->rep_h[r];
-                v.x = wrap_coord(v.x, p.L[0], p.Linv[0]);
-                v.y = wrap_coord(v.y, p.L[1], p.Linv[1]);
-                v.z = wrap_coord(v.z, p.L[2], p.Linv[2]);
-            }
-            outs[k][3 * (size_t)i] = v.x;
-            outs[k][3 * (size_t)i + 1] = v.y;
-            outs[k][3 * (size_t)i + 2] = v.z;
-        }
-    }
+    StateOutArgs a{};
+    a.pos[0] = e->pos[0].p; a.pos[1] = e->pos[1].p; a.vel = e->vel.p; a.force = e->force.p;
+    a.slot_of = e->slot_of.p; a.tile_rep = e->tile_rep.p; a.rep = e->rep.p; a.st = e->rst.p;
+    a.nrep = e->R; a.natom = e->N;
+    float* const outs[3] = {pos, vel, force};
+    HIPCHECK(md_state_out(a, outs, e->host_ring, e->st));
     return MD_OK;
 }
 

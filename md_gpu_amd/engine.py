@@ -236,14 +236,14 @@ class Engine:
         _check(lib().md_upload_state(self._h, _ptr(pos), _ptr(vel)))
 
     def download(self):
-        pos = np.zeros((self.N, 3), np.float32)
-        vel = np.zeros((self.N, 3), np.float32)
-        frc = np.zeros((self.N, 3), np.float32)
+        pos = np.empty((self.N, 3), np.float32)
+        vel = np.empty((self.N, 3), np.float32)
+        frc = np.empty((self.N, 3), np.float32)
         _check(lib().md_download_state(self._h, _ptr(pos), _ptr(vel), _ptr(frc)))
         return pos, vel, frc
 
     def compute_forces(self):
-        F = np.zeros((self.N, 3), np.float32)
+        F = np.empty((self.N, 3), np.float32)
         E = np.zeros((self.nrep, 4), np.float64)
         W = np.zeros(self.nrep, np.float64)
         _check(lib().md_compute_forces(self._h, _ptr(F), _ptr(E), _ptr(W)))

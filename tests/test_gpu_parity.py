@@ -397,3 +397,48 @@ def test_launch_variants_match_oracle(E, orc, kind, variant):
     assert np.abs(dpos).max() < 2e-4
     assert np.allclose(st["temp"][:, 0], r["temp"], rtol=1e-4)
     e.close()
+
+
+def lattice(n, seed):
+    """n argon atoms on a jittered 4 A lattice, off the box faces."""
+    m = int(np.ceil(n ** (1 / 3)))
+    m = max(m, 8)
+    rng = np.random.default_rng(seed)
+    s = S.argon(ncell=4).copy()
+    L = 4.0 * m
+    s.box = np.full(3, L, np.float32)
+    g = rng.permutation(m ** 3)[:n]
+    x = (np.stack([g // m // m, g // m % m, g % m], 1) + 0.5) * 4.0 - L / 2 + rng.uniform(-0.5, 0.5, (n, 3))
+    s.pos = x.astype(np.float32)
+    s.vel = rng.normal(0.0, 1e-3, (n, 3)).astype(np.float32)
+    s.type, s.charge = np.zeros(n, np.int32), np.zeros(n, np.float32)
+    return s
+
+
+# 14,560 atoms fill a slot with three arrays, 43,680 with one; more go in several chunks, from
+# 29,128 (87,382) on copied by threads; 700,003 use every slot again
+@pytest.mark.parametrize("n,one_cpu", [((2,), 0), ((255,), 0), ((257, 3), 0), ((14560,), 0), ((14561,), 0), ((43681, 100), 0),
+                                       ((29128,), 0), ((87400,), 0), ((50000, 150003), 0), ((700003,), 0),
+                                       ((43681, 100), 1), ((50000, 150003), 1)], ids=str)
+def test_download_edges(n, one_cpu):
+    """What was uploaded inside the box comes back bit for bit, whole and one array at a time,
+    copied by threads and (one CPU to run on) without."""
+    import os
+    from md_gpu_amd.engine import Engine, _check, _ptr, lib
+    say("download", n, one_cpu)
+    sys_ = [lattice(k, 7 + i) for i, k in enumerate(n)]
+    pos, vel = np.concatenate([s.pos for s in sys_]), np.concatenate([s.vel for s in sys_])
+    e = Engine.from_system(sys_)
+    mine = os.sched_getaffinity(0)
+    try:
+        if one_cpu:
+            os.sched_setaffinity(0, {min(mine)})
+        p, v, f = e.download()
+        only = [np.full((len(pos), 3), np.nan, np.float32) for _ in range(3)]
+        for k in range(3):
+            _check(lib().md_download_state(e._h, *[_ptr(only[k]) if j == k else None for j in range(3)]))
+    finally:
+        os.sched_setaffinity(0, mine)
+    e.close()
+    assert np.array_equal(p, pos) and np.array_equal(v, vel) and np.isfinite(f).all()
+    assert np.array_equal(only[0], pos) and np.array_equal(only[1], vel) and np.array_equal(only[2], f)
