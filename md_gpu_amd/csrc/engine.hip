@@ -32,18 +32,19 @@
 #include "mdgpu/md_api.h"
 
 extern "C" hipError_t md_launch_rebuild(const BuildArgs& a, int commit, hipStream_t st);
-extern "C" hipError_t md_launch_force_trip(RepState* s, Gate* g, int nrep, hipStream_t st);
-extern "C" hipError_t md_launch_set_target(RepState* s, Gate* g, int nrep, long long nsteps, hipStream_t st);
+extern "C" hipError_t md_launch_force_trip(RepState* s, Gate* g, int nrep, int force, int* tmax, int ntmax,
+                                           const int* err, int* err_out, hipStream_t st);
 extern "C" hipError_t md_launch_step(const StepArgs& a, int lanes, int coul, hipStream_t st, hipEvent_t ev0,
                                      hipEvent_t ev1);
 extern "C" hipError_t md_launch_step_finalize(const StepArgs& a, int lanes, hipStream_t st);
 extern "C" hipError_t md_launch_kick(const KickArgs& a, hipStream_t st);
-extern "C" hipError_t md_launch_thermo_fix(ThState* th, const RepParam* rep, int nrep, int thermostat, float dt,
-                                           int mode, hipStream_t st);
+extern "C" hipError_t md_launch_thermo_end(ThState* th, int nrep, hipStream_t st);
 extern "C" hipError_t md_launch_fm_adjoint(const StepArgs& a, double* part, double* out, int lanes, int coul, int nt,
                                            hipStream_t st, hipEvent_t ev0, hipEvent_t ev1);
 extern "C" hipError_t md_launch_fm_fused(const StepArgs& a, double* part, double* out, int lanes, int coul, int nt,
                                          hipStream_t st, hipEvent_t ev0, hipEvent_t ev1);
+extern "C" hipError_t md_launch_run_begin(RunBeginArgs a, int npair, const void* const* src, void* const* dst,
+                                          const long long* bytes, hipStream_t st);
 extern "C" hipError_t md_launch_copies(int npair, const void* const* src, void* const* dst, const long long* bytes,
                                        hipStream_t st);
 extern "C" hipError_t md_launch_check_lists(const BuildArgs& a, int row_g, int* bad, hipStream_t st);
@@ -51,7 +52,6 @@ extern "C" hipError_t md_launch_state_sums(const float4* vel, const float4* forc
                                            hipStream_t st);
 extern "C" hipError_t md_launch_persist(const PersistArgs& a, int lanes, size_t shmem, hipStream_t st, hipEvent_t ev0,
                                         hipEvent_t ev1);
-extern "C" hipError_t md_launch_persist_clear(unsigned* flags, hipStream_t st);
 extern "C" hipError_t md_launch_settle(const SettleArgs& a, hipStream_t st);
 extern "C" int md_launch_pme(const PmeArgs& a, const PmeFftArgs* f, hipfftHandle r2c, hipfftHandle c2r, int energy,
                              hipStream_t st);
@@ -227,7 +227,7 @@ struct md_engine {
     DBuf<uint8_t> rperm;           // [S] per tile: atoms by decreasing row length
     DBuf<int> tmax;                // [2][S/64] builds' longest row / largest set per tile (running maxima)
     DBuf<int> tflag;               // [S/64] skin-check flag per tile (kick)
-    DBuf<RunReport> report;        // run progress for the host
+    RunReport* report = nullptr;   // run progress, in pinned host memory
     DBuf<int> badcnt;              // list invariant counters (md_check_lists)
     DBuf<int4> excl, ang_list;
     std::vector<int4> excl_bond;   // host copy of the 1-2 exclusions (md_set_topology)
@@ -315,6 +315,7 @@ struct md_engine {
         drop_graphs();
         drop_pme_plans();
         for (auto e : ev_pool) (void)hipEventDestroy(e);
+        if (report) (void)hipHostFree(report);
         if (st) (void)hipStreamDestroy(st);
     }
     void drop_graphs() {
@@ -834,8 +835,6 @@ int enqueue_step(md_engine* e, int energy_every, TimedSpan* ts, bool chain_mid =
     return MD_OK;
 }
 
-// Copy of the state a run may be rolled back to (restore = false), or back
-// (restore = true): one copy kernel for all arrays.
 // Pressure coupling changes the boxes on the device: copy them to the host
 // parameters (wrapping at download, cell set-up and later uploads use them).
 int sync_box(md_engine* e) {
@@ -845,45 +844,86 @@ int sync_box(md_engine* e) {
     return MD_OK;
 }
 
+// The arrays a run may have to be rolled back to, copied by one kernel (besides these the
+// replicas' states, thermostats and the gates).
 // Between runs every replica is at step e->step with phase 0, so its positions
 // are in pos[e->step & 1] (the other buffer is overwritten by the next step) and
 // only velocity Verlet reads the force array at a run's start (first half
 // kick): the snapshot holds what a replay from the run's start reads.
-int snapshot(md_engine* e, bool restore) {
-    struct Pair { void* a; void* b; size_t n; };
+struct Snapshot {
+    const void* live[12];
+    void* copy[12];
+    long long nb[12];
+    int n = 0;
+    template <class T>
+    void add(DBuf<T>& c, const DBuf<T>& l) {
+        live[n] = l.p;
+        copy[n] = c.p;
+        nb[n++] = (long long)l.bytes();
+    }
+};
+Snapshot snapshot_arrays(md_engine* e) {
     const int cb = (int)(e->step & 1);
-    DBuf<float4>& sp = cb ? e->snap_pos1 : e->snap_pos0;
-    std::vector<Pair> list = {
-        {sp.p, e->pos[cb].p, e->pos[cb].bytes()},
-        {e->snap_vel.p, e->vel.p, e->vel.bytes()},
-        {e->snap_ids.p, e->ids.p, e->ids.bytes()}, {e->snap_typ.p, e->typ.p, e->typ.bytes()},
-        {e->snap_slot_of.p, e->slot_of.p, e->slot_of.bytes()}, {e->snap_th.p, e->th.p, e->th.bytes()},
-        {e->snap_rst.p, e->rst.p, e->rst.bytes()}, {e->snap_gate.p, e->gate.p, e->gate.bytes()},
-        {e->snap_rep.p, e->rep.p, e->rep.bytes()}};   // the box, under pressure coupling
-    if (e->in.integrator == MD_VVERLET) list.push_back({e->snap_force.p, e->force.p, e->force.bytes()});
-    const int np = (int)list.size();
+    Snapshot s;
+    s.add(cb ? e->snap_pos1 : e->snap_pos0, e->pos[cb]);
+    s.add(e->snap_vel, e->vel);
+    s.add(e->snap_ids, e->ids);
+    s.add(e->snap_typ, e->typ);
+    s.add(e->snap_slot_of, e->slot_of);
+    s.add(e->snap_rep, e->rep);   // the box, under pressure coupling
+    if (e->in.integrator == MD_VVERLET) s.add(e->snap_force, e->force);
+    return s;
+}
+
+// Queue the start of a run: snapshot, cleared maxima, error word and barrier flags, targets.
+// nsteps < 0: the persistent kernel, which counts its steps itself.
+int run_begin(md_engine* e, long long nsteps) {
+    const Snapshot s = snapshot_arrays(e);
+    RunBeginArgs a{};
+    a.st = e->rst.p; a.snap_st = e->snap_rst.p; a.th = e->th.p; a.snap_th = e->snap_th.p;
+    a.gate = e->gate.p; a.snap_gate = e->snap_gate.p; a.rep = e->rep.p; a.err = e->err.p;
+    a.tmax = e->tmax.p; a.ntmax = nsteps < 0 ? 0 : 2LL * e->ntiles();
+    a.pk_flags = nsteps < 0 ? e->pk_flags.p : nullptr;
+    a.nsteps = nsteps; a.nrep = e->R; a.dt = e->in.dt; a.thermostat = e->in.thermostat;
+    a.th_begin = nsteps >= 0 && e->in.integrator == MD_VVERLET;
+    HIPCHECK(md_launch_run_begin(a, s.n, s.live, s.copy, s.nb, e->st));
+    return MD_OK;
+}
+
+// Queue the way back to the snapshot.
+int run_rollback(md_engine* e) {
+    Snapshot s = snapshot_arrays(e);
+    s.add(e->snap_th, e->th);
+    s.add(e->snap_rst, e->rst);
+    s.add(e->snap_gate, e->gate);
     const void* src[12];
     void* dst[12];
-    long long nb[12];
-    for (int k = 0; k < np; k++) {
-        src[k] = restore ? list[k].a : list[k].b;
-        dst[k] = restore ? list[k].b : list[k].a;
-        nb[k] = (long long)list[k].n;
+    for (int k = 0; k < s.n; k++) {
+        src[k] = s.copy[k];
+        dst[k] = const_cast<void*>(s.live[k]);
     }
-    HIPCHECK(md_launch_copies(np, src, dst, nb, e->st));
+    HIPCHECK(md_launch_copies(s.n, src, dst, s.nb, e->st));
     return MD_OK;
 }
 
-// The builds' longest rows and largest sets per tile accumulate in tmax until cleared.
-int clear_rowmax(md_engine* e) {
-    HIPCHECK(hipMemsetAsync(e->tmax.p, 0, e->tmax.bytes(), e->st));
+// Every list stale (force) and the builds' longest rows and largest sets per tile, which
+// accumulate in tmax, cleared.
+int list_begin(md_engine* e, bool force) {
+    HIPCHECK(md_launch_force_trip(e->rst.p, e->gate.p, e->R, force ? 1 : 0, e->tmax.p, 2 * e->ntiles(), nullptr, nullptr, e->st));
     return MD_OK;
 }
 
-// Queue the run report and its copy; the caller synchronises the stream.
-int queue_report(md_engine* e, RunReport* host) {
-    HIPCHECK(md_launch_report(e->rst.p, e->R, e->tmax.p, e->ntiles(), e->err.p, e->report.p, e->st));
-    HIPCHECK(hipMemcpyAsync(host, e->report.p, sizeof(RunReport), hipMemcpyDeviceToHost, e->st));
+// Every list stale: rebuilt when next needed.
+int force_trip(md_engine* e) {
+    HIPCHECK(md_launch_force_trip(e->rst.p, e->gate.p, e->R, 1, nullptr, 0, nullptr, nullptr, e->st));
+    return MD_OK;
+}
+
+// Queue the run report (into pinned memory) and wait for the stream.
+int read_report(md_engine* e, RunReport* r) {
+    HIPCHECK(md_launch_report(e->rst.p, e->R, e->tmax.p, e->ntiles(), e->err.p, e->report, e->st));
+    HIPCHECK(hipStreamSynchronize(e->st));
+    *r = *e->report;
     return MD_OK;
 }
 
@@ -893,12 +933,10 @@ bool overflowed(const md_engine* e, const RunReport& r) { return r.rowmax > e->c
 // growing the list capacities until every row and tile set fits.
 int full_rebuild(md_engine* e) {
     for (int attempt = 0; attempt < 6; attempt++) {
-        HIPCHECK(md_launch_force_trip(e->rst.p, e->gate.p, e->R, e->st));
-        CHECK(clear_rowmax(e));
+        CHECK(list_begin(e, true));
         CHECK(enqueue_rebuild(e, nullptr));
         RunReport rr;
-        CHECK(queue_report(e, &rr));
-        HIPCHECK(hipStreamSynchronize(e->st));
+        CHECK(read_report(e, &rr));
         if (!overflowed(e, rr)) return MD_OK;
         CHECK(grow_list(e, rr.rowmax, rr.setmax));
     }
@@ -907,11 +945,10 @@ int full_rebuild(md_engine* e) {
 
 // Queue a rebuild chain (it runs only for replicas whose list is stale).
 int refresh_lists(md_engine* e) {
-    CHECK(clear_rowmax(e));
+    CHECK(list_begin(e, false));
     CHECK(enqueue_rebuild(e, nullptr));
     RunReport rr;
-    CHECK(queue_report(e, &rr));
-    HIPCHECK(hipStreamSynchronize(e->st));
+    CHECK(read_report(e, &rr));
     if (overflowed(e, rr)) CHECK(full_rebuild(e));
     return MD_OK;
 }
@@ -984,9 +1021,14 @@ int md_create(md_engine** out, int device) {
         return fail(MD_E_HIP, "hipStreamCreate failed");
     }
     if (e->ljtab.alloc(64) || e->ctab.alloc(MD_CTAB + 1) || e->err.alloc(1) || e->fm_acc.alloc(2 + 2 * 64) ||
-        e->report.alloc(1) || e->badcnt.alloc(8) || e->sums.alloc(6)) {
+        e->badcnt.alloc(8) || e->sums.alloc(6)) {
         md_destroy(e);
         return MD_E_HIP;
+    }
+    if (hipHostMalloc((void**)&e->report, sizeof(RunReport), hipHostMallocCoherent) != hipSuccess) {
+        e->report = nullptr;
+        md_destroy(e);
+        return fail(MD_E_HIP, "hipHostMalloc failed");
     }
     if (!ev_get(e, 1)) {   // events 0 and 1 exist from here on: timing allocates no events later
         md_destroy(e);
@@ -1524,9 +1566,7 @@ int run_persist(md_engine* e, int nsteps, int energy_every, bool want_stats, int
             *use_tiles = 1;
             return MD_OK;
         }
-        CHECK(snapshot(e, false));
-        HIPCHECK(md_launch_persist_clear(e->pk_flags.p, e->st));
-        HIPCHECK(hipMemsetAsync(e->err.p, 0, sizeof(int), e->st));
+        CHECK(run_begin(e, -1));
         PersistArgs a{};
         a.pos[0] = e->pos[0].p; a.pos[1] = e->pos[1].p; a.vel = e->vel.p; a.force = e->force.p;
         a.ids = e->ids.p; a.typ = e->typ.p; a.ljtab = e->ljtab.p;
@@ -1544,12 +1584,13 @@ int run_persist(md_engine* e, int nsteps, int energy_every, bool want_stats, int
             if (!ev0 || !ev1) return fail(MD_E_HIP, "hipEventCreate failed");
         }
         HIPCHECK(md_launch_persist(a, G, persist_lds(e, cap_l), e->st, ev0, ev1));
-        int err = 0;
-        HIPCHECK(hipMemcpyAsync(&err, e->err.p, sizeof(int), hipMemcpyDeviceToHost, e->st));
+        // the tile path's lists were built for earlier positions: stale after a run without errors
+        HIPCHECK(md_launch_force_trip(e->rst.p, e->gate.p, e->R, 1, nullptr, 0, e->err.p, &e->report->err, e->st));
         HIPCHECK(hipStreamSynchronize(e->st));
+        const int err = e->report->err;
         if (err & MD_PK_ERR_WAIT) return fail(MD_E_HIP, "persistent kernel: a grid barrier wait timed out");
         if (err & MD_PK_ERR_ROWS) {   // a row outgrew its length: replay the run with longer rows
-            CHECK(snapshot(e, true));
+            CHECK(run_rollback(e));
             HIPCHECK(hipStreamSynchronize(e->st));
             e->pk_cap = 2 * cap_l;
             e->pk_replays++;
@@ -1566,8 +1607,6 @@ int run_persist(md_engine* e, int nsteps, int energy_every, bool want_stats, int
         e->pk_runs++;
         break;
     }
-    // the tile path's lists were built for earlier positions
-    HIPCHECK(md_launch_force_trip(e->rst.p, e->gate.p, e->R, e->st));
     return MD_OK;
 }
 
@@ -1605,11 +1644,7 @@ int md_run(md_engine* e, int nsteps, int energy_every, md_step_stats* stats) {
     }
     int retries = 0;
     while (tiles) {   // one attempt; repeated only after a list-capacity overflow
-        CHECK(snapshot(e, false));
-        CHECK(clear_rowmax(e));
-        HIPCHECK(hipMemsetAsync(e->err.p, 0, sizeof(int), e->st));
-        HIPCHECK(md_launch_set_target(e->rst.p, e->gate.p, e->R, nsteps, e->st));
-        if (vv) HIPCHECK(md_launch_thermo_fix(e->th.p, e->rep.p, e->R, e->in.thermostat, e->in.dt, 0, e->st));
+        CHECK(run_begin(e, nsteps));
         if (fused) {
             // leapfrog-form velocity Verlet: a valid list, then the first half-kick and drift of
             // the run's first step; every step kernel then ends one step and begins the next
@@ -1626,8 +1661,7 @@ int md_run(md_engine* e, int nsteps, int energy_every, md_step_stats* stats) {
                 CHECK(enqueue_step(e, energy_every, &span, true));
             }
             launched = nsteps;
-            CHECK(queue_report(e, &rr));
-            HIPCHECK(hipStreamSynchronize(e->st));
+            CHECK(read_report(e, &rr));
             for (auto& pr : span.steps) {
                 float ms = 0;
                 HIPCHECK(hipEventElapsedTime(&ms, pr.first, pr.second));
@@ -1647,8 +1681,7 @@ int md_run(md_engine* e, int nsteps, int energy_every, md_step_stats* stats) {
                 const long long nbl = std::max(1LL, (want + ce - 1) / ce);
                 CHECK(launch_blocks(e, energy_every, nbl));
                 launched += nbl * ce;
-                CHECK(queue_report(e, &rr));
-                HIPCHECK(hipStreamSynchronize(e->st));
+                CHECK(read_report(e, &rr));
                 const long long lag = target - rr.min_step;
                 if (lag <= 0 || overflowed(e, rr) || rr.err) break;
                 want = (long long)std::ceil(lag * std::max(e->queue_ratio, 1.0) * 1.1) + 1;
@@ -1659,7 +1692,7 @@ int md_run(md_engine* e, int nsteps, int energy_every, md_step_stats* stats) {
             if (++retries > 4)
                 return fail(MD_E_CAPACITY, "neighbor list capacity keeps overflowing (rows %d > %d or sets %d > %d)",
                             rr.rowmax, e->cap, rr.setmax, e->jcap);
-            CHECK(snapshot(e, true));
+            CHECK(run_rollback(e));
             CHECK(grow_list(e, rr.rowmax, rr.setmax));
             CHECK(full_rebuild(e));
             continue;
@@ -1682,7 +1715,7 @@ int md_run(md_engine* e, int nsteps, int energy_every, md_step_stats* stats) {
     }
     if (tiles && vv && !fused) {   // (leapfrog form: the last step kernel left full-step velocities)
         HIPCHECK(md_launch_kick(kick_args(e, 0), e->st));
-        HIPCHECK(md_launch_thermo_fix(e->th.p, e->rep.p, e->R, e->in.thermostat, e->in.dt, 1, e->st));
+        HIPCHECK(md_launch_thermo_end(e->th.p, e->R, e->st));
     }
     if (stats) {
         std::vector<StatRec> rec((size_t)nsteps * e->R);
@@ -1795,7 +1828,7 @@ int md_set_list_capacity(md_engine* e, int cap) {
     e->pk_req = cap;
     e->pk_cap = 0;
     e->pk_off = false;
-    HIPCHECK(md_launch_force_trip(e->rst.p, e->gate.p, e->R, e->st));   // every list is rebuilt when next needed
+    CHECK(force_trip(e));   // every list is rebuilt when next needed
     HIPCHECK(hipStreamSynchronize(e->st));
     return MD_OK;
 }
@@ -1932,7 +1965,7 @@ int md_autotune(md_engine* e, int nsteps, double* best_ms) {
             CHECK(restore());
             HIPCHECK(hipEventRecord(t0, e->st));
             for (int k = 0; k < 3; k++) {
-                HIPCHECK(md_launch_force_trip(e->rst.p, e->gate.p, e->R, e->st));
+                CHECK(force_trip(e));
                 CHECK(enqueue_rebuild(e, nullptr));
             }
             HIPCHECK(hipEventRecord(t1, e->st));
@@ -2062,7 +2095,7 @@ int md_rebuild_bench(md_engine* e, int reps, double* ms) {
     hipEvent_t t0 = ev_get(e, 0), t1 = ev_get(e, 1);
     HIPCHECK(hipEventRecord(t0, e->st));
     for (int k = 0; k < reps; k++) {
-        HIPCHECK(md_launch_force_trip(e->rst.p, e->gate.p, e->R, e->st));
+        CHECK(force_trip(e));
         CHECK(enqueue_rebuild(e, nullptr));
     }
     HIPCHECK(hipEventRecord(t1, e->st));

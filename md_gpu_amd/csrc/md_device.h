@@ -295,6 +295,33 @@ struct RunReport {
     int pad;
 };
 
+// Pairs of buffers to copy, 16-byte units each.
+struct CopyPlan {
+    const float4* src[12];
+    float4* dst[12];
+    long long n16[12];
+    int npair;
+};
+
+// Start of a run (k_run_begin)
+struct RunBeginArgs {
+    CopyPlan copy;          // the arrays of the snapshot (without the three below)
+    RepState* st;
+    RepState* snap_st;
+    ThState* th;
+    ThState* snap_th;
+    Gate* gate;
+    Gate* snap_gate;
+    const RepParam* rep;
+    int* tmax;
+    long long ntmax;        // list maxima to clear
+    int* err;
+    unsigned* pk_flags;     // persistent kernel: barrier flags, else nullptr
+    long long nsteps;       // < 0: targets and gates stay (the persistent kernel keeps its own count)
+    int nrep, th_begin, thermostat;
+    float dt;
+};
+
 // Streaming kernel of velocity Verlet (begin of step): v = S v + F dt/2m; x += v dt
 struct KickArgs {
     float4* pos[2];

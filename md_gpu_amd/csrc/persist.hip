@@ -422,13 +422,3 @@ extern "C" hipError_t md_launch_persist(const PersistArgs& a, int lanes, size_t 
     if (rc != hipSuccess) return rc;
     return hipGetLastError();
 }
-
-// zero the barrier flags before a launch (a fill kernel, so a caller may capture it)
-__global__ void k_persist_clear(unsigned* flags) {
-    if (threadIdx.x < 2 * MD_PK_WG) flags[threadIdx.x] = 0u;
-}
-
-extern "C" hipError_t md_launch_persist_clear(unsigned* flags, hipStream_t st) {
-    hipLaunchKernelGGL(k_persist_clear, dim3(1), dim3(2 * MD_PK_WG), 0, st, flags);
-    return hipGetLastError();
-}

@@ -798,28 +798,14 @@ __global__ __launch_bounds__(256) void k_vv_kick(const KickArgs a) {
     if (lane == 0) a.tflag[s >> 6] = tb ? 1 : 0;
 }
 
-// Thermostat bookkeeping at run boundaries (one workgroup).
-//   mode 0 (velocity-Verlet run start): begin-of-step half from ke2_cur -> S
-//   mode 1 (velocity-Verlet run end):   restore the state after the end-of-step half
-__global__ void k_thermo_fix(ThState* th, const RepParam* rep, int nrep, int thermostat, float dt, int mode) {
+// Velocity-Verlet run end (one workgroup): the thermostat state after the end-of-step half.
+__global__ void k_thermo_end(ThState* th, int nrep) {
     for (int r = threadIdx.x; r < nrep; r += blockDim.x) {
         ThState& t = th[r];
-        if (mode == 0) {
-            if (thermostat == 2) {
-                double K = 0.5 * t.ke2_cur, xi = t.xi, vxi = t.vxi;
-                double s = nh_half(xi, vxi, K, rep[r].nf, rep[r].kT0, rep[r].Q, dt);
-                t.xi = xi;
-                t.vxi = vxi;
-                t.S = s;
-            } else {
-                t.S = 1.0;
-            }
-        } else {
-            t.xi = t.xi_end;
-            t.vxi = t.vxi_end;
-            t.S = 1.0;
-            t.S_end = 1.0;
-        }
+        t.xi = t.xi_end;
+        t.vxi = t.vxi_end;
+        t.S = 1.0;
+        t.S_end = 1.0;
     }
 }
 
@@ -869,34 +855,8 @@ __global__ __launch_bounds__(256) void k_kick_finalize(const KickArgs a, int wid
     }
 }
 
-// Start of a run: target = step + nsteps for every replica; recount the gates.
-__global__ void k_set_target(RepState* st, Gate* g, int nrep, long long nsteps) {
-    __shared__ int cnt[3];
-    if (threadIdx.x < 3) cnt[threadIdx.x] = 0;
-    __syncthreads();
-    int ns = 0, nr = 0, nf = 0;
-    for (int r = threadIdx.x; r < nrep; r += blockDim.x) {
-        RepState& s = st[r];
-        s.start = s.step;
-        s.target = s.step + nsteps;
-        const bool st_ = stale(s);
-        ns += st_;
-        nr += !st_ && s.phase == 0 && s.step < s.target;
-        nf += !st_ && s.phase == 1;
-    }
-    atomicAdd(&cnt[0], ns);
-    atomicAdd(&cnt[1], nr);
-    atomicAdd(&cnt[2], nf);
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        g->n_stale = cnt[0];
-        g->n_run = cnt[1];
-        g->n_force = cnt[2];
-    }
-}
-
 // Run report: one workgroup reduces the replicas' step counters and the
-// builds' maxima (see RunReport).
+// builds' maxima (see RunReport) into pinned host memory.
 __global__ __launch_bounds__(1024) void k_report(const RepState* st, int nrep, const int* tmax, int ntiles,
                                                  const int* err, RunReport* out) {
     constexpr int NT = 1024, NW = NT / 64, U = 4;
@@ -948,20 +908,80 @@ __global__ __launch_bounds__(1024) void k_report(const RepState* st, int nrep, c
     }
 }
 
-// Copy of the engine state a run may have to be rolled back to (one launch;
-// the caller passes matching buffer pairs).  nbytes per pair, 16-byte units.
-struct CopyPlan {
-    const float4* src[12];
-    float4* dst[12];
-    long long n16[12];   // 16-byte units per pair
-    int npair;
-};
-__global__ __launch_bounds__(256) void k_copy_plan(const CopyPlan c) {
-    const long long stride = (long long)gridDim.x * blockDim.x;
+// Copies between pairs of buffers, in 16-byte units (the caller passes matching pairs).
+__device__ __forceinline__ void copy_pairs(const CopyPlan& c, long long first, long long stride) {
     for (int k = 0; k < c.npair; k++) {
         const float4* __restrict__ s = c.src[k];
         float4* __restrict__ d = c.dst[k];
-        for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < c.n16[k]; i += stride) d[i] = s[i];
+        for (long long i = first; i < c.n16[k]; i += stride) d[i] = s[i];
+    }
+}
+__global__ __launch_bounds__(256) void k_copy_plan(const CopyPlan c) {
+    copy_pairs(c, (long long)blockIdx.x * blockDim.x + threadIdx.x, (long long)gridDim.x * blockDim.x);
+}
+
+// Start of a run, in one launch (it was five: copies, fills of the list maxima and the error
+// word, thermostat, targets; 21 us of kernels and as many gaps): the copy of the state that a
+// run may be rolled back to, and
+//   list maxima, the error word and the persistent kernel's barrier flags cleared
+//   target = step + nsteps for every replica, gates recounted (a.nsteps < 0: neither)
+//   velocity Verlet's begin-of-step thermostat half from ke2_cur -> S (a.th_begin)
+// The last workgroup copies the replicas' states, thermostats and the gates itself before it
+// changes them; the others share the arrays.
+__global__ __launch_bounds__(256) void k_run_begin(const RunBeginArgs a) {
+    const int nb = (int)gridDim.x - 1;
+    if ((int)blockIdx.x < nb) {
+        const long long first = (long long)blockIdx.x * blockDim.x + threadIdx.x, stride = (long long)nb * blockDim.x;
+        copy_pairs(a.copy, first, stride);
+        for (long long i = first; i < a.ntmax; i += stride) a.tmax[i] = 0;
+        return;
+    }
+    __shared__ int cnt[3];
+    if (threadIdx.x < 3) cnt[threadIdx.x] = 0;
+    if (threadIdx.x == 3) *a.err = 0;
+    if (a.pk_flags)
+        for (int i = threadIdx.x; i < 2 * MD_PK_WG; i += blockDim.x) a.pk_flags[i] = 0u;
+    const Gate g0 = *a.gate;
+    __syncthreads();
+    int ns = 0, nr = 0, nf = 0;
+    for (int r = threadIdx.x; r < a.nrep; r += blockDim.x) {
+        RepState s = a.st[r];
+        ThState t = a.th[r];
+        a.snap_st[r] = s;
+        a.snap_th[r] = t;
+        if (a.nsteps < 0) continue;
+        s.start = s.step;
+        s.target = s.step + a.nsteps;
+        a.st[r].start = s.start;
+        a.st[r].target = s.target;
+        const bool st_ = stale(s);
+        ns += st_;
+        nr += !st_ && s.phase == 0 && s.step < s.target;
+        nf += !st_ && s.phase == 1;
+        if (a.th_begin) {
+            if (a.thermostat == 2) {
+                double K = 0.5 * t.ke2_cur, xi = t.xi, vxi = t.vxi;
+                const double sc = nh_half(xi, vxi, K, a.rep[r].nf, a.rep[r].kT0, a.rep[r].Q, a.dt);
+                t.xi = xi;
+                t.vxi = vxi;
+                t.S = sc;
+            } else {
+                t.S = 1.0;
+            }
+            a.th[r] = t;
+        }
+    }
+    if (ns) atomicAdd(&cnt[0], ns);
+    if (nr) atomicAdd(&cnt[1], nr);
+    if (nf) atomicAdd(&cnt[2], nf);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        *a.snap_gate = g0;
+        if (a.nsteps >= 0) {
+            a.gate->n_stale = cnt[0];
+            a.gate->n_run = cnt[1];
+            a.gate->n_force = cnt[2];
+        }
     }
 }
 
@@ -1034,14 +1054,8 @@ extern "C" hipError_t md_launch_kick(const KickArgs& a, hipStream_t st) {
     return hipGetLastError();
 }
 
-extern "C" hipError_t md_launch_thermo_fix(ThState* th, const RepParam* rep, int nrep, int thermostat, float dt,
-                                           int mode, hipStream_t st) {
-    hipLaunchKernelGGL(k_thermo_fix, dim3(1), dim3(256), 0, st, th, rep, nrep, thermostat, dt, mode);
-    return hipGetLastError();
-}
-
-extern "C" hipError_t md_launch_set_target(RepState* s, Gate* g, int nrep, long long nsteps, hipStream_t st) {
-    hipLaunchKernelGGL(k_set_target, dim3(1), dim3(256), 0, st, s, g, nrep, nsteps);
+extern "C" hipError_t md_launch_thermo_end(ThState* th, int nrep, hipStream_t st) {
+    hipLaunchKernelGGL(k_thermo_end, dim3(1), dim3(256), 0, st, th, nrep);
     return hipGetLastError();
 }
 
@@ -1081,21 +1095,36 @@ extern "C" hipError_t md_launch_report(const RepState* st, int nrep, const int* 
     return hipGetLastError();
 }
 
-// copies: npair (src, dst, bytes) with 16-byte aligned sizes
-extern "C" hipError_t md_launch_copies(int npair, const void* const* src, void* const* dst, const long long* bytes,
-                                       hipStream_t st) {
-    if (npair < 0 || npair > 12) return hipErrorInvalidValue;
-    CopyPlan c{};
+// copies: npair (src, dst, bytes) with 16-byte aligned sizes; the longest in 16-byte units, or -1
+static long long plan_copies(int npair, const void* const* src, void* const* dst, const long long* bytes, CopyPlan& c) {
+    if (npair < 0 || npair > 12) return -1;
     long long most = 0;
     for (int k = 0; k < npair; k++) {
-        if (bytes[k] % 16) return hipErrorInvalidValue;
+        if (bytes[k] % 16) return -1;
         c.src[k] = static_cast<const float4*>(src[k]);
         c.dst[k] = static_cast<float4*>(dst[k]);
         c.n16[k] = bytes[k] / 16;
         most = std::max(most, c.n16[k]);
     }
     c.npair = npair;
+    return most;
+}
+
+extern "C" hipError_t md_launch_copies(int npair, const void* const* src, void* const* dst, const long long* bytes,
+                                       hipStream_t st) {
+    CopyPlan c{};
+    const long long most = plan_copies(npair, src, dst, bytes, c);
+    if (most < 0) return hipErrorInvalidValue;
     const int grid = (int)std::max(1LL, std::min(2048LL, (most + 255) / 256));
     hipLaunchKernelGGL(k_copy_plan, dim3(grid), dim3(256), 0, st, c);
+    return hipGetLastError();
+}
+
+extern "C" hipError_t md_launch_run_begin(RunBeginArgs a, int npair, const void* const* src, void* const* dst,
+                                          const long long* bytes, hipStream_t st) {
+    const long long most = plan_copies(npair, src, dst, bytes, a.copy);
+    if (most < 0) return hipErrorInvalidValue;
+    const int grid = (int)std::max(1LL, std::min(2048LL, (most + 255) / 256)) + 1;
+    hipLaunchKernelGGL(k_run_begin, dim3(grid), dim3(256), 0, st, a);
     return hipGetLastError();
 }
