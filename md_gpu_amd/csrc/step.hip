@@ -19,8 +19,14 @@
 // its row of 16-bit local indices (the LDS-staged tiles of
 // src/pair_forces_tiles.cu:98-155, restricted to the atoms that are
 // neighbors).  Per-atom sums are reduced across the G lanes with DPP row
-// moves; KE / energies / virial and the skin-check flag are reduced per
-// workgroup into FP64 partial slots, one per tile (plain stores).
+// moves; the tile's last wavefront (the shortest rows) then integrates all 64
+// atoms, a lane each, and with bonded terms it computes the bonds before its
+// rows, the wavefront before it the angles: the kernel is bound by VALU issue
+// (196,608 water atoms: 100 % busy, Ar-Xe replicas 84 %), and with 64 / G active
+// lanes these ends cost every wavefront as much as full ones (40 steps of water
+// 7.94 -> 7.63 ms with them on one wavefront, 60 steps of 512 Ar-Xe replicas
+// 15.3 -> 14.8 ms, the same bits).  KE / energies / virial and the skin-check flag
+// are reduced per workgroup into FP64 partial slots, one per tile (plain stores).
 // k_step_finalize, launched next, reduces a replica's slots and computes its
 // temperature, thermostat update and statistics record, folds the skin-check
 // flag into the list state and advances the step counter.  No device-scope
@@ -275,6 +281,7 @@ __global__ __launch_bounds__(64 * G, COUL == 3 ? 5 : 4) void k_step(const StepAr
     static_assert(MD_CTAB == 256, "the table is loaded by the first 256 threads");
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int sub = tid & (G - 1);
+    __shared__ float4 s_f[64];            // force of the tile's atoms
     const int tile = xcd_block(blockIdx.x, gridDim.x);   // tiles contiguous per XCD
     if (a.prefilter) {
         // Many replicas, no deferred finalize: a tile whose replica does not step in
@@ -324,11 +331,22 @@ __global__ __launch_bounds__(64 * G, COUL == 3 ? 5 : 4) void k_step(const StepAr
     const uint4* __restrict__ row4 = reinterpret_cast<const uint4*>(a.nl16 + (size_t)slot * a.cap);
     const uint4 q0 = row4[sub];
     const uint4 q1 = row4[(a.cap >= 16 * G ? G : 0) + sub];   // block 1 when the capacity holds one
-    float4 v_e = make_float4(0.f, 0.f, 0.f, 0.f), pb_e = v_e, fr_e = v_e;
-    if (sub == 0) {
-        v_e = a.vel[slot];
-        pb_e = a.pos_build[slot];
-        if (COUL == 2 && a.frec) fr_e = a.frec[slot];   // PME: long-range force of the atom
+    // The last wavefront (the tile's shortest rows) ends the step of all 64 atoms, a lane each;
+    // with bonded terms it also computes the bonds, and the one before it the angles.
+    const int uw = __builtin_amdgcn_readfirstlane(wave);
+    const bool last = uw == NW - 1;
+    const int eslot = tile * 64 + lane;
+    float4 v_e = make_float4(0.f, 0.f, 0.f, 0.f), pb_e = v_e, fr_e = v_e, xea = v_e, xeb = v_e;
+    int eid = -1;
+    if (uw >= NW - 2) {
+        eid = a.ids[eslot];
+        xea = a.pos[0][eslot];
+        xeb = a.pos[1][eslot];
+        if (last) {
+            v_e = a.vel[eslot];
+            pb_e = a.pos_build[eslot];
+            if (COUL == 2 && a.frec) fr_e = a.frec[eslot];   // PME: long-range force of the atom
+        }
     }
     loads_issued();
     if (tid < 64) s_lj[tid] = lj_v;
@@ -479,82 +497,125 @@ __global__ __launch_bounds__(64 * G, COUL == 3 ? 5 : 4) void k_step(const StepAr
             evi += (double)(ff * rsq);
         }
     };
+    // Bonded terms of an atom: at most four bonds and four angles, each as the vector and
+    // factor that lane k of the atom's group adds after its row (zeros past the last).
+    float4* s_bd = s_j + a.jcap + 1;   // [4 bonds, 4 angles][64], allocated with bonded terms
+    double ebo = 0.0, ean = 0.0, bvi = 0.0;
+    if (a.bonded && uw >= NW - 2) {
+        const float4 xe = cb ? xeb : xea;
+        if (last) {
+            const int nb = eid >= 0 ? a.nbond[eid] : 0;
+            for (int b = 0; b < 4; b++) {          // src/bonded_forces.cu:50-84
+                float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
+                if (b < nb) {
+                    const uint32_t e = a.bond_list[(size_t)eid * 4 + b];
+                    const int js = a.slot_of[e & MD_JMASK];
+                    const int bt = (int)(e >> MD_JBITS);
+                    const float4 pj = pin[js];
+                    const float dx = minimg(xe.x - pj.x, L0, Li0);
+                    const float dy = minimg(xe.y - pj.y, L1, Li1);
+                    const float dz = minimg(xe.z - pj.z, L2, Li2);
+                    const float rsq = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
+                    const float kk = a.bk2[bt], r0 = a.br0[bt];
+                    const float fa = kk * (r0 * __builtin_amdgcn_rsqf(rsq) - 1.0f);
+                    o = make_float4(dx, dy, dz, fa);
+                    if (ENMODE != 0 && en) {
+                        const float dr = sqrtf(rsq) - r0;
+                        ebo += 0.25 * (double)kk * (double)dr * (double)dr;   // each bond is seen from both atoms
+                        bvi += 0.5 * (double)(fa * rsq);
+                    }
+                }
+                s_bd[b * 64 + lane] = o;
+            }
+        } else {
+            const int na = eid >= 0 ? a.nang[eid] : 0;
+            for (int q = 0; q < 4; q++) {          // src/bonded_forces.cu:119-188
+                float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
+                if (q < na) {
+                    const int4 e = a.ang_list[(size_t)eid * 4 + q];
+                    const int role = e.x & 0xff, at = e.x >> 8;
+                    const float4 pA = pin[a.slot_of[e.y]];
+                    const float4 pk = pin[a.slot_of[e.z]];
+                    float4 pi = xe, pc = pA;
+                    if (role == 1) { pi = pA; pc = xe; }
+                    float ax = minimg(pi.x - pc.x, L0, Li0), ay = minimg(pi.y - pc.y, L1, Li1), az = minimg(pi.z - pc.z, L2, Li2);
+                    float ai_ = __builtin_amdgcn_rsqf(fmaf(az, az, fmaf(ay, ay, ax * ax)));
+                    float bx = minimg(pk.x - pc.x, L0, Li0), by = minimg(pk.y - pc.y, L1, Li1), bz = minimg(pk.z - pc.z, L2, Li2);
+                    float bi = __builtin_amdgcn_rsqf(fmaf(bz, bz, fmaf(by, by, bx * bx)));
+                    const float ab = fmaf(az, bz, fmaf(ay, by, ax * bx));
+                    float cang = ab * ai_ * bi;
+                    cang = fminf(fmaxf(cang, -0.9999999f), 0.9999999f);
+                    const float th = acosf(cang);
+                    const float fk = a.ak2[at] * (th - a.at0[at]) * __builtin_amdgcn_rsqf(1.0f - cang * cang) * ai_ * bi;
+                    const float ca = ab * ai_ * ai_;
+                    float gx = bx - ca * ax, gy = by - ca * ay, gz = bz - ca * az;
+                    if (role == 1) {
+                        const float cbb = ab * bi * bi;
+                        gx = cbb * bx - ax - gx;
+                        gy = cbb * by - ay - gy;
+                        gz = cbb * bz - az - gz;
+                    }
+                    o = make_float4(gx, gy, gz, fk);
+                    if (ENMODE != 0 && en) {
+                        const double d = (double)th - (double)a.at0[at];
+                        ean += (0.5 / 3.0) * (double)a.ak2[at] * d * d;   // each angle is seen from 3 atoms
+                    }
+                }
+                s_bd[(4 + q) * 64 + lane] = o;
+            }
+        }
+    }
     // lane groups hold the tile's atoms by decreasing row length (rperm)
     if (ENMODE != 0 && en)
         walk_row_sorted<G>(s_j, row4, nn, sub, q0, q1, [&](const float4& pj) { pair(pj, std::true_type{}); });
     else
         walk_row_sorted<G>(s_j, row4, nn, sub, q0, q1, [&](const float4& pj) { pair(pj, std::false_type{}); });
 
-    // bonded terms (lanes of the atom's group share them)
-    double ebo = 0.0, ean = 0.0, bvi = 0.0;
-    if (a.bonded && active) {
-        const int nb = a.nbond[id];
-        for (int b = sub; b < nb; b += G) {          // src/bonded_forces.cu:50-84
-            const uint32_t e = a.bond_list[(size_t)id * 4 + b];
-            const int js = a.slot_of[e & MD_JMASK];
-            const int bt = (int)(e >> MD_JBITS);
-            const float4 pj = pin[js];
-            const float dx = minimg(xi.x - pj.x, L0, Li0);
-            const float dy = minimg(xi.y - pj.y, L1, Li1);
-            const float dz = minimg(xi.z - pj.z, L2, Li2);
-            const float rsq = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
-            const float kk = a.bk2[bt], r0 = a.br0[bt];
-            const float fa = kk * (r0 * __builtin_amdgcn_rsqf(rsq) - 1.0f);
-            fx = fmaf(fa, dx, fx);
-            fy = fmaf(fa, dy, fy);
-            fz = fmaf(fa, dz, fz);
-            if (ENMODE != 0 && en) {
-                const float dr = sqrtf(rsq) - r0;
-                ebo += 0.25 * (double)kk * (double)dr * (double)dr;   // each bond is seen from both atoms
-                bvi += 0.5 * (double)(fa * rsq);
-            }
-        }
-        const int na = a.nang[id];
-        for (int q = sub; q < na; q += G) {          // src/bonded_forces.cu:119-188
-            const int4 e = a.ang_list[(size_t)id * 4 + q];
-            const int role = e.x & 0xff, at = e.x >> 8;
-            const float4 pA = pin[a.slot_of[e.y]];
-            const float4 pk = pin[a.slot_of[e.z]];
-            float4 pi = xi, pc = pA;
-            if (role == 1) { pi = pA; pc = xi; }
-            float ax = minimg(pi.x - pc.x, L0, Li0), ay = minimg(pi.y - pc.y, L1, Li1), az = minimg(pi.z - pc.z, L2, Li2);
-            float ai_ = __builtin_amdgcn_rsqf(fmaf(az, az, fmaf(ay, ay, ax * ax)));
-            float bx = minimg(pk.x - pc.x, L0, Li0), by = minimg(pk.y - pc.y, L1, Li1), bz = minimg(pk.z - pc.z, L2, Li2);
-            float bi = __builtin_amdgcn_rsqf(fmaf(bz, bz, fmaf(by, by, bx * bx)));
-            const float ab = fmaf(az, bz, fmaf(ay, by, ax * bx));
-            float cang = ab * ai_ * bi;
-            cang = fminf(fmaxf(cang, -0.9999999f), 0.9999999f);
-            const float th = acosf(cang);
-            const float fk = a.ak2[at] * (th - a.at0[at]) * __builtin_amdgcn_rsqf(1.0f - cang * cang) * ai_ * bi;
-            const float ca = ab * ai_ * ai_;
-            float gx = bx - ca * ax, gy = by - ca * ay, gz = bz - ca * az;
-            if (role == 1) {
-                const float cbb = ab * bi * bi;
-                gx = cbb * bx - ax - gx;
-                gy = cbb * by - ay - gy;
-                gz = cbb * bz - az - gz;
-            }
-            fx = fmaf(fk, gx, fx);
-            fy = fmaf(fk, gy, fy);
-            fz = fmaf(fk, gz, fz);
-            if (ENMODE != 0 && en) {
-                const double d = (double)th - (double)a.at0[at];
-                ean += (0.5 / 3.0) * (double)a.ak2[at] * d * d;   // each angle is seen from 3 atoms
-            }
+    if (a.bonded) {   // the atom's lanes take its bonded terms
+        __syncthreads();
+        if (sub < 4) {
+            const float4 b = s_bd[sub * 64 + (slot & 63)], q = s_bd[(4 + sub) * 64 + (slot & 63)];
+            fx = fmaf(b.w, b.x, fx);
+            fy = fmaf(b.w, b.y, fy);
+            fz = fmaf(b.w, b.z, fz);
+            fx = fmaf(q.w, q.x, fx);
+            fy = fmaf(q.w, q.y, fy);
+            fz = fmaf(q.w, q.z, fz);
         }
     }
     fx = group_sum<G>(fx);
     fy = group_sum<G>(fy);
     fz = group_sum<G>(fz);
+    if (sub == 0) s_f[slot & 63] = make_float4(fx, fy, fz, 0.0f);
+    if (ENMODE != 0 && en) {
+        double vals[MD_NSTAT] = {};
+        vals[ACC_LJ] = elj;
+        vals[ACC_COUL] = eco;
+        vals[ACC_BOND] = ebo;
+        vals[ACC_ANGLE] = ean;
+        vals[ACC_VIR] = evi + 2.0 * bvi;
+#pragma unroll
+        for (int k = 0; k < MD_NSTAT - 2; k++)
+            if (k != ACC_KE2) vals[k] = wave_sum_d(vals[k]);
+        if (lane == 0) {
+#pragma unroll
+            for (int k = 0; k < MD_NSTAT; k++) s_red[wave][k] = vals[k];
+        }
+    }
+    __syncthreads();
+    if (!last) return;
     double dke = 0.0;
     int trip = 0;
-    if (active && sub == 0) {
+    if (eid >= 0) {
+        const float4 xe = cb ? xeb : xea;
+        const float4 fe = s_f[lane];
+        fx = fe.x, fy = fe.y, fz = fe.z;
         if (COUL == 2 && a.frec) {
             fx += fr_e.x;
             fy += fr_e.y;
             fz += fr_e.z;
         }
-        a.force[slot] = make_float4(fx, fy, fz, 0.0f);
+        a.force[eslot] = make_float4(fx, fy, fz, 0.0f);
         if (a.mode == MODE_LF) {
             float4 v = v_e;                 // loaded in the first round trip
             const float4 pb = pb_e;         // for the skin check
@@ -579,10 +640,10 @@ __global__ __launch_bounds__(64 * G, COUL == 3 ? 5 : 4) void k_step(const StepAr
                 v.z = fmaf(fz, massif, v.z) * lam;
                 dke = ((double)v.x * v.x + (double)v.y * v.y + (double)v.z * v.z) / (double)v.w;
             }
-            a.vel[slot] = v;
+            a.vel[eslot] = v;
             if (drift) {
-                const float x = fmaf(v.x, a.dt, xi.x), y = fmaf(v.y, a.dt, xi.y), z = fmaf(v.z, a.dt, xi.z);
-                pout[slot] = make_float4(x, y, z, xi.w);
+                const float x = fmaf(v.x, a.dt, xe.x), y = fmaf(v.y, a.dt, xe.y), z = fmaf(v.z, a.dt, xe.z);
+                pout[eslot] = make_float4(x, y, z, xe.w);
                 if (!a.baro) {
                     const float ddx = minimg(x - pb.x, L0, Li0), ddy = minimg(y - pb.y, L1, Li1), ddz = minimg(z - pb.z, L2, Li2);
                     if (fmaf(ddz, ddz, fmaf(ddy, ddy, ddx * ddx)) >= a.skin2q) trip = 1;   // src/neighborlist.cu:174
@@ -605,43 +666,30 @@ __global__ __launch_bounds__(64 * G, COUL == 3 ? 5 : 4) void k_step(const StepAr
             v.x = fmaf(fx, h, v.x);
             v.y = fmaf(fy, h, v.y);
             v.z = fmaf(fz, h, v.z);
-            a.vel[slot] = v;
+            a.vel[eslot] = v;
             dke = ((double)v.x * v.x + (double)v.y * v.y + (double)v.z * v.z) / (double)v.w;
         }
     }
-    // the workgroup's partial sums go to the tile's slot (plain stores; the next
-    // kernel reduces the replica's slots)
-    double vals[MD_NSTAT] = {dke, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-    if (ENMODE != 0 && en) {
-        vals[ACC_LJ] = elj;
-        vals[ACC_COUL] = eco;
-        vals[ACC_BOND] = ebo;
-        vals[ACC_ANGLE] = ean;
-        vals[ACC_VIR] = evi + 2.0 * bvi;
-    }
-#pragma unroll
-    for (int k = 0; k < MD_NSTAT - 2; k++) {
-        if (ENMODE == 0 && k != ACC_KE2) continue;
-        vals[k] = wave_sum_d(vals[k]);
-    }
+    // the tile's partial sums go to its slot (plain stores; the next kernel reduces the
+    // replica's slots)
+    const double ke2 = wave_sum_d(dke);
     const unsigned long long tb = __ballot(trip != 0);
-    if (lane == 0) {
+    if (lane < MD_NSTAT) {
+        double t = 0.0;
+        if (ENMODE != 0 && en) {
+            t = s_red[0][lane];
 #pragma unroll
-        for (int k = 0; k < MD_NSTAT; k++) s_red[wave][k] = vals[k];
-        s_red[wave][MD_NSTAT - 1] = tb ? 1.0 : 0.0;
-    }
-    __syncthreads();
-    if (tid < MD_NSTAT) {
-        double t = s_red[0][tid];
-#pragma unroll
-        for (int w = 1; w < NW; w++) t += s_red[w][tid];
-        if (COUL == 2 && a.pme_e && ENMODE != 0 && en && leader) {
-            // PME: the replica's long-range terms (the slots hold sums over ordered
-            // pairs, halved by the finalize)
-            if (tid == ACC_COUL) t += 2.0 * a.pme_e[0];
-            if (tid == ACC_VIR) t += 2.0 * a.pme_e[1];
+            for (int w = 1; w < NW; w++) t += s_red[w][lane];
+            if (COUL == 2 && a.pme_e && leader) {
+                // PME: the replica's long-range terms (the slots hold sums over ordered
+                // pairs, halved by the finalize)
+                if (lane == ACC_COUL) t += 2.0 * a.pme_e[0];
+                if (lane == ACC_VIR) t += 2.0 * a.pme_e[1];
+            }
         }
-        a.part[((size_t)a.par * MD_NSTAT + tid) * a.ntiles + tile] = t;
+        if (lane == ACC_KE2) t = ke2;
+        if (lane == MD_NSTAT - 1) t = tb ? 1.0 : 0.0;
+        a.part[((size_t)a.par * MD_NSTAT + lane) * a.ntiles + tile] = t;
     }
 }
 
@@ -1020,8 +1068,8 @@ static void launch_g(const StepArgs& a, int coul, size_t shmem, hipStream_t st, 
     }
 }
 
-// dynamic LDS of the step kernel: the staged set and its dummy
-static size_t step_shmem(const StepArgs& a) { return (size_t)(a.jcap + 1) * sizeof(float4); }
+// dynamic LDS of the step kernel: the staged set and its dummy, the bonded terms
+static size_t step_shmem(const StepArgs& a) { return (size_t)(a.jcap + 1 + (a.bonded ? 8 * 64 : 0)) * sizeof(float4); }
 
 extern "C" hipError_t md_launch_step(const StepArgs& a, int lanes, int coul, hipStream_t st, hipEvent_t ev0,
                                      hipEvent_t ev1) {

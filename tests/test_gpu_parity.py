@@ -442,3 +442,43 @@ def test_download_edges(n, one_cpu):
     e.close()
     assert np.array_equal(p, pos) and np.array_equal(v, vel) and np.isfinite(f).all()
     assert np.array_equal(only[0], pos) and np.array_equal(only[1], vel) and np.array_equal(only[2], f)
+
+
+def stars(n, seed=3):
+    """n molecules of a center with four bonds and four angles (the most an atom can have)."""
+    m = max(6, int(np.ceil(n ** (1 / 3))))
+    rng = np.random.default_rng(seed)
+    s = S.water(nmol=8).copy()
+    L = 6.0 * m
+    g = rng.permutation(m ** 3)[:n]
+    c = (np.stack([g // m // m, g // m % m, g % m], 1) + 0.5) * 6.0 - L / 2
+    arm = np.array([[1, 1, 1], [1, -1, -1], [-1, 1, -1], [-1, -1, 1]]) / np.sqrt(3.0)
+    x = np.concatenate([c[:, None], c[:, None] + arm[None]], 1) + rng.uniform(-0.15, 0.15, (n, 5, 3))
+    s.box = np.full(3, L, np.float32)
+    s.pos = x.reshape(-1, 3).astype(np.float32)
+    s.vel = np.zeros_like(s.pos)
+    s.type = np.tile([0, 1, 1, 1, 1], n).astype(np.int32)
+    s.charge = np.tile([-0.8, 0.2, 0.2, 0.2, 0.2], n).astype(np.float32)
+    b = 5 * np.arange(n)
+    z = np.zeros_like(b)
+    s.bonds = np.concatenate([np.stack([b, b + k, z], 1) for k in range(1, 5)]).astype(np.int32)
+    s.angles = np.concatenate([np.stack([b + k, b, b + k % 4 + 1, z], 1) for k in range(1, 5)]).astype(np.int32)
+    return s
+
+
+@pytest.mark.parametrize("lanes", [4, 8, 16])
+@pytest.mark.parametrize("n", [1, 13, 205])
+def test_bonded_terms_at_their_most(E, orc, n, lanes):
+    """Four bonds and four angles on an atom, in a tile alone, across a tile's end and over
+    several tiles: forces, energies and virial against the oracle at the usual bars."""
+    s = stars(n)
+    say("stars", s.n, "lanes", lanes)
+    e = E.Engine.from_system(s)
+    e.set_launch(lanes=lanes)
+    F, En, W = e.compute_forces()
+    Fo, Eo, Wo = orc.forces(s)
+    say("  force rel rms", rel_rms(F, Fo), "E gpu", En[0], "E orc", Eo, "W", W[0], Wo)
+    assert rel_rms(F, Fo) < FORCE_TOL
+    assert np.all(np.abs(En[0] - Eo) <= 1e-5 * max(np.abs(Eo).sum(), 1.0))
+    assert abs(W[0] - Wo) <= 1e-5 * max(abs(Wo), np.abs(Fo).sum() * 1e-3, 1.0)
+    e.close()
