@@ -462,6 +462,7 @@ __global__ __launch_bounds__(512, 6) void k_nl_tbuild(BuildArgs a) {
             expand(0);
             __syncthreads();
             if (tid < T) fetch();
+            __syncthreads();   // s_cand is read before the next chunk's candidates replace it
             for (int base = 0; base < T; base += NT) {
                 float4 cx = nx;
                 const uint32_t info = nj | ((uint32_t)nty << MD_JBITS);
