@@ -207,6 +207,7 @@ struct md_engine {
     float rc2 = 0, rl2 = 0, skin2q = 0;
     float palfa = 0, spiialfa = 0, alfasq = 0, wolf = 0, reacf = 0, ecut = 0, log2rc = 0;
     int coul_kernel = MD_COUL_NONE;
+    uint32_t ljfree = 0;          // types without Lennard-Jones interactions
 
     int R = 0, N = 0, S = 0, ncell_total = 0;
     std::vector<int> natom, atom_off, slot_off;
@@ -544,6 +545,9 @@ int ensure_stats(md_engine* e, int nrec) {
     return MD_OK;
 }
 
+// types the step kernel's rows may leave the Lennard-Jones term out for (with charges)
+uint32_t ljfree(const md_engine* e) { return e->coul_kernel != MD_COUL_NONE ? e->ljfree : 0; }
+
 // NVE velocity Verlet runs in leapfrog form (one step kernel per step)
 bool vv_fused(const md_engine* e) {
     return e->in.integrator == MD_VVERLET && e->in.thermostat == MD_TH_NONE && e->vv_fuse;
@@ -559,7 +563,7 @@ BuildArgs build_args(md_engine* e) {
     b.pos_build = e->pos_build.p;
     b.key = e->key.p; b.rank = e->rank.p; b.tmp = e->tmp.p; b.tmpid = e->tmpid.p;
     b.cell_count = e->cell_count.p; b.cell_start = e->cell_start.p; b.cell_rank = e->cell_rank.p;
-    b.slot_of = e->slot_of.p; b.nl16 = e->nl16.p; b.ncount = e->ncount.p; b.rperm = e->rperm.p;
+    b.slot_of = e->slot_of.p; b.nl16 = e->nl16.p; b.ncount = e->ncount.p; b.rperm = e->rperm.p; b.ljfree = ljfree(e);
     b.jset = e->jset.p; b.jcount = e->jcount.p;
     b.tilemax = e->tmax.p; b.jmax = e->tmax.p + e->ntiles();
     b.excl = e->excl.p; b.st = e->rst.p; b.gate = e->gate.p;
@@ -574,7 +578,7 @@ StepArgs step_args(md_engine* e, int mode, int energy_every) {
     StepArgs a{};
     a.pos[0] = e->pos[0].p; a.pos[1] = e->pos[1].p; a.vel = e->vel.p; a.force = e->force.p;
     a.ids = e->ids.p; a.typ = e->typ.p; a.nl16 = e->nl16.p; a.ncount = e->ncount.p; a.pos_build = e->pos_build.p;
-    a.rperm = e->rperm.p;
+    a.rperm = e->rperm.p; a.ljfree = ljfree(e);
     a.jset = e->jset.p; a.jcount = e->jcount.p;
     a.tile_rep = e->tile_rep.p; a.rep = e->rep.p; a.st = e->rst.p; a.gate = e->gate.p; a.th = e->th.p; a.part = e->part.p;
     a.lst = e->lst.p; a.lagmode = 0; a.lag = 0; a.par = 0; a.open = 0;
@@ -1062,6 +1066,12 @@ int md_set_forcefield(md_engine* e, const md_forcefield* f) {
     if (e->ff.qfac == 0.0f) e->ff.qfac = 1389.35427611722f;
     derive_ff(e);
     CHECK(upload_ljtab(e, e->ff.lj1, e->ff.lj2));
+    e->ljfree = 0;
+    for (int i = 0; i < e->ff.ntype; i++) {
+        bool none = true;
+        for (int j = 0; j < e->ff.ntype; j++) none &= e->ff.lj1[e->ff.ntype * i + j] == 0.0f && e->ff.lj2[e->ff.ntype * i + j] == 0.0f;
+        if (none) e->ljfree |= 1u << i;
+    }
     if (e->ff.coulomb == MD_COUL_WOLF || e->ff.coulomb == MD_COUL_DAMPED) {
         const std::vector<float4> t = coulomb_table(e->ff.alpha, e->ff.rc, e->ff.coulomb == MD_COUL_WOLF);
         HIPCHECK(hipMemcpy(e->ctab.p, t.data(), (MD_CTAB + 1) * sizeof(float4), hipMemcpyHostToDevice));

@@ -18,7 +18,8 @@
 //               byte offset of the staged entry; sets hold at most MD_JMAX entries), in
 //               the block layout of lpos16(); entries past the row length up to the end
 //               of the row's last block are 0 (the dummy), ncount[S] = row length
-//   rperm[S]    uint8 per tile: the tile's atoms (0..63) by decreasing row length; the
+//   rperm[S]    uint8 per tile: the tile's atoms (0..63) by decreasing row length (types
+//               without Lennard-Jones interactions after the others); the
 //               step kernel gives lane group g the atom rperm[g], so the atoms of a
 //               wavefront have rows of similar length
 // The step kernel stages the tile's set into LDS once per step, each position
@@ -170,7 +171,7 @@ struct StepArgs {
     const int* typ;
     const uint16_t* nl16;     // [S][cap] rows of local indices x 16 (lpos16 layout)
     const int* ncount;
-    const uint8_t* rperm;     // [S] per tile: atoms by decreasing row length
+    const uint8_t* rperm;     // [S] per tile: atoms by decreasing row length, those of ljfree types last
     const uint32_t* jset;     // [ntiles][jcap] tile neighbor sets
     const int* jcount;        // [ntiles]
     const float4* pos_build;
@@ -210,6 +211,7 @@ struct StepArgs {
     int mode;             // MODE_*
     int thermostat;
     int bonded;
+    uint32_t ljfree;      // bit per type: no Lennard-Jones interaction with any type
     int energy_every;     // energies at steps with step % energy_every == 0 (0: never)
     int force_energy;     // MODE_FORCE: compute energies
     int stat_cap;         // records per replica in stats
@@ -426,6 +428,7 @@ struct BuildArgs {
     uint16_t* nl16;
     int* ncount;
     uint8_t* rperm;
+    uint32_t ljfree;      // StepArgs
     uint32_t* jset;
     int* jcount;
     int* tilemax;         // [S/64] longest row per 64-slot tile over the builds since the host cleared it

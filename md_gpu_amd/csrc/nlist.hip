@@ -601,6 +601,7 @@ __global__ __launch_bounds__(512, 6) void k_nl_tbuild(BuildArgs a) {
     // the rows' last entries, padded to the end of the last block (the dummy, local
     // index 0), row lengths, longest row of the wavefront
     int mx = 0;
+    const int my_t = a.ljfree != 0 && tid < 64 ? a.typ_s[slot0 + tid] : 0;
 #pragma unroll
     for (int i = 0; i < AW; i++) {
         const int c = cnt[i];
@@ -616,14 +617,20 @@ __global__ __launch_bounds__(512, 6) void k_nl_tbuild(BuildArgs a) {
     }
     if (lane == 0) s_wmax[wave] = mx;
     __syncthreads();
-    // the tile's atoms by decreasing row length (ties by slot): the step kernel's
-    // wavefronts then hold atoms whose rows end in the same block
+    // the tile's atoms, those with Lennard-Jones interactions first, by decreasing row
+    // length (ties by slot): the step kernel's wavefronts then hold atoms whose rows end in
+    // the same block
     if (tid < 64) {
-        const int c = s_cnt[tid];
+        const int c = s_cnt[tid] + (((a.ljfree >> my_t) & 1) ? 0 : 1 << 24);
+        if (a.ljfree != 0) {   // one wavefront: its LDS accesses stay in order
+            s_cnt[tid] = c;
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        }
+        const int add = a.ljfree != 0 ? 0 : 1 << 24;
         int rank = 0;
 #pragma unroll 4
         for (int k = 0; k < 64; k++) {
-            const int d = s_cnt[k];
+            const int d = s_cnt[k] + add;
             rank += (d > c) || (d == c && k < tid);
         }
         a.rperm[slot0 + rank] = (uint8_t)tid;

@@ -233,13 +233,14 @@ __device__ __forceinline__ void sum_tiles(const double* part, int t0, int t1, in
 // One pair: force factor (F_i += ff * d) and, with EN, the pair energies.
 // Wolf / damped forces come from the cubic table of h(r) in LDS (s_ct); the
 // energies keep the closed form.
-template <int COUL, bool EN>
+// LJ = false: no Lennard-Jones term (the same bits as with zero parameters).
+template <int COUL, bool EN, bool LJ>
 __device__ __forceinline__ float pair_ff(const StepArgs& a, const float4* s_ct, float qi, float qj, float rsq,
                                          const float4 lj, float& ulj, float& ucoul) {
     const float ri = __builtin_amdgcn_rsqf(rsq);
     const float ri2 = ri * ri, ri3 = ri2 * ri;
     const float ri6 = ri3 * ri3, ri8 = ri6 * ri2;
-    const float flj = fmaf(lj.x, ri6, -lj.y) * ri8;   // lj1 r^-14 - lj2 r^-8, src/pair_forces.cu:190-193
+    const float flj = LJ ? fmaf(lj.x, ri6, -lj.y) * ri8 : 0.0f;   // lj1 r^-14 - lj2 r^-8, src/pair_forces.cu:190-193
     float ff = flj;
     if (COUL == 0) {           // reaction field, src/pair_forces.cu:88-91
         const float qq = qi * qj;
@@ -270,7 +271,10 @@ __device__ __forceinline__ float pair_ff(const StepArgs& a, const float4* s_ct, 
 // NT2: at most two atom types, so the LJ parameters of a pair are one of the
 // two entries of the atom's table row, held in registers and picked by a select
 // (no LDS read per pair); otherwise the row is read from LDS per pair.
-template <int G, int COUL, int ENMODE, bool NT2>
+// LJF: types without any Lennard-Jones interaction exist (a.ljfree): a walk without the
+// term besides the other (its code costs launches of short kernels instruction fetches:
+// 30 steps of 32,768 ions with smooth PME 3.05 ms with it in every variant, else 3.02).
+template <int G, int COUL, int ENMODE, bool NT2, bool LJF>
 __global__ __launch_bounds__(64 * G, COUL == 3 ? 5 : 4) void k_step(const StepArgs a) {
     constexpr int NW = G;                 // wavefronts: 64 atoms x G lanes
     extern __shared__ float4 s_j[];       // [jcap + 1] the tile's staged neighbor set
@@ -469,14 +473,24 @@ __global__ __launch_bounds__(64 * G, COUL == 3 ? 5 : 4) void k_step(const StepAr
     const float4 lj_d = make_float4(lj_b.x - lj_a.x, lj_b.y - lj_a.y, lj_b.z - lj_a.z, 0.0f);
     float fx = 0.f, fy = 0.f, fz = 0.f;
     double elj = 0.0, eco = 0.0, evi = 0.0;
-    auto pair = [&](const float4& pj, auto en_tag) {
-        constexpr bool EN = decltype(en_tag)::value;
+    auto pair = [&](const float4& pj, auto en_tag, auto lj_tag) {
+        constexpr bool EN = decltype(en_tag)::value, LJ = decltype(lj_tag)::value;
         float4 lj;
-        if (NT2 && !CHG) {   // w = type (0 or 1) as a float: the row entry by interpolation
+        if (!LJ) {
+            lj = make_float4(0.f, 0.f, 0.f, 0.f);
+        } else if (NT2 && !CHG) {   // w = type (0 or 1) as a float: the row entry by interpolation
             lj = make_float4(fmaf(pj.w, lj_d.x, lj_a.x), fmaf(pj.w, lj_d.y, lj_a.y), fmaf(pj.w, lj_d.z, lj_a.z), 0.0f);
         } else if (NT2) {
-            const bool tb = (__float_as_uint(pj.w) & 1u) != 0;   // type 1 (types are 0 or 1)
-            lj = make_float4(tb ? lj_b.x : lj_a.x, tb ? lj_b.y : lj_a.y, tb ? lj_b.z : lj_a.z, 0.0f);
+            // type 1 (types are 0 or 1): its bit as a mask, one bit-field insert per parameter
+            // (written out: the compiler makes a compare and two selects of it)
+            int m;
+            asm("v_bfe_i32 %0, %1, 0, 1" : "=v"(m) : "v"(pj.w));
+            auto pick = [&](float x, float y) {
+                float z;
+                asm("v_bfi_b32 %0, %1, %2, %3" : "=v"(z) : "v"(m), "v"(y), "v"(x));
+                return z;
+            };
+            lj = make_float4(pick(lj_a.x, lj_b.x), pick(lj_a.y, lj_b.y), pick(lj_a.z, lj_b.z), 0.0f);
         } else {
             lj = s_lji[CHG ? staged_type(pj) : (int)pj.w];
         }
@@ -485,7 +499,7 @@ __global__ __launch_bounds__(64 * G, COUL == 3 ? 5 : 4) void k_step(const StepAr
         float ulj = 0.0f, ucoul = 0.0f;
         float ff;
         if (COUL == 3 && !EN) ff = pair_ff_lj(rsq, lj);
-        else ff = pair_ff<COUL, EN>(a, s_ct, qi, pj.w, rsq, lj, ulj, ucoul);
+        else ff = pair_ff<COUL, EN, LJ>(a, s_ct, qi, pj.w, rsq, lj, ulj, ucoul);
         const bool use = !(rsq > a.rc2);   // cutoff as src/pair_forces.cu:195 (zero for rsq > rc2)
         ff = use ? ff : 0.0f;
         fx = fmaf(ff, dx, fx);
@@ -565,11 +579,24 @@ __global__ __launch_bounds__(64 * G, COUL == 3 ? 5 : 4) void k_step(const StepAr
             }
         }
     }
-    // lane groups hold the tile's atoms by decreasing row length (rperm)
+    // Lane groups hold the tile's atoms by decreasing row length (rperm), those of types
+    // without any Lennard-Jones interaction (a.ljfree; water's hydrogens) after the others, so
+    // whole wavefronts leave the term out: 27 VALU instructions per pair instead of 35 (40
+    // steps of 196,608 water atoms 7.51 -> 7.23 ms, the same bits).
+    int nn0 = __builtin_amdgcn_readfirstlane(nn);   // the wavefront's longest row
+    bool ljw = true;                                // any atom of it has the term
+    if (LJF) {
+        const bool fr = ((a.ljfree >> tyi) & 1) != 0;
+        const unsigned long long fm = __ballot(fr);
+        if (fm) nn0 = max(nn0, __builtin_amdgcn_readlane(nn, __builtin_ctzll(fm)));
+        ljw = __ballot(active && !fr) != 0;
+    }
     if (ENMODE != 0 && en)
-        walk_row_sorted<G>(s_j, row4, nn, sub, q0, q1, [&](const float4& pj) { pair(pj, std::true_type{}); });
+        walk_row_sorted<G>(s_j, row4, nn, nn0, sub, q0, q1, [&](const float4& pj) { pair(pj, std::true_type{}, std::true_type{}); });
+    else if (!LJF || ljw)
+        walk_row_sorted<G>(s_j, row4, nn, nn0, sub, q0, q1, [&](const float4& pj) { pair(pj, std::false_type{}, std::true_type{}); });
     else
-        walk_row_sorted<G>(s_j, row4, nn, sub, q0, q1, [&](const float4& pj) { pair(pj, std::false_type{}); });
+        walk_row_sorted<G>(s_j, row4, nn, nn0, sub, q0, q1, [&](const float4& pj) { pair(pj, std::false_type{}, std::false_type{}); });
 
     if (a.bonded) {   // the atom's lanes take its bonded terms
         __syncthreads();
@@ -1044,15 +1071,21 @@ static void launch_k(K kern, const StepArgs& a, int grid, int threads, size_t sh
     else hipLaunchKernelGGL(kern, dim3(grid), dim3(threads), shmem, st, a);
 }
 
-template <int G, int EM, bool NT2>
+template <int G, int EM, bool NT2, bool LJF>
 static void launch_ge(const StepArgs& a, int coul, size_t shmem, hipStream_t st, hipEvent_t ev0, hipEvent_t ev1) {
     const int grid = a.ntiles;
     switch (coul) {
-    case 0: launch_k(k_step<G, 0, EM, NT2>, a, grid, 64 * G, shmem, st, ev0, ev1); break;
-    case 1: launch_k(k_step<G, 1, EM, NT2>, a, grid, 64 * G, shmem, st, ev0, ev1); break;
-    case 2: launch_k(k_step<G, 2, EM, NT2>, a, grid, 64 * G, shmem, st, ev0, ev1); break;
-    default: launch_k(k_step<G, 3, EM, NT2>, a, grid, 64 * G, shmem, st, ev0, ev1); break;
+    case 0: launch_k(k_step<G, 0, EM, NT2, LJF>, a, grid, 64 * G, shmem, st, ev0, ev1); break;
+    case 1: launch_k(k_step<G, 1, EM, NT2, LJF>, a, grid, 64 * G, shmem, st, ev0, ev1); break;
+    case 2: launch_k(k_step<G, 2, EM, NT2, LJF>, a, grid, 64 * G, shmem, st, ev0, ev1); break;
+    default: launch_k(k_step<G, 3, EM, NT2, false>, a, grid, 64 * G, shmem, st, ev0, ev1); break;
     }
+}
+
+template <int G, int EM, bool NT2>
+static void launch_gf(const StepArgs& a, int coul, size_t shmem, hipStream_t st, hipEvent_t ev0, hipEvent_t ev1) {
+    if (a.ljfree != 0) launch_ge<G, EM, NT2, true>(a, coul, shmem, st, ev0, ev1);
+    else launch_ge<G, EM, NT2, false>(a, coul, shmem, st, ev0, ev1);
 }
 
 template <int G>
@@ -1060,11 +1093,11 @@ static void launch_g(const StepArgs& a, int coul, size_t shmem, hipStream_t st, 
     const bool em = (a.mode == MODE_FORCE) ? a.force_energy != 0 : a.energy_every > 0;
     const bool nt2 = a.ntype <= 2;
     if (em) {
-        if (nt2) launch_ge<G, 1, true>(a, coul, shmem, st, ev0, ev1);
-        else launch_ge<G, 1, false>(a, coul, shmem, st, ev0, ev1);
+        if (nt2) launch_gf<G, 1, true>(a, coul, shmem, st, ev0, ev1);
+        else launch_gf<G, 1, false>(a, coul, shmem, st, ev0, ev1);
     } else {
-        if (nt2) launch_ge<G, 0, true>(a, coul, shmem, st, ev0, ev1);
-        else launch_ge<G, 0, false>(a, coul, shmem, st, ev0, ev1);
+        if (nt2) launch_gf<G, 0, true>(a, coul, shmem, st, ev0, ev1);
+        else launch_gf<G, 0, false>(a, coul, shmem, st, ev0, ev1);
     }
 }
 

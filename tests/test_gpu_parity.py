@@ -482,3 +482,38 @@ def test_bonded_terms_at_their_most(E, orc, n, lanes):
     assert np.all(np.abs(En[0] - Eo) <= 1e-5 * max(np.abs(Eo).sum(), 1.0))
     assert abs(W[0] - Wo) <= 1e-5 * max(abs(Wo), np.abs(Fo).sum() * 1e-3, 1.0)
     e.close()
+
+
+@pytest.mark.parametrize("lanes", [4, 8, 16])
+@pytest.mark.parametrize("coulomb", [S.COUL_RF, S.COUL_WOLF, S.COUL_DAMPED, None])
+@pytest.mark.parametrize("ntype", [2, 3])
+def test_types_without_lennard_jones(E, lanes, coulomb, ntype):
+    """Atoms of types without Lennard-Jones interactions (their wavefronts leave the term out)
+    get the bits of the general path, which the same parameters take when the force field
+    has one more type, of no atom, that all types interact with: forces, energies and a short
+    run, with two types and more, every Coulomb kind and none (no charges)."""
+    say("no LJ types", lanes, coulomb, ntype)
+    s = perturbed(S.water(nmol=700), 0.05)
+    out = []
+    for nt in (ntype, ntype + 1):
+        eps, sig = np.zeros((nt, nt)), np.ones((nt, nt))
+        eps[0, 0], sig[0, 0] = 0.65, 3.166
+        if nt > ntype:
+            eps[ntype, :] = eps[:, ntype] = 1.0
+        ff = dataclasses.replace(s.ff, names=["O", "H", "D", "X"][:nt], masses=np.array([16.0, 1.008, 2.014, 1.0][:nt]),
+                                 lj1=48.0 * eps * sig ** 12, lj2=24.0 * eps * sig ** 6,
+                                 coulomb=S.COUL_WOLF if coulomb is None else coulomb)
+        t = dataclasses.replace(s.copy(), ff=ff)
+        if ntype == 3:
+            t.type = t.type.copy()
+            t.type[2::3] = 2
+        if coulomb is None:
+            t.charge = np.zeros_like(t.charge)
+        e = E.Engine.from_system(t)
+        e.set_launch(lanes=lanes)
+        r = list(e.compute_forces())
+        e.run(12, stats=False)
+        out.append(r + list(e.download()))
+        e.close()
+    for a, b in zip(*out):
+        assert np.isfinite(a).all() and np.array_equal(a, b)
