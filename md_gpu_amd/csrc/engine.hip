@@ -276,8 +276,7 @@ struct md_engine {
     int pk_req = 0;                // list capacity the caller set (entries per atom): bounds the lane rows
     long long pk_runs = 0, pk_replays = 0;   // runs on the persistent kernel, replays after a row overflow
     size_t lds_max = 65536;        // LDS per workgroup on this device
-    DBuf<unsigned> pk_flags;       // [2][MD_PK_WG] barrier flags
-    DBuf<double> pk_pub;           // [2][MD_PK_WG][4] partial sums published at the barriers
+    DBuf<uint64_t> pk_xch;         // published positions and sums (persistent kernel)
     static constexpr double kQueueRatio0 = 1.15;
     double queue_ratio = kQueueRatio0;   // launched / completed steps, learned per launch configuration
     int fm_nframes = 0;
@@ -887,7 +886,8 @@ int run_begin(md_engine* e, long long nsteps) {
     a.st = e->rst.p; a.snap_st = e->snap_rst.p; a.th = e->th.p; a.snap_th = e->snap_th.p;
     a.gate = e->gate.p; a.snap_gate = e->snap_gate.p; a.rep = e->rep.p; a.err = e->err.p;
     a.tmax = e->tmax.p; a.ntmax = nsteps < 0 ? 0 : 2LL * e->ntiles();
-    a.pk_flags = nsteps < 0 ? e->pk_flags.p : nullptr;
+    a.pk_xch = nsteps < 0 ? e->pk_xch.p : nullptr;
+    a.npk = nsteps < 0 ? MD_PK_PUB + 4 * e->N : 0;
     a.nsteps = nsteps; a.nrep = e->R; a.dt = e->in.dt; a.thermostat = e->in.thermostat;
     a.th_begin = nsteps >= 0 && e->in.integrator == MD_VVERLET;
     HIPCHECK(md_launch_run_begin(a, s.n, s.live, s.copy, s.nb, e->st));
@@ -1534,11 +1534,19 @@ bool persist_eligible(const md_engine* e) {
 }
 bool persist_ok(const md_engine* e) { return e->persist && persist_eligible(e); }
 
+// Threads per workgroup: half of MD_PK_THREADS while the workgroups still fit one XCD
+// (a CU each), which shares the work of a step among twice the CUs.
+int persist_xcd(const md_engine* e) { return std::min(e->ncu / 8, MD_PK_WG); }
+int persist_wgs(const md_engine* e, int nth) { return (e->N + nth / e->lanes - 1) / (nth / e->lanes); }
+int persist_threads(const md_engine* e) {
+    return persist_wgs(e, MD_PK_THREADS / 2) <= persist_xcd(e) ? MD_PK_THREADS / 2 : MD_PK_THREADS;
+}
+
 // Dynamic LDS of a launch: staged positions and types (20 B per slot) and the
 // lane rows (2 B per entry and thread); at least half the CU's 160 KB, so that
 // no two of the workgroups share a CU.
 size_t persist_lds(const md_engine* e, int cap_l) {
-    const size_t need = (size_t)e->S * 20 + (size_t)cap_l * MD_PK_THREADS * 2;
+    const size_t need = (size_t)e->S * 20 + (size_t)cap_l * persist_threads(e) * 2;
     return std::max(need, (size_t)81920);
 }
 
@@ -1560,14 +1568,12 @@ int persist_cap(const md_engine* e) {
 // rows do not fit the kernel's LDS: the caller runs the tile path instead.
 int run_persist(md_engine* e, int nsteps, int energy_every, bool want_stats, int* use_tiles) {
     *use_tiles = 0;
-    const int G = e->lanes, apw = MD_PK_THREADS / G;
-    const int nwg = (e->S + apw - 1) / apw;
-    if (nwg > MD_PK_WG) {   // (S <= MD_PK_SLOTS and apw >= 64 keep nwg <= 64)
+    const int G = e->lanes, nth = persist_threads(e), nwg = persist_wgs(e, nth);
+    if (nwg > MD_PK_WG) {   // (S <= MD_PK_SLOTS and 64 atoms or more per workgroup keep nwg <= 64)
         *use_tiles = 1;
         return MD_OK;
     }
-    if (!e->pk_flags.p) CHECK(e->pk_flags.alloc(2 * MD_PK_WG));
-    if (!e->pk_pub.p) CHECK(e->pk_pub.alloc(2 * MD_PK_WG * 4));
+    if (!e->pk_xch.p) CHECK(e->pk_xch.alloc(MD_PK_PUB + 4 * MD_PK_SLOTS));
     const size_t static_lds = 2048;   // the kernel's own tables and sums (1.4 KB)
     for (;;) {
         const int cap_l = persist_cap(e);
@@ -1581,9 +1587,12 @@ int run_persist(md_engine* e, int nsteps, int energy_every, bool want_stats, int
         a.pos[0] = e->pos[0].p; a.pos[1] = e->pos[1].p; a.vel = e->vel.p; a.force = e->force.p;
         a.ids = e->ids.p; a.typ = e->typ.p; a.ljtab = e->ljtab.p;
         a.st = e->rst.p; a.th = e->th.p; a.rep = e->rep.p;
-        a.flags = e->pk_flags.p; a.pub = e->pk_pub.p; a.err = e->err.p;
+        a.pub = e->pk_xch.p; a.hint = e->pk_xch.p + 2 * MD_PK_WG * 6; a.xch = e->pk_xch.p + MD_PK_PUB; a.err = e->err.p;
         a.stats = want_stats ? e->stats.p : nullptr; a.stat_cap = e->stat_cap;
-        a.nslot = e->S; a.nwg = nwg; a.nsteps = nsteps; a.energy_every = energy_every;
+        a.nslot = e->S; a.natom = e->N; a.nth = nth; a.nwg = nwg;
+        // on one XCD where they fit: workgroups are dealt to the XCDs in turn
+        a.spread = nwg <= persist_xcd(e) ? 8 : 1;
+        a.nsteps = nsteps; a.energy_every = energy_every;
         a.leapfrog = e->in.integrator == MD_LEAPFROG ? 1 : 0;
         a.thermostat = e->in.thermostat; a.ntype = e->ff.ntype; a.cap_l = cap_l;
         a.dt = e->in.dt; a.tau = e->in.tau; a.rc2 = e->rc2; a.rl2 = e->rl2; a.skin2q = e->skin2q;
@@ -1598,7 +1607,7 @@ int run_persist(md_engine* e, int nsteps, int energy_every, bool want_stats, int
         HIPCHECK(md_launch_force_trip(e->rst.p, e->gate.p, e->R, 1, nullptr, 0, e->err.p, &e->report->err, e->st));
         HIPCHECK(hipStreamSynchronize(e->st));
         const int err = e->report->err;
-        if (err & MD_PK_ERR_WAIT) return fail(MD_E_HIP, "persistent kernel: a grid barrier wait timed out");
+        if (err & MD_PK_ERR_WAIT) return fail(MD_E_HIP, "persistent kernel: a wait for another workgroup timed out");
         if (err & MD_PK_ERR_ROWS) {   // a row outgrew its length: replay the run with longer rows
             CHECK(run_rollback(e));
             HIPCHECK(hipStreamSynchronize(e->st));

@@ -318,7 +318,8 @@ struct RunBeginArgs {
     int* tmax;
     long long ntmax;        // list maxima to clear
     int* err;
-    unsigned* pk_flags;     // persistent kernel: barrier flags, else nullptr
+    uint64_t* pk_xch;       // persistent kernel: npk words of the exchange buffer to clear
+    int npk;
     long long nsteps;       // < 0: targets and gates stay (the persistent kernel keeps its own count)
     int nrep, th_begin, thermostat;
     float dt;
@@ -370,11 +371,12 @@ struct SettleArgs {
 // Persistent kernel for small single systems (persist.hip): all steps of a run
 // in one launch of at most MD_PK_WG workgroups of MD_PK_THREADS threads.
 #define MD_PK_SLOTS 4096          // largest system (slots): the staged positions fill at most 64 KB of LDS
-#define MD_PK_WG 64               // most workgroups (one wavefront polls every barrier flag)
+#define MD_PK_WG 64               // most workgroups (a lane of one wavefront reads each one's sums)
+#define MD_PK_PUB (2 * MD_PK_WG * 7)   // words of the exchange buffer for sums and hints (positions follow)
 #define MD_PK_THREADS 1024
-#define MD_PK_TIMEOUT 50000000ull // barrier wait limit, 100 MHz wall-clock ticks (0.5 s)
+#define MD_PK_TIMEOUT 50000000ull // wait limit, 100 MHz wall-clock ticks (0.5 s)
 #define MD_PK_ERR_ROWS 4          // err bit: a lane's row outgrew cap_l (the run is replayed with longer rows)
-#define MD_PK_ERR_WAIT 8          // err bit: a barrier wait timed out
+#define MD_PK_ERR_WAIT 8          // err bit: a wait timed out
 
 struct PersistArgs {
     float4* pos[2];
@@ -386,13 +388,17 @@ struct PersistArgs {
     RepState* st;         // replica 0
     ThState* th;
     const RepParam* rep;
-    unsigned* flags;      // [2][MD_PK_WG] barrier flags, zero at launch
-    double* pub;          // [2][MD_PK_WG][4] partial sums published at the barriers (2 KE, LJ, virial)
+    uint64_t* xch;        // [2][natom][2] published positions, zero at launch
+    uint64_t* hint;       // [2][MD_PK_WG] step numbers a workgroup has published, zero at launch
+    uint64_t* pub;        // [2][MD_PK_WG][6] published partial sums (2 KE, LJ, virial), zero at launch
     int* err;             // 1: an atom left the box; MD_PK_ERR_*
     StatRec* stats;       // [stat_cap] or null
     int stat_cap;
     int nslot;
-    int nwg;              // ceil(nslot / (MD_PK_THREADS / lanes))
+    int natom;            // atoms in slots 0 .. natom - 1
+    int nth;              // threads per workgroup: MD_PK_THREADS or half of them
+    int nwg;              // ceil(natom / (nth / lanes))
+    int spread;           // workgroups launched per working one
     long long nsteps;
     int energy_every;
     int leapfrog;         // 1: leapfrog (thermostat none or Berendsen); 0: NVE velocity Verlet

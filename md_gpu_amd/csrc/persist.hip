@@ -3,35 +3,47 @@
 // For one replica of at most MD_PK_SLOTS slots (Lennard-Jones only, no bonded
 // terms) a step is microseconds of pair work spread over a handful of tiles,
 // and a launch per step (plus its finalize) costs more than the step.  Here a
-// few workgroups of 1024 threads, one per CU and all resident at once, run
-// every step of a run and meet at a grid barrier once per step:
-//   - workgroup w owns the 1024/G slots from w 1024/G (G lanes per atom) and
+// few workgroups of 512 or 1024 threads, one per CU and all resident at once,
+// run every step of a run and exchange positions once per step:
+//   - workgroup w owns the NTH/G slots from w NTH/G (G lanes per atom) and
 //     keeps their position, velocity, force and build position in registers;
-//   - after each barrier it stages the positions of the whole system into LDS
-//     (at most 64 KB) and walks its atoms' rows there, minimum image per pair
+//   - each step it stages the positions of the whole system into LDS (at most
+//     64 KB) and walks its atoms' rows there, minimum image per pair
 //     (src/neighborlist.cu:271-273), LJ force as src/pair_forces.cu:190-195;
 //   - the rows are private to the lanes: lane l of an atom lists the
 //     neighbors j = l (mod G) within r_list, 16-bit slot indices in LDS.  They
 //     are built by a scan of the staged system at the run's first step and
-//     whenever the previous step's skin check tripped anywhere (each workgroup
-//     reads every workgroup's flag at the barrier, so all rebuild together);
-//     the build wraps the atoms into the box, as the tile path's build does;
-//   - at the barrier each workgroup also publishes its FP64 partial sums (2 KE,
-//     LJ energy, virial), so the Berendsen factor (src/integrator.cu:146-147,
-//     from the previous step's temperature) and the statistics record of each
-//     step come from the same sums, added in the same order, everywhere.
+//     whenever the previous step's skin check tripped anywhere (the flag rides on
+//     the atom's published position, so all rebuild together); the build wraps the
+//     atoms into the box, as the tile path's build does;
+//   - where the Berendsen factor (src/integrator.cu:146-147, from the previous
+//     step's temperature) or the statistics records need them, each workgroup also
+//     publishes its FP64 partial sums (2 KE, LJ energy, virial), added in the same
+//     order everywhere.
 // Integrators: leapfrog (src/nve_leapfrog.cu:37-55, src/nvt_leapfrog_ber.cu:35-55)
 // and NVE velocity Verlet in the leapfrog form of the step kernel (each step
 // ends with the second half kick and begins the next with the first).
 //
-// The barrier: plain stores of the published data, then an agent-scope release
-// fence and a relaxed store of the workgroup's flag; one wavefront polls every
-// workgroup's flag with relaxed loads, then an agent-scope acquire fence.  Flags
-// alternate between two banks by barrier parity: a workgroup one barrier ahead
-// never overwrites a flag another is still reading.  Every wait is bounded
-// (MD_PK_TIMEOUT ticks of the 100 MHz wall clock): a workgroup that times out
-// sets MD_PK_ERR_WAIT and leaves, the others leave at their next wait, and the
-// host reports the error.
+// The exchange: every published 64-bit word carries the number of its step beside
+// 32 bits of data (48 of a position), stored and loaded whole at agent scope, so a
+// reader that sees the number has the data and no fence, cache write-back or
+// invalidation orders anything.  One wavefront waits for the workgroups' hints (a word
+// each, stored once its positions are on the way), then every thread loads its
+// slots and repeats those whose number is still the old one.  Two banks by step
+// parity: a workgroup writes step n + 2 only after it has read every atom of step
+// n + 1, and their owners had read step n before they wrote those.  Every wait is
+// bounded (MD_PK_TIMEOUT ticks of the 100 MHz wall clock): a workgroup that times
+// out sets MD_PK_ERR_WAIT and leaves, the others leave at their next wait, and
+// the host reports the error.
+//
+// Bound by that latency (about 1.8 of 3.3 us a step at 864 atoms) and the walk's VALU
+// work on few CUs.  While they fit, the workgroups are placed on one XCD (the others are
+// launched for every one that works and leave: workgroups are dealt to the XCDs in turn)
+// and have 512 threads, twice as many CUs.  100 steps with a download, 864 atoms: 497
+// us with a grid barrier of release and acquire fences per step, 447 with agent-scope
+// words instead on one XCD, 428 with 512 threads, 377 without the barrier; 256 atoms, 10
+// steps: 81, 76, 71, 71.  (Every thread polling its slots instead of a hint: 376 there, but
+// 863 instead of 503 at 2,048 atoms; 256 threads: 484 instead of 444 with 8 lanes.)
 #include <hip/hip_ext.h>
 
 #include <type_traits>
@@ -41,61 +53,37 @@
 
 namespace {
 
-constexpr int NTH = MD_PK_THREADS;
-constexpr unsigned FL_TRIP = 1u, FL_ROWS = 2u, FL_STOP = 4u;   // flag bits below the barrier count
+constexpr unsigned FL_TRIP = 1u, FL_ROWS = 2u, FL_STOP = 4u;   // flag bits below the step number
 
-// Grid barrier number b with the workgroup's flag bits; returns the OR of every
-// workgroup's bits (FL_STOP also when this workgroup's wait timed out).  Called
-// by every thread of the workgroup.
-__device__ unsigned pk_barrier(const PersistArgs& a, int b, unsigned bits, unsigned* s_bits) {
-    const int tid = threadIdx.x, lane = tid & 63;
-    unsigned* fl = a.flags + (b & 1) * MD_PK_WG;
-    __syncthreads();   // the workgroup's published stores precede thread 0's release fence
-    if (tid == 0) {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-        __hip_atomic_store(fl + blockIdx.x, ((unsigned)(b + 1) << 3) | bits, __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_AGENT);
-    }
-    if (tid < 64) {
-        const unsigned want = (unsigned)(b + 1);
-        const unsigned long long t0 = wall_clock64();
-        unsigned mine = 0;
-        bool late = false;
-        for (;;) {
-            bool ok = true;
-            if (lane < a.nwg) {
-                const unsigned v = __hip_atomic_load(fl + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                ok = (v >> 3) >= want;
-                mine = v & 7u;
-            }
-            if (__all(ok)) break;
-            if (wall_clock64() - t0 > MD_PK_TIMEOUT) {
-                late = true;
-                break;
-            }
-            __builtin_amdgcn_s_sleep(1);
-        }
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-        unsigned all = 0;
-        if (__ballot((mine & FL_TRIP) != 0)) all |= FL_TRIP;
-        if (__ballot((mine & FL_ROWS) != 0)) all |= FL_ROWS;
-        if (__ballot((mine & FL_STOP) != 0)) all |= FL_STOP;
-        if (late) {
-            all |= FL_STOP;
-            if (lane == 0) atomicOr(a.err, MD_PK_ERR_WAIT);
-        }
-        if (lane == 0) *s_bits = all;
-    }
-    __syncthreads();
-    return *s_bits;
+// A published word: 32 bits of data and above them the step number << 3 (sums), or 48 bits
+// of data and above them the step number's low 13 bits and the atom's flag bits (positions).
+__device__ __forceinline__ void put(uint64_t* p, uint32_t v, unsigned tag) {
+    __hip_atomic_store(p, (uint64_t)v | ((uint64_t)tag << 32), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+__device__ __forceinline__ uint64_t get(const uint64_t* p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ bool of_step(uint64_t w, unsigned n) { return (unsigned)(w >> 51) == (n & 0x1fffu); }   // position
+__device__ __forceinline__ bool is_step(uint64_t w, unsigned n) { return (unsigned)(w >> 35) == n; }
+
+// The limit of a wait: looked at every 64 tries.
+struct Wait {
+    unsigned long long t0 = 0;
+    unsigned tries = 0;
+    __device__ __forceinline__ bool late() {
+        if ((++tries & 63u) != 0) return false;
+        const unsigned long long t = wall_clock64();
+        if (tries == 64u) t0 = t;
+        return t - t0 > MD_PK_TIMEOUT;
+    }
+};
 
 }  // namespace
 
-// G lanes per atom (1024 / G atoms per workgroup); NT1: one atom type (the LJ
+// G lanes per atom (NTH / G atoms per workgroup); NT1: one atom type (the LJ
 // parameters sit in registers).
-template <int G, bool NT1>
-__global__ __launch_bounds__(MD_PK_THREADS) void k_persist(const PersistArgs a) {
+template <int G, bool NT1, int NTH>
+__global__ __launch_bounds__(NTH) void k_persist(const PersistArgs a) {
     constexpr int APW = NTH / G, NW = NTH / 64;
     extern __shared__ float4 s_dyn[];
     float4* s_pos = s_dyn;                                                 // [nslot] x, y, z, type (-1: padding)
@@ -105,10 +93,11 @@ __global__ __launch_bounds__(MD_PK_THREADS) void k_persist(const PersistArgs a) 
     __shared__ float4 s_lj[64];
     __shared__ double s_red[NW][3];
     __shared__ double s_lam;         // Berendsen factor of the current step
-    __shared__ unsigned s_bits;      // flag bits of all workgroups at the last barrier
-    __shared__ unsigned s_wgb;       // this workgroup's flag bits of the current step
+    __shared__ unsigned s_bits[2];   // flag bits of all atoms' last steps, by step parity
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, sub = tid & (G - 1);
-    const int slot = blockIdx.x * APW + tid / G;
+    if (blockIdx.x % a.spread) return;   // launched only for the placement
+    const int bid = blockIdx.x / a.spread;
+    const int slot = bid * APW + tid / G;
     const bool inr = slot < a.nslot;
     const int id = inr ? a.ids[slot] : -1;
     const bool active = id >= 0;
@@ -131,8 +120,42 @@ __global__ __launch_bounds__(MD_PK_THREADS) void k_persist(const PersistArgs a) 
     double lamd = a.leapfrog ? a.th[0].S : 1.0;   // leapfrog: the factor of the run's first step
     const bool need_lam = a.leapfrog && a.thermostat == 1;
     const bool need_ke = need_lam || a.stats != nullptr;   // the published sums have a reader
-    int b = 0;                                      // barriers passed
-    unsigned bits = 0;
+    // the atom's position, published as step number n (into bank n & 1)
+    auto publish = [&](unsigned n, float4 y, unsigned fl) {
+        uint64_t* q = a.xch + ((size_t)(n & 1) * a.natom + slot) * 2;
+        const unsigned tag = ((n << 3) | fl) << 16, iy = __float_as_uint(y.y);
+        put(q, __float_as_uint(y.x), tag | (iy >> 16));
+        put(q + 1, __float_as_uint(y.z), tag | (iy & 0xffffu));
+    };
+    // every workgroup's sums of step number n (lane w: workgroup w's); false: the wait timed out
+    auto sums_of = [&](unsigned n, double& t0, double& t1, double& t2) {
+        bool ok = true;
+        if (lane < a.nwg) {
+            const uint64_t* q = a.pub + ((size_t)(n & 1) * MD_PK_WG + lane) * 6;
+            uint64_t w[6];
+            Wait wait;
+            for (;;) {
+                bool all = true;
+#pragma unroll
+                for (int c = 0; c < 6; c++) w[c] = get(q + c);
+#pragma unroll
+                for (int c = 0; c < 6; c++) all = all && is_step(w[c], n);
+                if (all) break;
+                if (wait.late()) {
+                    ok = false;
+                    break;
+                }
+            }
+            auto dbl = [](uint64_t hi, uint64_t lo) { return __longlong_as_double((long long)((hi << 32) | (lo & 0xffffffffull))); };
+            t0 = dbl(w[1], w[0]);
+            t1 = dbl(w[3], w[2]);
+            t2 = dbl(w[5], w[4]);
+        }
+        if (__all(ok)) return true;
+        if (lane == 0) atomicOr(a.err, MD_PK_ERR_WAIT);
+        return false;
+    };
+    if (tid < 2) s_bits[tid] = 0u;
     if (!a.leapfrog) {
         // velocity Verlet: the first half kick and drift of the run's first step
         // (k_vv_kick's arithmetic with S = 1)
@@ -142,9 +165,10 @@ __global__ __launch_bounds__(MD_PK_THREADS) void k_persist(const PersistArgs a) 
             v.y = fmaf(f.y, h, v.y);
             v.z = fmaf(f.z, h, v.z);
             x = make_float4(fmaf(v.x, a.dt, x.x), fmaf(v.y, a.dt, x.y), fmaf(v.z, a.dt, x.z), x.w);
-            if (sub == 0) a.pos[cb0 ^ 1][slot] = x;
+            if (sub == 0) publish(1u, x, 0u);
         }
-        bits = pk_barrier(a, b++, 0u, &s_bits);
+        __syncthreads();
+        if (tid == 0) put(a.hint + MD_PK_WG + bid, 1u, 0u);
     }
     float4 xb = x;                  // build position (skin check)
     int cnt = 0;                    // this lane's row length
@@ -154,28 +178,74 @@ __global__ __launch_bounds__(MD_PK_THREADS) void k_persist(const PersistArgs a) 
     if (NT1) lj1 = s_lj[0];
     const int nsteps = (int)a.nsteps;
     int done = 0;
-    for (int k = 0; k < nsteps && !(bits & FL_STOP); k++) {
-        // positions of the step whose forces this iteration computes
-        const long long sx = a.leapfrog ? step0 + k : step0 + k + 1;
-        const float4* __restrict__ pin = a.pos[(int)(sx & 1)];
-        if (tid == 0) s_wgb = 0;   // every thread read the last value before the previous barrier
-        for (int q = tid; q < a.nslot; q += NTH) {
-            const float4 y = pin[q];
-            s_pos[q] = make_float4(y.x, y.y, y.z, s_tyf[q]);
+    for (int k = 0; k < nsteps; k++) {
+        // the positions of the step whose forces this iteration computes, step number k + 1:
+        // each thread waits for its slots (leapfrog's first ones are the run's start)
+        unsigned fl = 0;
+        if (k > 0 || !a.leapfrog) {
+            constexpr int SPT = MD_PK_SLOTS / NTH;
+            const unsigned n = (unsigned)(k + 1);
+            const uint64_t* bank = a.xch + (size_t)(n & 1) * a.natom * 2;
+            if (wave == 0) {   // the hints: nothing relies on them but the time of the first try
+                bool ok = true;
+                if (lane < a.nwg) {
+                    const uint64_t* q = a.hint + (n & 1) * MD_PK_WG + lane;
+                    Wait wait;
+                    while ((unsigned)get(q) != n) {
+                        if (wait.late()) {
+                            ok = false;
+                            break;
+                        }
+                        __builtin_amdgcn_s_sleep(1);
+                    }
+                }
+                if (!ok) {
+                    atomicOr(a.err, MD_PK_ERR_WAIT);
+                    fl |= FL_STOP;
+                }
+            }
+            __syncthreads();
+            unsigned miss = 0;
+#pragma unroll
+            for (int u = 0; u < SPT; u++)
+                if (tid + u * NTH < a.natom) miss |= 1u << u;
+            Wait wait;
+            while (miss) {
+                uint64_t w[SPT][2];
+#pragma unroll
+                for (int u = 0; u < SPT; u++)
+                    if ((miss >> u) & 1u) {
+                        const uint64_t* q = bank + (size_t)(tid + u * NTH) * 2;
+                        w[u][0] = get(q);
+                        w[u][1] = get(q + 1);
+                    }
+#pragma unroll
+                for (int u = 0; u < SPT; u++)
+                    if (((miss >> u) & 1u) && of_step(w[u][0], n) && of_step(w[u][1], n)) {
+                        const int q = tid + u * NTH;
+                        const unsigned iy = ((unsigned)(w[u][0] >> 32) << 16) | ((unsigned)(w[u][1] >> 32) & 0xffffu);
+                        s_pos[q] = make_float4(__uint_as_float((uint32_t)w[u][0]), __uint_as_float(iy),
+                                               __uint_as_float((uint32_t)w[u][1]), s_tyf[q]);
+                        fl |= (unsigned)(w[u][0] >> 48) & 7u;
+                        miss &= ~(1u << u);
+                    }
+                if (miss && wait.late()) {
+                    atomicOr(a.err, MD_PK_ERR_WAIT);
+                    fl |= FL_STOP;
+                    break;
+                }
+            }
+        } else {
+            for (int q = tid; q < a.natom; q += NTH) {
+                const float4 y = a.pos[cb0][q];
+                s_pos[q] = make_float4(y.x, y.y, y.z, s_tyf[q]);
+            }
         }
-        // The previous step's sums, wanted by the Berendsen factor (every workgroup)
-        // and the statistics record (workgroup 0): loaded now by wavefront 0, added
-        // after the pair loop (in the same order everywhere).  The bank stays intact
-        // until this workgroup has passed its next barrier.
-        const bool want_sums = k > 0 && wave == 0 && (need_lam || (blockIdx.x == 0 && a.stats));
-        double t0 = 0.0, t1 = 0.0, t2 = 0.0;
-        if (want_sums && lane < a.nwg) {
-            const double* pb = a.pub + (size_t)((b - 1) & 1) * MD_PK_WG * 4;
-            t0 = pb[lane * 4 + 0];
-            t1 = pb[lane * 4 + 1];
-            t2 = pb[lane * 4 + 2];
-        }
+        if (fl) atomicOr(&s_bits[k & 1], fl);
         __syncthreads();
+        const unsigned bits = s_bits[k & 1];
+        if (tid == 0) s_bits[(k + 1) & 1] = 0u;   // read by all before this step's barriers
+        if (bits & FL_STOP) break;
         // rows: at the first step and after any skin trip.  The atom's G lanes test
         // the slots j = c G + lane in chunks c and compact the hits in slot order,
         // entry e of the row going to lane e mod G: the lanes' rows differ in length
@@ -190,16 +260,16 @@ __global__ __launch_bounds__(MD_PK_THREADS) void k_persist(const PersistArgs a) 
             xb = x;
             const int g0 = lane & ~(G - 1);   // the group's first lane in the wavefront
             int n = 0;                        // the atom's entries so far (the same in its G lanes)
-            for (int j0 = 0; j0 < a.nslot; j0 += G) {
+            for (int j0 = 0; j0 < a.natom; j0 += G) {
                 const int j = j0 + sub;
                 bool hit = false;
-                if (active && j < a.nslot) {
+                if (active && j < a.natom) {
                     const float4 pj = s_pos[j];
                     const float dx = minimg(x.x - pj.x, L0, Li0);
                     const float dy = minimg(x.y - pj.y, L1, Li1);
                     const float dz = minimg(x.z - pj.z, L2, Li2);
                     const float rsq = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
-                    hit = rsq < a.rl2 && j != slot && pj.w >= 0.0f;
+                    hit = rsq < a.rl2 && j != slot;
                 }
                 const unsigned gm = (unsigned)(__ballot(hit) >> g0) & ((1u << G) - 1u);
                 if (hit) {
@@ -216,7 +286,7 @@ __global__ __launch_bounds__(MD_PK_THREADS) void k_persist(const PersistArgs a) 
             if ((n + G - 1) / G > a.cap_l) mybits |= FL_ROWS;
             nbuild++;
         }
-        const bool en = a.energy_every > 0 && ((step0 + k) % a.energy_every) == 0;
+        const bool en = a.stats && a.energy_every > 0 && ((step0 + k) % a.energy_every) == 0;
         // pair forces of the own atom (this lane's share of its row), two entries per
         // LDS word so that both neighbors' loads are in flight together
         float fx = 0.f, fy = 0.f, fz = 0.f;
@@ -258,14 +328,20 @@ __global__ __launch_bounds__(MD_PK_THREADS) void k_persist(const PersistArgs a) 
         fx = group_sum<G>(fx);
         fy = group_sum<G>(fy);
         fz = group_sum<G>(fz);
+        // The previous step's sums, wanted by the Berendsen factor (every workgroup) and the
+        // statistics record (workgroup 0): read by wavefront 0 before its atoms are published,
+        // so their bank is not written again before.
+        const bool want_sums = k > 0 && wave == 0 && (need_lam || (bid == 0 && a.stats));
         if (want_sums) {   // the previous step's totals: Berendsen factor and record
+            double t0 = 0.0, t1 = 0.0, t2 = 0.0;
+            if (!sums_of((unsigned)(k + 1), t0, t1, t2) && lane == 0) atomicOr(&s_bits[(k + 1) & 1], FL_STOP);
             t0 = wave_sum_d(t0);
             t1 = wave_sum_d(t1);
             t2 = wave_sum_d(t2);
             const double T = t0 / ((double)p.nf * MD_KB_REF);
             if (need_lam && lane == 0) s_lam = sqrt(1.0 + dtd / taud * ((double)p.T0 / T - 1.0));
             const long long ks = k - 1;
-            if (blockIdx.x == 0 && lane == 0 && a.stats && ks < a.stat_cap) {
+            if (bid == 0 && lane == 0 && a.stats && ks < a.stat_cap) {
                 const bool en_p = a.energy_every > 0 && ((step0 + ks) % a.energy_every) == 0;
                 StatRec rec;
                 rec.ke = 0.5 * t0;
@@ -284,10 +360,8 @@ __global__ __launch_bounds__(MD_PK_THREADS) void k_persist(const PersistArgs a) 
                 a.stats[ks] = rec;
             }
         }
-        if (need_lam && k > 0) {
-            __syncthreads();   // s_lam
-            lamd = s_lam;
-        }
+        __syncthreads();   // every row is walked: s_pos is free for the next step; s_lam
+        if (need_lam && k > 0) lamd = s_lam;
         // integrate (every lane of the group holds the same bits; lane 0 stores)
         double dke = 0.0;
         const bool last = k + 1 == nsteps;
@@ -300,14 +374,14 @@ __global__ __launch_bounds__(MD_PK_THREADS) void k_persist(const PersistArgs a) 
                 v.x = fmaf(fx, massif, v.x) * lam;
                 v.y = fmaf(fy, massif, v.y) * lam;
                 v.z = fmaf(fz, massif, v.z) * lam;
-                dke = ((double)v.x * v.x + (double)v.y * v.y + (double)v.z * v.z) / (double)v.w;
+                if (need_ke) dke = ((double)v.x * v.x + (double)v.y * v.y + (double)v.z * v.z) / (double)v.w;
             } else {
                 // v(t) = v(t - dt/2) + F dt/2m ends the step; v(t + dt/2) = v(t) + F dt/2m begins the next
                 const float h = 0.5f * a.dt * v.w;
                 v.x = fmaf(fx, h, v.x);
                 v.y = fmaf(fy, h, v.y);
                 v.z = fmaf(fz, h, v.z);
-                dke = ((double)v.x * v.x + (double)v.y * v.y + (double)v.z * v.z) / (double)v.w;
+                if (need_ke) dke = ((double)v.x * v.x + (double)v.y * v.y + (double)v.z * v.z) / (double)v.w;
                 drift = !last;
                 if (drift) {
                     v.x = fmaf(fx, h, v.x);
@@ -317,54 +391,56 @@ __global__ __launch_bounds__(MD_PK_THREADS) void k_persist(const PersistArgs a) 
             }
             if (drift) {
                 x = make_float4(fmaf(v.x, a.dt, x.x), fmaf(v.y, a.dt, x.y), fmaf(v.z, a.dt, x.z), x.w);
-                if (sub == 0) a.pos[(int)((sx + 1) & 1)][slot] = x;
                 const float ddx = minimg(x.x - xb.x, L0, Li0), ddy = minimg(x.y - xb.y, L1, Li1),
                             ddz = minimg(x.z - xb.z, L2, Li2);
                 if (fmaf(ddz, ddz, fmaf(ddy, ddy, ddx * ddx)) >= a.skin2q) mybits |= FL_TRIP;   // src/neighborlist.cu:174
                 if (!(fabsf(x.x) <= L0 && fabsf(x.y) <= L1 && fabsf(x.z) <= L2)) mybits |= FL_STOP;
             }
+            if (sub == 0) {
+                if (mybits & FL_STOP) atomicOr(a.err, 1);   // an atom left the box: unstable
+                if (mybits & FL_ROWS) {                      // the run is replayed with longer rows
+                    atomicOr(a.err, MD_PK_ERR_ROWS);
+                    mybits |= FL_STOP;
+                }
+                if (!last) publish((unsigned)(k + 2), x, mybits);
+            }
             if (sub != 0) dke = 0.0;
         }
-        // the workgroup's partial sums and flag bits
-        const double q0 = need_ke ? wave_sum_d(dke) : 0.0;
-        const double q1 = en ? wave_sum_d(elj) : 0.0;
-        const double q2 = en ? wave_sum_d(evi) : 0.0;
-        const unsigned wb = (__ballot((mybits & FL_TRIP) != 0) ? FL_TRIP : 0u) |
-                            (__ballot((mybits & FL_ROWS) != 0) ? FL_ROWS : 0u) |
-                            (__ballot((mybits & FL_STOP) != 0) ? FL_STOP : 0u);
-        if (lane == 0) {
-            s_red[wave][0] = q0;
-            s_red[wave][1] = q1;
-            s_red[wave][2] = q2;
-            if (wb) atomicOr(&s_wgb, wb);
+        if (need_ke) {   // the workgroup's partial sums
+            const double q0 = wave_sum_d(dke);
+            const double q1 = en ? wave_sum_d(elj) : 0.0;
+            const double q2 = en ? wave_sum_d(evi) : 0.0;
+            if (lane == 0) {
+                s_red[wave][0] = q0;
+                s_red[wave][1] = q1;
+                s_red[wave][2] = q2;
+            }
+            __syncthreads();
+            if (tid < 3) {
+                double t = s_red[0][tid];
+                for (int w = 1; w < NW; w++) t += s_red[w][tid];
+                const uint64_t d = (uint64_t)__double_as_longlong(t);
+                const unsigned n = (unsigned)(k + 2);
+                uint64_t* q = a.pub + ((size_t)(n & 1) * MD_PK_WG + bid) * 6 + 2 * tid;
+                put(q, (uint32_t)d, n << 3);
+                put(q + 1, (uint32_t)(d >> 32), n << 3);
+            }
         }
-        __syncthreads();
-        unsigned wgbits = s_wgb;
-        if (tid < 3 && need_ke) {
-            double t = s_red[0][tid];
-            for (int w = 1; w < NW; w++) t += s_red[w][tid];
-            a.pub[((size_t)(b & 1) * MD_PK_WG + blockIdx.x) * 4 + tid] = t;
+        if (!last) {
+            __syncthreads();
+            if (tid == 0) put(a.hint + (k & 1) * MD_PK_WG + bid, (unsigned)(k + 2), 0u);
         }
-        if ((wgbits & FL_STOP) && tid == 0) atomicOr(a.err, 1);   // an atom left the box: unstable
-        if ((wgbits & FL_ROWS) && tid == 0) atomicOr(a.err, MD_PK_ERR_ROWS);
-        if (wgbits & FL_ROWS) wgbits |= FL_STOP;   // the run is replayed with longer rows
-        bits = pk_barrier(a, b++, wgbits, &s_bits);
         done = k + 1;
     }
     // the last step's record and factor
     if (done == nsteps && nsteps > 0) {
-        if (wave == 0) {
-            const double* pb = a.pub + (size_t)((b - 1) & 1) * MD_PK_WG * 4;
+        if (wave == 0 && bid == 0) {
             double t0 = 0.0, t1 = 0.0, t2 = 0.0;
-            if (lane < a.nwg) {
-                t0 = pb[lane * 4 + 0];
-                t1 = pb[lane * 4 + 1];
-                t2 = pb[lane * 4 + 2];
-            }
+            if (need_ke) sums_of((unsigned)(nsteps + 1), t0, t1, t2);
             t0 = wave_sum_d(t0);
             t1 = wave_sum_d(t1);
             t2 = wave_sum_d(t2);
-            if (blockIdx.x == 0 && lane == 0) {
+            if (lane == 0) {
                 const long long ks = nsteps - 1;
                 const double T = t0 / ((double)p.nf * MD_KB_REF);
                 if (a.stats && ks < a.stat_cap) {
@@ -394,6 +470,7 @@ __global__ __launch_bounds__(MD_PK_THREADS) void k_persist(const PersistArgs a) 
             }
         }
         if (active && sub == 0) {
+            a.pos[(int)((step0 + nsteps) & 1)][slot] = x;
             a.vel[slot] = v;
             a.force[slot] = f;
         }
@@ -402,7 +479,7 @@ __global__ __launch_bounds__(MD_PK_THREADS) void k_persist(const PersistArgs a) 
 
 extern "C" hipError_t md_launch_persist(const PersistArgs& a, int lanes, size_t shmem, hipStream_t st, hipEvent_t ev0,
                                         hipEvent_t ev1) {
-    const dim3 grid(a.nwg), block(MD_PK_THREADS);
+    const dim3 grid(a.nwg * a.spread), block(a.nth);
     const bool nt1 = a.ntype == 1;
     hipError_t rc = hipSuccess;
     auto go = [&](auto kern) {
@@ -413,10 +490,15 @@ extern "C" hipError_t md_launch_persist(const PersistArgs& a, int lanes, size_t 
         if (ev0) hipExtLaunchKernelGGL(kern, grid, block, shmem, st, ev0, ev1, 0, a);
         else hipLaunchKernelGGL(kern, grid, block, shmem, st, a);
     };
+    auto pick = [&](auto g) {
+        constexpr int G = decltype(g)::value;
+        if (a.nth == 512) nt1 ? go(k_persist<G, true, 512>) : go(k_persist<G, false, 512>);
+        else nt1 ? go(k_persist<G, true, 1024>) : go(k_persist<G, false, 1024>);
+    };
     switch (lanes) {
-    case 4: nt1 ? go(k_persist<4, true>) : go(k_persist<4, false>); break;
-    case 8: nt1 ? go(k_persist<8, true>) : go(k_persist<8, false>); break;
-    case 16: nt1 ? go(k_persist<16, true>) : go(k_persist<16, false>); break;
+    case 4: pick(std::integral_constant<int, 4>{}); break;
+    case 8: pick(std::integral_constant<int, 8>{}); break;
+    case 16: pick(std::integral_constant<int, 16>{}); break;
     default: return hipErrorInvalidValue;
     }
     if (rc != hipSuccess) return rc;

@@ -998,7 +998,7 @@ __global__ __launch_bounds__(256) void k_copy_plan(const CopyPlan c) {
 // Start of a run, in one launch (it was five: copies, fills of the list maxima and the error
 // word, thermostat, targets; 21 us of kernels and as many gaps): the copy of the state that a
 // run may be rolled back to, and
-//   list maxima, the error word and the persistent kernel's barrier flags cleared
+//   list maxima, the error word and the persistent kernel's exchange buffer cleared
 //   target = step + nsteps for every replica, gates recounted (a.nsteps < 0: neither)
 //   velocity Verlet's begin-of-step thermostat half from ke2_cur -> S (a.th_begin)
 // The last workgroup copies the replicas' states, thermostats and the gates itself before it
@@ -1009,13 +1009,12 @@ __global__ __launch_bounds__(256) void k_run_begin(const RunBeginArgs a) {
         const long long first = (long long)blockIdx.x * blockDim.x + threadIdx.x, stride = (long long)nb * blockDim.x;
         copy_pairs(a.copy, first, stride);
         for (long long i = first; i < a.ntmax; i += stride) a.tmax[i] = 0;
+        for (long long i = first; i < a.npk; i += stride) a.pk_xch[i] = 0;
         return;
     }
     __shared__ int cnt[3];
     if (threadIdx.x < 3) cnt[threadIdx.x] = 0;
     if (threadIdx.x == 3) *a.err = 0;
-    if (a.pk_flags)
-        for (int i = threadIdx.x; i < 2 * MD_PK_WG; i += blockDim.x) a.pk_flags[i] = 0u;
     const Gate g0 = *a.gate;
     __syncthreads();
     int ns = 0, nr = 0, nf = 0;

@@ -198,3 +198,41 @@ def test_persist_nve_drift_10000_steps(E, orc):
     say("  drift per 1000 steps gpu", sg * 1e3, "+-", eg * 1e3, "oracle", so * 1e3, "+-", eo * 1e3)
     assert abs(H[0] - Ho[0]) <= 1e-4 * abs(Ho[0])
     assert abs(sg) <= abs(so) + 2.0 * sigma
+
+
+# the workgroups' edges: two atoms, part of a workgroup, 32 workgroups of 512 threads (they fit
+# one XCD) and 33 (then 1024 threads), the most atoms, more workgroups than an XCD has CUs
+@pytest.mark.parametrize("n,lanes", [(2, 4), (33, 16), (1024, 16), (1025, 16), (2048, 8), (2049, 8), (4096, 4),
+                                     (2049, 16), (4096, 16)])
+@pytest.mark.parametrize("thermostat", ["none", "berendsen"])
+def test_persist_workgroup_edges(E, orc, n, lanes, thermostat):
+    """Forces of the last step equal the oracle's at the positions that came with them, and the
+    recorded kinetic energy is that of the velocities, whatever the split into workgroups."""
+    say("persist edges", n, lanes, thermostat)
+    rng = np.random.default_rng(n)
+    s = S.argon(ncell=4).copy()
+    m = max(9, int(np.ceil(n ** (1 / 3))))
+    g = rng.permutation(m ** 3)[:n]
+    L = 4.0 * m
+    x = (np.stack([g // m // m, g // m % m, g % m], 1) + 0.5) * 4.0 - L / 2 + rng.uniform(-0.3, 0.3, (n, 3))
+    s.box, s.pos = np.full(3, L, np.float32), x.astype(np.float32)
+    s.vel = rng.normal(0.0, 2e-3, (n, 3)).astype(np.float32)
+    s.type, s.charge = np.zeros(n, np.int32), np.zeros(n, np.float32)
+    s.integrator, s.thermostat = ("vverlet", "none") if thermostat == "none" else ("leapfrog", "berendsen")
+    e = E.Engine.from_system(s)
+    e.set_launch(lanes=lanes, persist=1)
+    x0 = e.download()[0]
+    st = e.run(5)
+    assert e.persist_info()["runs"] == 1
+    p, v, f = e.download()
+    so = s.copy()
+    # velocity Verlet returns forces and positions of one time, leapfrog forces of the step before
+    so.pos = p if thermostat == "none" else S.wrap_centered(p.astype(np.float64) - s.dt * v.astype(np.float64),
+                                                            s.box.astype(np.float64)).astype(np.float32)
+    Fo = orc.forces(so)[0]
+    # leapfrog: the position is rounded once more (2^-23 L), against a curvature of some 1e3 kJ/mol/A^2
+    assert np.abs(f - Fo).max() <= (1e-5 if thermostat == "none" else 1e-3) * max(np.abs(Fo).max(), 1.0)
+    ke = 0.5 * (1e4 * s.ff.masses[0] * v.astype(np.float64) ** 2).sum()
+    assert abs(st["ke"][-1, 0] - ke) <= 1e-6 * ke
+    assert not np.array_equal(p, x0)
+    e.close()
