@@ -581,7 +581,10 @@ StepArgs step_args(md_engine* e, int mode, int energy_every) {
     a.jset = e->jset.p; a.jcount = e->jcount.p;
     a.tile_rep = e->tile_rep.p; a.rep = e->rep.p; a.st = e->rst.p; a.gate = e->gate.p; a.th = e->th.p; a.part = e->part.p;
     a.lst = e->lst.p; a.lagmode = 0; a.lag = 0; a.par = 0; a.open = 0;
-    a.prefilter = e->R > 1 ? 1 : 0;   // cleared for deferred-finalize blocks (every tile takes part)
+    // Cleared for deferred-finalize blocks (every tile takes part).  A single system's tiles look
+    // first once they no longer start all together (an idle launch of 196,608 water atoms
+    // 15.7 us without, 40 steps of them 7.09 -> 6.82 ms); below, the look only delays them.
+    a.prefilter = e->R > 1 || e->ntiles() >= 8 * e->ncu ? 1 : 0;
     a.vvfused = vv_fused(e) ? 1 : 0;
     a.err = e->err.p; a.stats = e->stats.p; a.stat_cap = e->stat_cap;
     a.ljtab = e->ljtab.p;
