@@ -563,6 +563,7 @@ BuildArgs build_args(md_engine* e) {
     b.key = e->key.p; b.rank = e->rank.p; b.tmp = e->tmp.p; b.tmpid = e->tmpid.p;
     b.cell_count = e->cell_count.p; b.cell_start = e->cell_start.p; b.cell_rank = e->cell_rank.p;
     b.slot_of = e->slot_of.p; b.nl16 = e->nl16.p; b.ncount = e->ncount.p; b.rperm = e->rperm.p; b.ljfree = ljfree(e);
+    b.wide = e->ntiles() <= e->ncu ? 1 : 0;
     b.jset = e->jset.p; b.jcount = e->jcount.p;
     b.tilemax = e->tmax.p; b.jmax = e->tmax.p + e->ntiles();
     b.excl = e->excl.p; b.st = e->rst.p; b.gate = e->gate.p;

@@ -435,6 +435,7 @@ struct BuildArgs {
     int* ncount;
     uint8_t* rperm;
     uint32_t ljfree;      // StepArgs
+    int wide;             // a tile's build on 16 wavefronts instead of 8
     uint32_t* jset;
     int* jcount;
     int* tilemax;         // [S/64] longest row per 64-slot tile over the builds since the host cleared it

@@ -258,9 +258,9 @@ __global__ __launch_bounds__(256) void k_nl_permute(BuildArgs a) {
     a.slot_of[myid] = f;
 }
 
-// Tile neighbor-set build: one workgroup of 8 wavefronts per 64-slot tile, 8 atoms (a
-// group of consecutive slots, so a compact one) per wavefront, their positions held as
-// wavefront-uniform values.
+// Tile neighbor-set build: one workgroup of NW = 8 (16 for few tiles) wavefronts per 64-slot
+// tile, 64 / NW atoms (a group of consecutive slots, so a compact one) per wavefront, their
+// positions held as wavefront-uniform values.
 //  1. The image cells within r_list of the tile's bounding box (region order, kTab cells a
 //     round, a thread per cell) write their members' slots to LDS, 512 per chunk.
 //  2. A thread per candidate finds the groups whose bounding box its image is within r_list of.
@@ -281,13 +281,14 @@ __global__ __launch_bounds__(256) void k_nl_permute(BuildArgs a) {
 // time; a group's own candidates are under half of the tile's.  Groups by bounding sphere
 // instead of box: 480 us (water).  80 registers keep three workgroups per CU (unbounded,
 // 114: one workgroup fewer, 542 us); 64 spill (500 us).
-template <bool EXCL>
-__global__ __launch_bounds__(512, 6) void k_nl_tbuild(BuildArgs a) {
-    constexpr int NW = 8, NT = 64 * NW, AW = 64 / NW;
+template <bool EXCL, int NW>
+__global__ __launch_bounds__(64 * NW, NW == 8 ? 6 : 4) void k_nl_tbuild(BuildArgs a) {
+    constexpr int NT = kTab, CW = NT / 64, AW = 64 / NW;   // candidates of a chunk, their wavefronts, atoms of a group
+    static_assert(NW >= CW && (NT / 64) * AW <= 64, "a candidate per thread, a mask per lane");
     __shared__ uint32_t s_cand[NT];       // the next chunk's candidates: slot | image shift code << 24
     __shared__ float4 s_cx[NT];           // the chunk: candidate position (unshifted), w = bits of the set entry
     __shared__ int s_cid[EXCL ? NT : 1];  // original index of the candidate (exclusions), bit 31: may be excluded
-    __shared__ uint2 s_gm[NW][NW];        // [wavefront of the candidates][group]: those in reach of the group
+    __shared__ uint2 s_gm[CW][NW];        // [wavefront of the candidates][group]: those in reach of the group
     __shared__ uint8_t s_hit[NT];         // the candidate hit some atom of the tile
     __shared__ uint16_t s_li[NT];         // row entry of a candidate of the set
     __shared__ uint16_t s_list[NW][NT];   // per wavefront the chunk's candidates in reach of its group
@@ -298,7 +299,7 @@ __global__ __launch_bounds__(512, 6) void k_nl_tbuild(BuildArgs a) {
     __shared__ float4 s_glo[NW], s_ghi[NW];   // per group: bounding box
     __shared__ int4 s_ex[EXCL ? 64 : 1];
     __shared__ float s_bb[6];
-    __shared__ int s_w[NW], s_cw[NW], s_wmax[NW];
+    __shared__ int s_w[NW], s_cw[CW], s_wmax[NW];
     __shared__ int s_cnt[64];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int tile = blockIdx.x;
@@ -330,7 +331,7 @@ __global__ __launch_bounds__(512, 6) void k_nl_tbuild(BuildArgs a) {
         s_shv[tid] = make_float4(-(float)kx * L0, -(float)ky * L1, -(float)kz * L2, 0.0f);
     }
     if (EXCL) {
-        s_bloom[tid] = 0u;   // NT = 512 words
+        if (tid < 512) s_bloom[tid] = 0u;
         __syncthreads();
     }
     if (tid < 64) {
@@ -353,12 +354,12 @@ __global__ __launch_bounds__(512, 6) void k_nl_tbuild(BuildArgs a) {
             lx = fminf(lx, __shfl_xor(lx, o, 64)); ly = fminf(ly, __shfl_xor(ly, o, 64)); lz = fminf(lz, __shfl_xor(lz, o, 64));
             hx = fmaxf(hx, __shfl_xor(hx, o, 64)); hy = fmaxf(hy, __shfl_xor(hy, o, 64)); hz = fmaxf(hz, __shfl_xor(hz, o, 64));
         };
-        for (int o = 1; o <= 4; o <<= 1) grow(o);
-        if ((lane & 7) == 0) {
-            s_glo[lane >> 3] = make_float4(lx, ly, lz, 0.0f);
-            s_ghi[lane >> 3] = make_float4(hx, hy, hz, 0.0f);
+        for (int o = 1; o < AW; o <<= 1) grow(o);
+        if ((lane & (AW - 1)) == 0) {
+            s_glo[lane / AW] = make_float4(lx, ly, lz, 0.0f);
+            s_ghi[lane / AW] = make_float4(hx, hy, hz, 0.0f);
         }
-        for (int o = 8; o <= 32; o <<= 1) grow(o);
+        for (int o = AW; o <= 32; o <<= 1) grow(o);
         if (tid == 0) {
             s_bb[0] = lx; s_bb[1] = ly; s_bb[2] = lz;
             s_bb[3] = hx; s_bb[4] = hy; s_bb[5] = hz;
@@ -428,10 +429,9 @@ __global__ __launch_bounds__(512, 6) void k_nl_tbuild(BuildArgs a) {
             };
             // ---- a region cell per thread: its first slot and image shift (cell), members (n)
             //      and the index of its first member among the candidates (first)
-            static_assert(kTab == NT, "a region cell per thread");
             int code = 0, n = 0;
             uint32_t cell = 0;
-            if (b0 + tid < nreg) {
+            if (tid < NT && b0 + tid < nreg) {
                 const int c = locate(b0 + tid, code);
                 if (c >= 0) {
                     const int rank = a.cell_rank[cell_off + c];
@@ -441,7 +441,7 @@ __global__ __launch_bounds__(512, 6) void k_nl_tbuild(BuildArgs a) {
                 }
             }
             int T;
-            const int first = block_scan<NT>(n, s_w, T);
+            const int first = block_scan<64 * NW>(n, s_w, T);
             // the candidates [q0, q0 + NT) to s_cand, each cell's by its thread
             auto expand = [&](int q0) {
                 const int e = min(first + n, q0 + NT);
@@ -461,14 +461,14 @@ __global__ __launch_bounds__(512, 6) void k_nl_tbuild(BuildArgs a) {
             };
             expand(0);
             __syncthreads();
-            if (tid < T) fetch();
+            if (tid < min(T, NT)) fetch();
             __syncthreads();   // s_cand is read before the next chunk's candidates replace it
             for (int base = 0; base < T; base += NT) {
                 float4 cx = nx;
                 const uint32_t info = nj | ((uint32_t)nty << MD_JBITS);
                 const int cid = nid;
                 // groups in reach: the image within `reach` of the group's bounding box
-                {
+                if (NW == CW || tid < NT) {
                     const bool valid = base + tid < T;
                     const float4 sv = s_shv[valid ? nj >> MD_SLOTBITS : MD_SHIFT0];
                     const float ix = valid ? cx.x - sv.x : MD_FAR, iy = cx.y - sv.y, iz = cx.z - sv.z;
@@ -485,23 +485,23 @@ __global__ __launch_bounds__(512, 6) void k_nl_tbuild(BuildArgs a) {
                         ghi = writelane((int)(uint32_t)(in >> 32), g, ghi);
                     }
                     if (lane < NW) s_gm[wave][lane] = make_uint2((uint32_t)glo, (uint32_t)ghi);
+                    cx.w = __uint_as_float(info);
+                    s_cx[tid] = cx;
+                    s_hit[tid] = 0;
                 }
-                cx.w = __uint_as_float(info);
-                s_cx[tid] = cx;
-                s_hit[tid] = 0;
-                if (EXCL) {
+                if (EXCL && (NW == CW || tid < NT)) {
                     const bool may = ((s_bloom[(cid >> 5) & 511] >> (cid & 31)) & 1u) &&
                                      ((s_bloom[excl_hash(cid) >> 5] >> (excl_hash(cid) & 31)) & 1u);
                     s_cid[tid] = cid | (may ? (int)0x80000000 : 0);
                 }
                 if (base + NT < T) expand(base + NT);
                 __syncthreads();
-                if (base + NT + tid < T) fetch();
+                if (tid < NT && base + NT + tid < T) fetch();
                 // ---- this wavefront's candidates of the chunk
                 int nl = 0;
-                const uint2 gm = s_gm[lane & (NW - 1)][wave];
+                const uint2 gm = s_gm[lane & (CW - 1)][wave];
 #pragma unroll
-                for (int w = 0; w < NW; w++) {
+                for (int w = 0; w < CW; w++) {
                     const uint32_t g0 = (uint32_t)__builtin_amdgcn_readlane((int)gm.x, w),
                                    g1 = (uint32_t)__builtin_amdgcn_readlane((int)gm.y, w);
                     const unsigned long long in = ((unsigned long long)g1 << 32) | g0;
@@ -509,7 +509,7 @@ __global__ __launch_bounds__(512, 6) void k_nl_tbuild(BuildArgs a) {
                     if (__builtin_amdgcn_inverse_ballot_w64(in)) s_list[wave][e] = (uint16_t)(w * 64 + lane);
                     nl += __popcll(in);
                 }
-                // ---- distance tests: hit masks of batch b and atom i in lane 8 b + i
+                // ---- distance tests: hit masks of batch b and atom i in lane AW b + i
                 int mlo = 0, mhi = 0;
                 const int nbat = (nl + 63) >> 6;
                 for (int b = 0; b < nbat; b++) {
@@ -561,12 +561,12 @@ __global__ __launch_bounds__(512, 6) void k_nl_tbuild(BuildArgs a) {
                 }
                 __syncthreads();
                 // ---- the chunk's set entries
-                const unsigned long long hm = __builtin_amdgcn_ballot_w64(s_hit[tid] != 0);
-                if (lane == 0) s_cw[wave] = __popcll(hm);
+                const unsigned long long hm = __builtin_amdgcn_ballot_w64(tid < NT && s_hit[tid & (NT - 1)] != 0);
+                if (lane == 0 && wave < CW) s_cw[wave] = __popcll(hm);
                 __syncthreads();
                 int li = jn + 1 + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(hm >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)hm, 0u));
 #pragma unroll
-                for (int w = 0; w < NW; w++) {
+                for (int w = 0; w < CW; w++) {
                     if (w < wave) li += s_cw[w];
                     jn += s_cw[w];
                 }
@@ -779,8 +779,16 @@ extern "C" hipError_t md_launch_rebuild(const BuildArgs& a, int commit, hipStrea
     hipLaunchKernelGGL(k_nl_scatter, dim3(nb), dim3(256), 0, st, a);
     hipLaunchKernelGGL(k_nl_permute, dim3(nb), dim3(256), 0, st, a);
     const dim3 ntiles(a.nslot / 64);
-    if (a.has_excl) hipLaunchKernelGGL((k_nl_tbuild<true>), ntiles, dim3(512), 0, st, a);
-    else hipLaunchKernelGGL((k_nl_tbuild<false>), ntiles, dim3(512), 0, st, a);
+    // 16 wavefronts a tile (groups of four atoms) while every tile has a CU of its own:
+    // 6,591 water atoms 79 -> 65 us a build (with more tiles than CUs, two
+    // workgroups of 8 share one and the wavefronts of both are in flight already).
+    if (a.wide) {
+        if (a.has_excl) hipLaunchKernelGGL((k_nl_tbuild<true, 16>), ntiles, dim3(1024), 0, st, a);
+        else hipLaunchKernelGGL((k_nl_tbuild<false, 16>), ntiles, dim3(1024), 0, st, a);
+    } else {
+        if (a.has_excl) hipLaunchKernelGGL((k_nl_tbuild<true, 8>), ntiles, dim3(512), 0, st, a);
+        else hipLaunchKernelGGL((k_nl_tbuild<false, 8>), ntiles, dim3(512), 0, st, a);
+    }
     if (commit) hipLaunchKernelGGL(k_nl_commit, dim3((a.nrep + 3) / 4), dim3(256), 0, st, a);
     return hipGetLastError();
 }

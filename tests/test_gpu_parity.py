@@ -517,3 +517,20 @@ def test_types_without_lennard_jones(E, lanes, coulomb, ntype):
         e.close()
     for a, b in zip(*out):
         assert np.isfinite(a).all() and np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("name", ["argon16384", "argon16385", "water16500"])
+def test_list_build_tiles_per_cu(E, orc, name):
+    """Neighbor sets where the tiles just have a CU each (256: 16 wavefronts a tile) and just
+    not (257 and 258: 8), without and with exclusions, equal the oracle's."""
+    s = water_geometry_perturbed(S.water(nmol=5500), 0.05) if name == "water16500" else lattice(int(name[5:]), 5)
+    say("list tiles", name, s.n)
+    e = E.Engine.from_system(s)
+    assert all(v == 0 for v in e.check_lists().values()), e.check_lists()
+    pos, _, _ = e.download()
+    counts, nbrs = e.neighbors()
+    oc, on = orc.nlist(pos, s.box, e.thresholds()[1], s.exclusions())
+    assert np.array_equal(counts, oc)
+    for i in range(s.n):
+        assert np.array_equal(np.sort(nbrs[i, :counts[i]]), on[i, :oc[i]]), f"atom {i}"
+    e.close()
