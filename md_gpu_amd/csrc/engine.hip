@@ -209,7 +209,7 @@ struct md_engine {
     int coul_kernel = MD_COUL_NONE;
     uint32_t ljfree = 0;          // types without Lennard-Jones interactions
 
-    int R = 0, N = 0, S = 0, ncell_total = 0;
+    int R = 0, N = 0, S = 0, ncell_total = 0, sort_lds = 0, sort_na = 0;
     std::vector<int> natom, atom_off, slot_off;
     std::vector<float> box, T0;
     std::vector<int> type_h;
@@ -474,6 +474,16 @@ int setup_cells(md_engine* e) {
         off += ncell;
     }
     e->ncell_total = off;
+    // a workgroup per replica sorts the atoms where its cells and keys fit 60 KB of LDS
+    long long mc = 0, ma = 0;
+    for (int r = 0; r < e->R; r++) {
+        const RepParam& p = e->rep_h[r];
+        mc = std::max(mc, (long long)p.nc[0] * p.nc[1] * p.nc[2]);
+        ma = std::max(ma, (long long)p.natom);
+    }
+    const long long lds = 4 * (mc + 1 + ma);
+    e->sort_lds = ma <= MD_SORT_ATOMS && lds <= 60 * 1024 ? (int)lds : 0;
+    e->sort_na = (int)((ma + 1023) / 1024);
     CHECK(e->cell_rank.alloc(off));
     CHECK(e->cell_count.alloc(off));
     CHECK(e->cell_start.alloc(off + e->R));
@@ -564,6 +574,7 @@ BuildArgs build_args(md_engine* e) {
     b.cell_count = e->cell_count.p; b.cell_start = e->cell_start.p; b.cell_rank = e->cell_rank.p;
     b.slot_of = e->slot_of.p; b.nl16 = e->nl16.p; b.ncount = e->ncount.p; b.rperm = e->rperm.p; b.ljfree = ljfree(e);
     b.wide = e->ntiles() <= e->ncu ? 1 : 0;
+    b.sort_lds = e->sort_lds; b.sort_na = e->sort_na;
     b.jset = e->jset.p; b.jcount = e->jcount.p;
     b.tilemax = e->tmax.p; b.jmax = e->tmax.p + e->ntiles();
     b.excl = e->excl.p; b.st = e->rst.p; b.gate = e->gate.p;

@@ -46,6 +46,7 @@
 #define MD_BAR_PER_KJMOL_A3 16605.390671738467   // 1 kJ/mol/A^3 in bar
 #define MD_NSTAT 8              // accumulators per replica
 #define MD_CTAB 256             // intervals of the Coulomb force table on [0, rc]
+#define MD_SORT_ATOMS 4096     // largest replica that one workgroup sorts at a build
 #define MD_SUBSHIFT 25          // list build: ranks and original indices stay below 2^25 (the slot limit is
                                 // lower); the eighth of the cell an atom sits in is packed above them
 #define MD_FAR 1.0e5f           // coordinate of the dummy neighbor (local index 0)
@@ -436,6 +437,8 @@ struct BuildArgs {
     uint8_t* rperm;
     uint32_t ljfree;      // StepArgs
     int wide;             // a tile's build on 16 wavefronts instead of 8
+    int sort_lds;         // > 0: every replica is sorted by one workgroup with this much dynamic LDS
+    int sort_na;          // and so many atoms per thread
     uint32_t* jset;
     int* jcount;
     int* tilemax;         // [S/64] longest row per 64-slot tile over the builds since the host cleared it

@@ -534,3 +534,31 @@ def test_list_build_tiles_per_cu(E, orc, name):
     for i in range(s.n):
         assert np.array_equal(np.sort(nbrs[i, :counts[i]]), on[i, :oc[i]]), f"atom {i}"
     e.close()
+
+
+@pytest.mark.parametrize("n,cell_div,L", [((2,), 2, 0), ((1024, 1025, 2048, 2049), 2, 0), ((4096,), 2, 0), ((4097, 64), 2, 0),
+                                          ((4096,), 3, 0), ((300, 5), 2, 240.0)])
+def test_sort_edges(E, orc, n, cell_div, L):
+    """Replicas at the edges of what one workgroup sorts (1, 2 and 4 atoms a thread, 4,096 and
+    more atoms, more cells than fit LDS): a sound order and lists, and the oracle's neighbor
+    sets and forces."""
+    say("sort edges", n, cell_div, L)
+    sys_ = [lattice(k, 17 + i) for i, k in enumerate(n)]
+    if L:
+        for s in sys_:
+            s.box = np.full(3, L, np.float32)
+    e = E.Engine.from_system(sys_)
+    e.set_launch(cell_div=cell_div)
+    assert all(v == 0 for v in e.check_lists().values()), e.check_lists()
+    counts, nbrs = e.neighbors()
+    F = e.compute_forces()[0]
+    off = 0
+    for s in sys_:
+        oc, on = orc.nlist(s.pos, s.box, e.thresholds()[1], s.exclusions())
+        assert np.array_equal(counts[off:off + s.n], oc)
+        for i in range(s.n):
+            assert np.array_equal(np.sort(nbrs[off + i, :oc[i]]) - off, on[i, :oc[i]]), f"atom {i}"
+        Fo = orc.forces(s)[0]
+        assert np.abs(F[off:off + s.n] - Fo).max() <= 1e-5 * max(np.abs(Fo).max(), 1.0)
+        off += s.n
+    e.close()
