@@ -16,6 +16,9 @@
 // walking its row (md_rows.h).  Each workgroup stores its FP64 sums in its own
 // slot of part (no atomics); k_fm_reduce adds the slots.
 // Algorithmic work per ordered pair: forward 65 flop + adjoint ~45 flop.
+#include <algorithm>
+
+#include "md_reduce.h"
 #include "md_rows.h"
 
 namespace {
@@ -28,7 +31,17 @@ __device__ __forceinline__ float lane_group_sum(float x) {
     return x;
 }
 
-// Common prologue of both kernels: the tables and the tile's set in LDS.
+// The same in FP64.
+template <int G>
+__device__ __forceinline__ double group_sum_d(double x) {
+    x += dpp_d<0xB1>(x);                          // quad_perm [1, 0, 3, 2]
+    x += dpp_d<0x4E>(x);                          // quad_perm [2, 3, 0, 1]
+    if constexpr (G >= 8) x += dpp_d<0x141>(x);   // row_half_mirror
+    if constexpr (G >= 16) x += dpp_d<0x140>(x);  // row_mirror
+    return x;
+}
+
+// Prologue of the adjoint walk: the tables and the tile's set in LDS.
 template <int COUL>
 __device__ __forceinline__ void fm_stage(const StepArgs& a, int tile, int r, float4* s_j, float4* s_lj, float4* s_ct,
                                          float4* s_sh, const float4* __restrict__ pin) {
@@ -146,34 +159,75 @@ __global__ __launch_bounds__(64 * G) void k_fm_adjoint(const StepArgs a, double*
 //   bc = sum_j q_j C(r)/r^2 d_ij,
 //   dloss/dlj1[ti,t] = (2/M) sum_i R_i . b14[t],  dloss/dlj2[ti,t] = -(2/M) sum_i R_i . b8[t],
 //   dloss/dqscale = (2/M) sum_i 2 qscale qfac q_i R_i . bc.
+// Bound by VALU issue (58 instructions a pair) and, with two workgroups a CU, by the round trips
+// before the rows: 4,096 ions x 64 frames 268 -> 244 us an evaluation with the loads of three
+// round trips issued together (six before), rows of similar length in a wavefront, parameters
+// by bit-field inserts instead of an LDS read, and the tile's sums on one wavefront (120 LDS
+// permutes in each before).
 // R_i . b is linear in b, so each lane dots the residual (known to all lanes of
 // the atom after the force reduction) with its own partial sums; a.qq_scale
 // holds qscale.
 template <int G, int COUL, int NT>
 __global__ __launch_bounds__(64 * G) void k_fm_fused(const StepArgs a, double* part) {
-    constexpr int NW = G;
     constexpr int NACC = 2 + 2 * NT * NT;
     extern __shared__ float4 s_j[];
-    __shared__ double s_red[NW][NACC];
     __shared__ float4 s_lj[64];
     __shared__ float4 s_ct[(COUL == 1 || COUL == 2) ? MD_CTAB + 1 : 1];
     __shared__ float4 s_sh[27];
-    const int tid = threadIdx.x;
+    constexpr int NTH = 64 * G, JPRE = 32 / G;
+    const int tid = threadIdx.x, lane = tid & 63;
     const int sub = tid & (G - 1), ai = tid / G;
     const int tile = xcd_block(blockIdx.x, gridDim.x);
-    const int slot = tile * 64 + ai;
+    // Three round trips before the rows are walked: the tile's order, replica, set entries (JPRE
+    // a thread; those past the set are loaded and not used) and the tables; the replica's state
+    // and the atom's data in both position buffers; the neighbors' positions.
+    const int slot = tile * 64 + a.rperm[tile * 64 + ai];   // rows of similar length share a wavefront
     const int r = __builtin_amdgcn_readfirstlane(a.tile_rep[tile]);
-    const float4* __restrict__ pin = a.pos[cur_buf(a.st[r])];
-    fm_stage<COUL>(a, tile, r, s_j, s_lj, s_ct, s_sh, pin);
-    const float qs = a.qq_scale;
-    double acc[NACC];
+    const int jn = min(a.jcount[tile], a.jcap);
+    const uint32_t* __restrict__ jt = a.jset + (size_t)tile * a.jcap;
+    uint32_t je[JPRE];
 #pragma unroll
-    for (int k = 0; k < NACC; k++) acc[k] = 0.0;
-    const int id = a.ids[slot];
+    for (int u = 0; u < JPRE; u++) je[u] = jt[min(tid + u * NTH, a.jcap - 1)];
+    if (tid < 64) s_lj[tid] = a.ljtab[tid];
+    if (COUL == 1 || COUL == 2) {
+        for (int k = tid; k <= MD_CTAB; k += NTH) s_ct[k] = a.ctab[k];
+    }
+    const RepState st = a.st[r];
+    const RepParam& p = a.rep[r];
+    const float L0 = p.L[0], L1 = p.L[1], L2 = p.L[2];
+    const int id = a.ids[slot], ti_s = a.typ[slot], nc_s = a.ncount[slot];
+    const float4 xa = a.pos[0][slot], xb = a.pos[1][slot], T = a.target[slot];
+    const uint4* __restrict__ row4 = reinterpret_cast<const uint4*>(a.nl16 + (size_t)slot * a.cap);
+    const uint4 q0 = row4[sub], q1 = row4[(a.cap >= 16 * G ? G : 0) + sub];   // block 1 when the capacity holds one
+    loads_issued();
+    stage_shift_table(s_sh, L0, L1, L2);
+    const int cb = cur_buf(st);
+    const float4* __restrict__ pin = a.pos[cb];
+    float4 xg[JPRE];
+#pragma unroll
+    for (int u = 0; u < JPRE; u++) xg[u] = pin[(tid + u * NTH < jn) ? (je[u] & MD_SLOTMASK) : 0u];
+    __syncthreads();   // the shift table
+#pragma unroll
+    for (int u = 0; u < JPRE; u++) {
+        const int k = tid + u * NTH;
+        if (k < jn) {
+            const float4 sv = s_sh[(je[u] >> MD_SLOTBITS) & 31u];
+            s_j[k + 1] = make_float4(xg[u].x + sv.x, xg[u].y + sv.y, xg[u].z + sv.z, staged_w<true>(xg[u].w, je[u]));
+        }
+    }
+    for (int k = tid + JPRE * NTH; k < jn; k += NTH) {   // sets beyond JPRE entries per thread
+        const uint32_t e = jt[k];
+        const float4 x = pin[e & MD_SLOTMASK];
+        const float4 sv = s_sh[(e >> MD_SLOTBITS) & 31u];
+        s_j[k + 1] = make_float4(x.x + sv.x, x.y + sv.y, x.z + sv.z, staged_w<true>(x.w, e));
+    }
+    if (tid == 0) s_j[0] = make_float4(MD_FAR, MD_FAR, MD_FAR, 0.0f);
+    __syncthreads();
+    const float qs = a.qq_scale;
     const bool active = id >= 0;
-    const float4 xi = pin[slot];
-    const int ti = active ? a.typ[slot] : 0;
-    const int nn = active ? min(a.ncount[slot], a.cap) : 0;
+    const float4 xi = cb ? xb : xa;
+    const int ti = active ? ti_s : 0;
+    const int nn = active ? min(nc_s, a.cap) : 0;
     const float qi = xi.w * a.qfac * (qs * qs);
     const float4* s_lji = s_lj + ti * 8;
     float f[3] = {0.0f, 0.0f, 0.0f}, bc[3] = {0.0f, 0.0f, 0.0f}, b14[NT][3], b8[NT][3];
@@ -181,10 +235,26 @@ __global__ __launch_bounds__(64 * G) void k_fm_fused(const StepArgs a, double* p
     for (int t = 0; t < NT; t++)
 #pragma unroll
         for (int c = 0; c < 3; c++) b14[t][c] = b8[t][c] = 0.0f;
-    const uint4* __restrict__ row4 = reinterpret_cast<const uint4*>(a.nl16 + (size_t)slot * a.cap);
-    walk_row<G>(s_j, row4, nn, sub, [&](const float4& pj) {
+    const int nn0 = longest_row(nn, a.ljfree, ti);
+    const float4 lj_a = s_lji[0], lj_b = s_lji[1];
+    // two types: one or the other by the type's bit, as a mask (m = ~0 for type 1)
+    auto pick = [](uint32_t m, float one, float zero) {
+        float z;
+        asm("v_bfi_b32 %0, %1, %2, %3" : "=v"(z) : "v"(m), "v"(one), "v"(zero));
+        return z;
+    };
+    walk_row_sorted<G>(s_j, row4, nn, nn0, sub, q0, q1, [&](const float4& pj) {
         const int tj = staged_type(pj);
-        const float4 lj = s_lji[tj];
+        uint32_t m = 0;
+        float4 lj;
+        if (NT == 1) {
+            lj = lj_a;
+        } else if (NT == 2) {
+            asm("v_bfe_i32 %0, %1, 0, 1" : "=v"(m) : "v"(pj.w));
+            lj = make_float4(pick(m, lj_b.x, lj_a.x), pick(m, lj_b.y, lj_a.y), 0.0f, 0.0f);
+        } else {
+            lj = s_lji[tj];
+        }
         const float d[3] = {xi.x - pj.x, xi.y - pj.y, xi.z - pj.z};
         const float rsq = fmaf(d[2], d[2], fmaf(d[1], d[1], d[0] * d[0]));
         const float ri = __builtin_amdgcn_rsqf(rsq);
@@ -208,7 +278,17 @@ __global__ __launch_bounds__(64 * G) void k_fm_fused(const StepArgs a, double* p
         }
 #pragma unroll
         for (int t = 0; t < NT; t++) {
-            const float x14 = tj == t ? w14 : 0.0f, x8 = tj == t ? w8 : 0.0f;
+            float x14, x8;
+            if (NT == 1) {
+                x14 = w14;
+                x8 = w8;
+            } else if (NT == 2) {   // the type's bit as a mask
+                x14 = t ? __uint_as_float(__float_as_uint(w14) & m) : pick(m, 0.0f, w14);
+                x8 = t ? __uint_as_float(__float_as_uint(w8) & m) : pick(m, 0.0f, w8);
+            } else {
+                x14 = tj == t ? w14 : 0.0f;
+                x8 = tj == t ? w8 : 0.0f;
+            }
 #pragma unroll
             for (int c = 0; c < 3; c++) {
                 b14[t][c] = fmaf(x14, d[c], b14[t][c]);
@@ -216,32 +296,50 @@ __global__ __launch_bounds__(64 * G) void k_fm_fused(const StepArgs a, double* p
             }
         }
     });
-    // the atom's force on all of its lanes, then the residual
+    // the atom's force on all of its lanes, then the residual; the atom's sums go to LDS and one
+    // wavefront adds the tile's, a lane per atom
+    constexpr int NS = 2 + 2 * NT;   // loss, qscale, lj1 and lj2 by partner type
 #pragma unroll
     for (int c = 0; c < 3; c++) f[c] = lane_group_sum<G>(f[c]);
-    if (active) {
-        const float4 T = a.target[slot];
-        const float R[3] = {f[0] - T.x, f[1] - T.y, f[2] - T.z};
-        if (sub == 0) acc[0] += (double)R[0] * R[0] + (double)R[1] * R[1] + (double)R[2] * R[2];
-        if (COUL <= 2)
-            acc[1] += (double)fmaf(R[2], bc[2], fmaf(R[1], bc[1], R[0] * bc[0])) * 2.0 * (double)qs *
-                      (double)a.qfac * (double)xi.w;
-        double* a1 = acc + 2;
-        double* a2 = acc + 2 + NT * NT;
+    const float R[3] = {f[0] - T.x, f[1] - T.y, f[2] - T.z};
+    double g[NS];
+    g[0] = (double)R[0] * R[0] + (double)R[1] * R[1] + (double)R[2] * R[2];
+    g[1] = 0.0;
+    if (COUL <= 2)
+        g[1] = group_sum_d<G>((double)fmaf(R[2], bc[2], fmaf(R[1], bc[1], R[0] * bc[0])) * 2.0 * (double)qs *
+                              (double)a.qfac * (double)xi.w);
+#pragma unroll
+    for (int t = 0; t < NT; t++) {
+        g[2 + t] = group_sum_d<G>((double)fmaf(R[2], b14[t][2], fmaf(R[1], b14[t][1], R[0] * b14[t][0])));
+        g[2 + NT + t] = group_sum_d<G>(-(double)fmaf(R[2], b8[t][2], fmaf(R[1], b8[t][1], R[0] * b8[t][0])));
+    }
+    __syncthreads();   // every row is walked: the staged set makes room
+    double* s_g = reinterpret_cast<double*>(s_j);   // [NS][64]
+    int* s_ti = reinterpret_cast<int*>(s_g + NS * 64);
+    if (sub == 0) {
+#pragma unroll
+        for (int k = 0; k < NS; k++) s_g[k * 64 + ai] = active ? g[k] : 0.0;
+        s_ti[ai] = ti;
+    }
+    __syncthreads();
+    if (tid >= 64) return;
+    const int tl = s_ti[lane];
+#pragma unroll
+    for (int k = 0; k < NS; k++) g[k] = s_g[k * 64 + lane];
+    double* out = part + (size_t)tile * NACC;
+    auto put = [&](int k, double v) {
+        v = wave_sum_d(v);
+        if (lane == 0) out[k] = v;
+    };
+    put(0, g[0]);
+    put(1, g[1]);
+#pragma unroll
+    for (int ta = 0; ta < NT; ta++)
 #pragma unroll
         for (int t = 0; t < NT; t++) {
-            const double g14 = (double)fmaf(R[2], b14[t][2], fmaf(R[1], b14[t][1], R[0] * b14[t][0]));
-            const double g8 = (double)fmaf(R[2], b8[t][2], fmaf(R[1], b8[t][1], R[0] * b8[t][0]));
-#pragma unroll
-            for (int ta = 0; ta < NT; ta++) {
-                if (ta == ti) {
-                    a1[ta * NT + t] += g14;
-                    a2[ta * NT + t] -= g8;
-                }
-            }
+            put(2 + ta * NT + t, ta == tl ? g[2 + t] : 0.0);
+            put(2 + NT * NT + ta * NT + t, ta == tl ? g[2 + NT + t] : 0.0);
         }
-    }
-    fm_flush<NW, NACC>(acc, s_red, part, tile);
 }
 
 // Workgroup k: out[k] = sum over the per-tile slots of accumulator k (fixed
@@ -260,7 +358,9 @@ __global__ __launch_bounds__(256) void k_fm_reduce(const double* part, int nslot
 
 template <bool FUSED, int G, int NT>
 static void launch_fm_g(const StepArgs& a, double* part, int coul, hipStream_t st) {
-    const size_t sh = (size_t)(a.jcap + 1) * sizeof(float4);
+    // the staged set; afterwards (fused) the atoms' sums and types in its place
+    const size_t sums = (2 + 2 * NT) * 64 * sizeof(double) + 64 * sizeof(int);
+    const size_t sh = std::max((size_t)(a.jcap + 1) * sizeof(float4), FUSED ? sums : 0);
     const dim3 grid(a.ntiles), blk(64 * G);
     switch (coul) {
     case 0: hipLaunchKernelGGL((FUSED ? k_fm_fused<G, 0, NT> : k_fm_adjoint<G, 0, NT>), grid, blk, sh, st, a, part); break;

@@ -90,6 +90,17 @@ __device__ __forceinline__ void walk_row_from(const float4* s_j, const uint4* __
     }
 }
 
+// The longest row of a wavefront whose lane groups hold atoms in rperm's order (decreasing
+// length, atoms of ljfree types after the others); nn, type: the lane's atom's.
+__device__ __forceinline__ int longest_row(int nn, uint32_t ljfree, int type) {
+    int n = __builtin_amdgcn_readfirstlane(nn);
+    if (ljfree != 0) {
+        const unsigned long long fm = __ballot(((ljfree >> type) & 1) != 0);
+        if (fm) n = max(n, __builtin_amdgcn_readlane(nn, __builtin_ctzll(fm)));
+    }
+    return n;
+}
+
 // walk_row_from for a workgroup whose lane groups hold a tile's atoms by
 // decreasing row length (the step kernel's rperm order).  nn0 = the wavefront's
 // longest row: in its last block no lane of the wavefront has more entries than

@@ -595,14 +595,8 @@ __global__ __launch_bounds__(64 * G, COUL == 3 ? 5 : 4) void k_step(const StepAr
     // without any Lennard-Jones interaction (a.ljfree; water's hydrogens) after the others, so
     // whole wavefronts leave the term out: 27 VALU instructions per pair instead of 35 (40
     // steps of 196,608 water atoms 7.51 -> 7.23 ms, the same bits).
-    int nn0 = __builtin_amdgcn_readfirstlane(nn);   // the wavefront's longest row
-    bool ljw = true;                                // any atom of it has the term
-    if (LJF) {
-        const bool fr = ((a.ljfree >> tyi) & 1) != 0;
-        const unsigned long long fm = __ballot(fr);
-        if (fm) nn0 = max(nn0, __builtin_amdgcn_readlane(nn, __builtin_ctzll(fm)));
-        ljw = __ballot(active && !fr) != 0;
-    }
+    const int nn0 = longest_row(nn, LJF ? a.ljfree : 0u, tyi);
+    const bool ljw = !LJF || __ballot(active && !((a.ljfree >> tyi) & 1)) != 0;   // any atom of the wavefront has the term
     if (ENMODE != 0 && en)
         walk_row_sorted<G>(s_j, row4, nn, nn0, sub, q0, q1, [&](const float4& pj) { pair(pj, std::true_type{}, std::true_type{}); });
     else if (!LJF || ljw)

@@ -98,3 +98,39 @@ def test_adam_step_through_torch_wrapper(problem):
     say("fm adam losses", losses)
     assert losses[-1] < losses[0]
     assert np.all(np.isfinite(theta))
+
+
+
+@pytest.mark.parametrize("lanes", [4, 8, 16])
+@pytest.mark.parametrize("ntype", [1, 2, 3])
+@pytest.mark.parametrize("coulomb", ["rf", "wolf", "damped"])
+def test_one_pass_small_matches_oracle(orc, lanes, ntype, coulomb):
+    """The single pass with every table size (1, 2 and 4 types), lane count and Coulomb kind, on
+    frames with a partial last tile, at the bars of the full-size problem."""
+    import dataclasses
+    from md_gpu_amd import engine as E, systems as S
+    from md_gpu_amd.fit import ForceMatch
+    say("fm small", lanes, ntype, coulomb)
+    s = S.nacl(nsites=10)
+    k = [0, 1, 1][:ntype]
+    ff = dataclasses.replace(s.ff, names=["Na", "Cl", "Br"][:ntype], masses=s.ff.masses[k], rc=8.0,
+                             lj1=s.ff.lj1[np.ix_(k, k)], lj2=s.ff.lj2[np.ix_(k, k)],
+                             coulomb={"rf": S.COUL_RF, "wolf": S.COUL_WOLF, "damped": S.COUL_DAMPED}[coulomb])
+    typ = np.zeros_like(s.type) if ntype == 1 else s.type.copy()
+    if ntype == 3:
+        typ[::3] = np.where(typ[::3] == 1, 2, typ[::3])
+    base = dataclasses.replace(s, ff=ff, type=typ)
+    rng = np.random.default_rng(4)
+    frames = S.wrap_centered(base.pos + np.clip(rng.normal(0.0, 0.2, (3, base.n, 3)), -0.5, 0.5),
+                             base.box.astype(np.float64)).astype(np.float32)
+    targets = rng.normal(0.0, 50.0, frames.shape).astype(np.float32)
+    e = E.Engine.from_system(base)
+    e.set_launch(lanes=lanes)
+    ForceMatch(e, base, frames, targets)
+    loss, g1, g2, gq = e.fm_loss_grad(ff.lj1, ff.lj2, 1.0)
+    e.close()
+    lo, o1, o2, oq = orc.fm_loss_grad(frames, base.type, base.charge, base.box, ff, 1.0, targets)
+    assert abs(loss - lo) <= 1e-5 * lo
+    assert abs(gq - oq) <= 1e-5 * abs(oq)
+    np.testing.assert_allclose(g1, o1, rtol=1e-5, atol=1e-5 * np.abs(o1).max())
+    np.testing.assert_allclose(g2, o2, rtol=1e-5, atol=1e-5 * np.abs(o2).max())
