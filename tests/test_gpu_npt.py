@@ -101,3 +101,30 @@ def test_athom_npt_writes_the_coupled_box(tmp_path, orc):
     d = pos.astype(np.float64) - ref["pos"]
     d -= box * np.rint(d / box)
     assert np.abs(d).max() < 5e-4
+
+
+@pytest.mark.parametrize("ncell,drop", [(8, 0), (9, 803), (9, 0), (13, 0)])
+def test_npt_scaling_past_the_loaded_positions(ncell, drop):
+    """Every slot is scaled, also past the positions the finalize loads early (2,048 with 4
+    lanes an atom, 8,192 with 16): one coupled step with 4 and 16 lanes gives the same box and
+    positions to FP32 rounding of the force sums, and the scaling moves every atom."""
+    from md_gpu_amd import engine as E
+    say("npt scaling", ncell, drop)
+    s = S.argon(ncell=ncell)
+    n = s.n - drop
+    s.pos, s.vel, s.type, s.charge = s.pos[:n].copy(), s.vel[:n].copy(), s.type[:n].copy(), s.charge[:n].copy()
+    s = dataclasses.replace(s, integrator="leapfrog", thermostat="berendsen", barostat="berendsen", tau=100.0,
+                            P0=1.0, tau_p=20.0, compress=4.5e-3)
+    out = []
+    for lanes in (4, 16):
+        e = E.Engine.from_system(s)
+        e.set_launch(lanes=lanes)
+        e.run(1, stats=False)
+        out.append((e.download()[0].astype(np.float64), np.asarray(e.box(), np.float64).ravel()))
+        e.close()
+    (p4, b4), (p16, b16) = out
+    assert np.all(np.abs(b4 - b16) <= 1e-6 * b4)
+    assert np.abs(b4 / s.box - 1.0).min() > 1e-6          # the box was scaled
+    d = p4 - p16
+    d -= b4 * np.rint(d / b4)
+    assert np.abs(d).max() <= 4e-6 * b4.max()
