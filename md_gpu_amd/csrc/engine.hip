@@ -16,6 +16,7 @@
 // tripped the skin criterion (src/neighborlist.cu:36,157-176) idles until the
 // next rebuild chain in the segment.
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -276,6 +277,8 @@ struct md_engine {
     int pk_req = 0;                // list capacity the caller set (entries per atom): bounds the lane rows
     long long pk_runs = 0, pk_replays = 0;   // runs on the persistent kernel, replays after a row overflow
     size_t lds_max = 65536;        // LDS per workgroup on this device
+    bool pk_placed = true;         // persistent kernel: all workgroups on XCD pk_xcd while they fit
+    int pk_xcd = 0;
     DBuf<uint64_t> pk_xch;         // published positions and sums (persistent kernel)
     static constexpr double kQueueRatio0 = 1.15;
     double queue_ratio = kQueueRatio0;   // launched / completed steps, learned per launch configuration
@@ -1049,6 +1052,8 @@ int md_create(md_engine** out, int device) {
         md_destroy(e);
         return fail(MD_E_HIP, "hipHostMalloc failed");
     }
+    static std::atomic<unsigned> engines{0};
+    e->pk_xcd = (int)(engines++ % 8);
     if (!ev_get(e, 1)) {   // events 0 and 1 exist from here on: timing allocates no events later
         md_destroy(e);
         return fail(MD_E_HIP, "hipEventCreate failed");
@@ -1554,7 +1559,7 @@ bool persist_ok(const md_engine* e) { return e->persist && persist_eligible(e); 
 int persist_xcd(const md_engine* e) { return std::min(e->ncu / 8, MD_PK_WG); }
 int persist_wgs(const md_engine* e, int nth) { return (e->N + nth / e->lanes - 1) / (nth / e->lanes); }
 int persist_threads(const md_engine* e) {
-    return persist_wgs(e, MD_PK_THREADS / 2) <= persist_xcd(e) ? MD_PK_THREADS / 2 : MD_PK_THREADS;
+    return e->pk_placed && persist_wgs(e, MD_PK_THREADS / 2) <= persist_xcd(e) ? MD_PK_THREADS / 2 : MD_PK_THREADS;
 }
 
 // Dynamic LDS of a launch: staged positions and types (20 B per slot) and the
@@ -1583,7 +1588,8 @@ int persist_cap(const md_engine* e) {
 // rows do not fit the kernel's LDS: the caller runs the tile path instead.
 int run_persist(md_engine* e, int nsteps, int energy_every, bool want_stats, int* use_tiles) {
     *use_tiles = 0;
-    const int G = e->lanes, nth = persist_threads(e), nwg = persist_wgs(e, nth);
+    const int G = e->lanes;
+    int nth = persist_threads(e), nwg = persist_wgs(e, nth);
     if (nwg > MD_PK_WG) {   // (S <= MD_PK_SLOTS and 64 atoms or more per workgroup keep nwg <= 64)
         *use_tiles = 1;
         return MD_OK;
@@ -1606,7 +1612,8 @@ int run_persist(md_engine* e, int nsteps, int energy_every, bool want_stats, int
         a.stats = want_stats ? e->stats.p : nullptr; a.stat_cap = e->stat_cap;
         a.nslot = e->S; a.natom = e->N; a.nth = nth; a.nwg = nwg;
         // on one XCD where they fit: workgroups are dealt to the XCDs in turn
-        a.spread = nwg <= persist_xcd(e) ? 8 : 1;
+        a.spread = e->pk_placed && nwg <= persist_xcd(e) ? 8 : 1;
+        a.xcd = a.spread > 1 ? e->pk_xcd : 0;
         a.nsteps = nsteps; a.energy_every = energy_every;
         a.leapfrog = e->in.integrator == MD_LEAPFROG ? 1 : 0;
         a.thermostat = e->in.thermostat; a.ntype = e->ff.ntype; a.cap_l = cap_l;
@@ -1622,6 +1629,15 @@ int run_persist(md_engine* e, int nsteps, int energy_every, bool want_stats, int
         HIPCHECK(md_launch_force_trip(e->rst.p, e->gate.p, e->R, 1, nullptr, 0, e->err.p, &e->report->err, e->st));
         HIPCHECK(hipStreamSynchronize(e->st));
         const int err = e->report->err;
+        if ((err & MD_PK_ERR_WAIT) && a.spread > 1) {   // the XCD is taken: replay on any CU from now on
+            CHECK(run_rollback(e));
+            HIPCHECK(hipStreamSynchronize(e->st));
+            e->pk_placed = false;
+            nth = persist_threads(e);
+            nwg = persist_wgs(e, nth);
+            e->pk_replays++;
+            continue;
+        }
         if (err & MD_PK_ERR_WAIT) return fail(MD_E_HIP, "persistent kernel: a wait for another workgroup timed out");
         if (err & MD_PK_ERR_ROWS) {   // a row outgrew its length: replay the run with longer rows
             CHECK(run_rollback(e));

@@ -376,6 +376,7 @@ struct SettleArgs {
 #define MD_PK_PUB (2 * MD_PK_WG * 7)   // words of the exchange buffer for sums and hints (positions follow)
 #define MD_PK_THREADS 1024
 #define MD_PK_TIMEOUT 50000000ull // wait limit, 100 MHz wall-clock ticks (0.5 s)
+#define MD_PK_TIMEOUT_FIRST 200000ull   // the same for the first exchange of workgroups placed on one XCD (2 ms)
 #define MD_PK_ERR_ROWS 4          // err bit: a lane's row outgrew cap_l (the run is replayed with longer rows)
 #define MD_PK_ERR_WAIT 8          // err bit: a wait timed out
 
@@ -399,7 +400,8 @@ struct PersistArgs {
     int natom;            // atoms in slots 0 .. natom - 1
     int nth;              // threads per workgroup: MD_PK_THREADS or half of them
     int nwg;              // ceil(natom / (nth / lanes))
-    int spread;           // workgroups launched per working one
+    int spread;           // workgroups launched per working one (those of residue xcd work)
+    int xcd;
     long long nsteps;
     int energy_every;
     int leapfrog;         // 1: leapfrog (thermostat none or Berendsen); 0: NVE velocity Verlet

@@ -38,7 +38,9 @@
 //
 // Bound by that latency (about 1.8 of 3.3 us a step at 864 atoms) and the walk's VALU
 // work on few CUs.  While they fit, the workgroups are placed on one XCD (the others are
-// launched for every one that works and leave: workgroups are dealt to the XCDs in turn)
+// launched for every one that works and leave: workgroups are dealt to the XCDs in turn;
+// engines take the XCDs in turn, and one that finds its XCD taken goes back to 1024 threads
+// on any CU)
 // and have 512 threads, twice as many CUs.  100 steps with a download, 864 atoms: 497
 // us with a grid barrier of release and acquire fences per step, 447 with agent-scope
 // words instead on one XCD, 428 with 512 threads, 377 without the barrier; 256 atoms, 10
@@ -70,11 +72,11 @@ __device__ __forceinline__ bool is_step(uint64_t w, unsigned n) { return (unsign
 struct Wait {
     unsigned long long t0 = 0;
     unsigned tries = 0;
-    __device__ __forceinline__ bool late() {
+    __device__ __forceinline__ bool late(unsigned long long limit) {
         if ((++tries & 63u) != 0) return false;
         const unsigned long long t = wall_clock64();
         if (tries == 64u) t0 = t;
-        return t - t0 > MD_PK_TIMEOUT;
+        return t - t0 > limit;
     }
 };
 
@@ -95,7 +97,7 @@ __global__ __launch_bounds__(NTH) void k_persist(const PersistArgs a) {
     __shared__ double s_lam;         // Berendsen factor of the current step
     __shared__ unsigned s_bits[2];   // flag bits of all atoms' last steps, by step parity
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, sub = tid & (G - 1);
-    if (blockIdx.x % a.spread) return;   // launched only for the placement
+    if ((int)(blockIdx.x % a.spread) != a.xcd) return;   // launched only for the placement
     const int bid = blockIdx.x / a.spread;
     const int slot = bid * APW + tid / G;
     const bool inr = slot < a.nslot;
@@ -141,7 +143,7 @@ __global__ __launch_bounds__(NTH) void k_persist(const PersistArgs a) {
 #pragma unroll
                 for (int c = 0; c < 6; c++) all = all && is_step(w[c], n);
                 if (all) break;
-                if (wait.late()) {
+                if (wait.late(MD_PK_TIMEOUT)) {
                     ok = false;
                     break;
                 }
@@ -183,6 +185,9 @@ __global__ __launch_bounds__(NTH) void k_persist(const PersistArgs a) {
         // each thread waits for its slots (leapfrog's first ones are the run's start)
         unsigned fl = 0;
         if (k > 0 || !a.leapfrog) {
+            // the first exchange also shows that every workgroup has its CU: placed on one XCD they
+            // may find it taken by another engine's, and the host then runs them spread out
+            const unsigned long long limit = a.spread > 1 && k <= 1 ? MD_PK_TIMEOUT_FIRST : MD_PK_TIMEOUT;
             constexpr int SPT = MD_PK_SLOTS / NTH;
             const unsigned n = (unsigned)(k + 1);
             const uint64_t* bank = a.xch + (size_t)(n & 1) * a.natom * 2;
@@ -192,7 +197,7 @@ __global__ __launch_bounds__(NTH) void k_persist(const PersistArgs a) {
                     const uint64_t* q = a.hint + (n & 1) * MD_PK_WG + lane;
                     Wait wait;
                     while ((unsigned)get(q) != n) {
-                        if (wait.late()) {
+                        if (wait.late(limit)) {
                             ok = false;
                             break;
                         }
@@ -229,7 +234,7 @@ __global__ __launch_bounds__(NTH) void k_persist(const PersistArgs a) {
                         fl |= (unsigned)(w[u][0] >> 48) & 7u;
                         miss &= ~(1u << u);
                     }
-                if (miss && wait.late()) {
+                if (miss && wait.late(limit)) {
                     atomicOr(a.err, MD_PK_ERR_WAIT);
                     fl |= FL_STOP;
                     break;

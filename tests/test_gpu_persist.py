@@ -236,3 +236,28 @@ def test_persist_workgroup_edges(E, orc, n, lanes, thermostat):
     assert abs(st["ke"][-1, 0] - ke) <= 1e-6 * ke
     assert not np.array_equal(p, x0)
     e.close()
+
+
+def test_persist_engines_side_by_side(E):
+    """Several engines' persistent runs at once, a thread each, give the bits of one alone."""
+    import threading
+    s = perturbed(S.argon(), 0.1)
+
+    def work(out, k):
+        e = persist_engine(E, s, 16)
+        for _ in range(10):
+            e.run(100, stats=False)
+        out[k] = e.download()
+        e.close()
+
+    alone, beside = {}, {}
+    work(alone, 0)
+    threads = [threading.Thread(target=work, args=(beside, k)) for k in range(3)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert len(beside) == 3
+    for k in beside:
+        for a, b in zip(alone[0], beside[k]):
+            assert np.isfinite(a).all() and np.array_equal(a, b)
