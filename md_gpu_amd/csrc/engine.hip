@@ -387,6 +387,17 @@ void make_ljtab(const md_engine* e, const float* lj1, const float* lj2, float4* 
         }
 }
 
+// types without any Lennard-Jones interaction in the tables, a bit each
+uint32_t lj_free(int nt, const float* lj1, const float* lj2) {
+    uint32_t m = 0;
+    for (int i = 0; i < nt; i++) {
+        bool none = true;
+        for (int j = 0; j < nt; j++) none &= lj1[nt * i + j] == 0.0f && lj2[nt * i + j] == 0.0f;
+        if (none) m |= 1u << i;
+    }
+    return m;
+}
+
 int upload_ljtab(md_engine* e, const float* lj1, const float* lj2) {
     std::vector<float4> t(64);
     make_ljtab(e, lj1, lj2, t.data());
@@ -557,7 +568,8 @@ int ensure_stats(md_engine* e, int nrec) {
     return MD_OK;
 }
 
-// types the step kernel's rows may leave the Lennard-Jones term out for (with charges)
+// types the step kernel's rows may leave the Lennard-Jones term out for (with charges), last in
+// the lists' row order
 uint32_t ljfree(const md_engine* e) { return e->coul_kernel != MD_COUL_NONE ? e->ljfree : 0; }
 
 // NVE velocity Verlet runs in leapfrog form (one step kernel per step)
@@ -592,7 +604,7 @@ StepArgs step_args(md_engine* e, int mode, int energy_every) {
     StepArgs a{};
     a.pos[0] = e->pos[0].p; a.pos[1] = e->pos[1].p; a.vel = e->vel.p; a.force = e->force.p;
     a.ids = e->ids.p; a.typ = e->typ.p; a.nl16 = e->nl16.p; a.ncount = e->ncount.p; a.pos_build = e->pos_build.p;
-    a.rperm = e->rperm.p; a.ljfree = ljfree(e);
+    a.rperm = e->rperm.p; a.ljfree = a.ljskip = ljfree(e);
     a.jset = e->jset.p; a.jcount = e->jcount.p;
     a.tile_rep = e->tile_rep.p; a.rep = e->rep.p; a.st = e->rst.p; a.gate = e->gate.p; a.th = e->th.p; a.part = e->part.p;
     a.lst = e->lst.p; a.lagmode = 0; a.lag = 0; a.par = 0; a.open = 0;
@@ -1086,12 +1098,7 @@ int md_set_forcefield(md_engine* e, const md_forcefield* f) {
     if (e->ff.qfac == 0.0f) e->ff.qfac = 1389.35427611722f;
     derive_ff(e);
     CHECK(upload_ljtab(e, e->ff.lj1, e->ff.lj2));
-    e->ljfree = 0;
-    for (int i = 0; i < e->ff.ntype; i++) {
-        bool none = true;
-        for (int j = 0; j < e->ff.ntype; j++) none &= e->ff.lj1[e->ff.ntype * i + j] == 0.0f && e->ff.lj2[e->ff.ntype * i + j] == 0.0f;
-        if (none) e->ljfree |= 1u << i;
-    }
+    e->ljfree = lj_free(e->ff.ntype, e->ff.lj1, e->ff.lj2);
     if (e->ff.coulomb == MD_COUL_WOLF || e->ff.coulomb == MD_COUL_DAMPED) {
         const std::vector<float4> t = coulomb_table(e->ff.alpha, e->ff.rc, e->ff.coulomb == MD_COUL_WOLF);
         HIPCHECK(hipMemcpy(e->ctab.p, t.data(), (MD_CTAB + 1) * sizeof(float4), hipMemcpyHostToDevice));
@@ -2240,6 +2247,7 @@ static int fm_evaluate(md_engine* e, const float* lj1, const float* lj2, float q
     HIPCHECK(hipMemcpyAsync(ljtab_d, e->fm_ljtab_h, 64 * sizeof(float4), hipMemcpyHostToDevice, e->st));
     StepArgs a = step_args(e, MODE_FORCE, 0);
     a.ljtab = ljtab_d;
+    a.ljskip &= lj_free(nt, lj1, lj2);   // the row order stays the build's (a.ljfree)
     a.stats = nullptr;
     const int coul = e->coul_kernel;
     hipEvent_t ev0 = e->timing ? ev_get(e, 0) : nullptr, ev1 = e->timing ? ev_get(e, 1) : nullptr;

@@ -212,7 +212,8 @@ struct StepArgs {
     int mode;             // MODE_*
     int thermostat;
     int bonded;
-    uint32_t ljfree;      // bit per type: no Lennard-Jones interaction with any type
+    uint32_t ljfree;      // types whose atoms come last in rperm (the build's BuildArgs::ljfree)
+    uint32_t ljskip;      // those of them without any Lennard-Jones interaction in this launch's ljtab
     int energy_every;     // energies at steps with step % energy_every == 0 (0: never)
     int force_energy;     // MODE_FORCE: compute energies
     int stat_cap;         // records per replica in stats
@@ -437,7 +438,7 @@ struct BuildArgs {
     uint16_t* nl16;
     int* ncount;
     uint8_t* rperm;
-    uint32_t ljfree;      // StepArgs
+    uint32_t ljfree;      // bit per type: no Lennard-Jones interaction with any type in the force field
     int wide;             // a tile's build on 16 wavefronts instead of 8
     int sort_lds;         // > 0: every replica is sorted by one workgroup with this much dynamic LDS
     int sort_na;          // and so many atoms per thread

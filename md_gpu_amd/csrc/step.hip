@@ -284,8 +284,10 @@ __device__ __forceinline__ float pair_ff(const StepArgs& a, const float4* s_ct, 
 // two entries of the atom's table row, held in registers and picked by a select
 // (no LDS read per pair); otherwise the row is read from LDS per pair.
 // LJF: types without any Lennard-Jones interaction exist (a.ljfree): a walk without the
-// term besides the other (its code costs launches of short kernels instruction fetches:
-// 30 steps of 32,768 ions with smooth PME 3.05 ms with it in every variant, else 3.02).
+// term besides the other, for wavefronts of a.ljskip types only (the row order follows the
+// force field, the term the table of the launch: force matching brings its own table).  The
+// second walk costs launches of short kernels instruction fetches: 30 steps of 32,768 ions
+// with smooth PME 3.05 ms with it in every variant, else 3.02.
 template <int G, int COUL, int ENMODE, bool NT2, bool LJF>
 __global__ __launch_bounds__(64 * G, COUL == 3 ? 5 : 4) void k_step(const StepArgs a) {
     constexpr int NW = G;                 // wavefronts: 64 atoms x G lanes
@@ -593,10 +595,10 @@ __global__ __launch_bounds__(64 * G, COUL == 3 ? 5 : 4) void k_step(const StepAr
     }
     // Lane groups hold the tile's atoms by decreasing row length (rperm), those of types
     // without any Lennard-Jones interaction (a.ljfree; water's hydrogens) after the others, so
-    // whole wavefronts leave the term out: 27 VALU instructions per pair instead of 35 (40
-    // steps of 196,608 water atoms 7.51 -> 7.23 ms, the same bits).
+    // whole wavefronts (of a.ljskip types) leave the term out: 27 VALU instructions per pair
+    // instead of 35 (40 steps of 196,608 water atoms 7.51 -> 7.23 ms, the same bits).
     const int nn0 = longest_row(nn, LJF ? a.ljfree : 0u, tyi);
-    const bool ljw = !LJF || __ballot(active && !((a.ljfree >> tyi) & 1)) != 0;   // any atom of the wavefront has the term
+    const bool ljw = !LJF || __ballot(active && !((a.ljskip >> tyi) & 1)) != 0;   // any atom of the wavefront has the term
     if (ENMODE != 0 && en)
         walk_row_sorted<G>(s_j, row4, nn, nn0, sub, q0, q1, [&](const float4& pj) { pair(pj, std::true_type{}, std::true_type{}); });
     else if (!LJF || ljw)

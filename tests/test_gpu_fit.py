@@ -134,3 +134,72 @@ def test_one_pass_small_matches_oracle(orc, lanes, ntype, coulomb):
     assert abs(gq - oq) <= 1e-5 * abs(oq)
     np.testing.assert_allclose(g1, o1, rtol=1e-5, atol=1e-5 * np.abs(o1).max())
     np.testing.assert_allclose(g2, o2, rtol=1e-5, atol=1e-5 * np.abs(o2).max())
+
+
+def _without_lj(ff, t):
+    """ff with every Lennard-Jones entry of type t zero."""
+    import dataclasses
+    lj1, lj2 = ff.lj1.copy(), ff.lj2.copy()
+    lj1[t, :] = lj1[:, t] = lj2[t, :] = lj2[:, t] = 0.0
+    return dataclasses.replace(ff, lj1=lj1, lj2=lj2)
+
+
+@pytest.mark.parametrize("lanes", [4, 8, 16])
+@pytest.mark.parametrize("free", [0, 1])
+def test_two_passes_follow_the_trial_table(orc, lanes, free):
+    """The base force field has no Lennard-Jones interactions on one type, the trial table has:
+    two passes and one pass both equal the oracle, at the bars of the full-size problem; so
+    they do for the base's own table."""
+    import dataclasses
+    from md_gpu_amd import engine as E, systems as S
+    from md_gpu_amd.fit import ForceMatch
+    say("fm type without LJ in the base", lanes, free)
+    s = S.nacl(nsites=10, ff=S.nacl_ff(rc=8.0))
+    base = dataclasses.replace(s, ff=_without_lj(s.ff, free))
+    rng = np.random.default_rng(6)
+    frames = S.wrap_centered(base.pos + np.clip(rng.normal(0.0, 0.2, (3, base.n, 3)), -0.5, 0.5),
+                             base.box.astype(np.float64)).astype(np.float32)
+    targets = rng.normal(0.0, 50.0, frames.shape).astype(np.float32)
+    e = E.Engine.from_system(base)
+    ForceMatch(e, base, frames, targets)
+    for ff in (s.ff, base.ff):
+        lo, o1, o2, oq = orc.fm_loss_grad(frames, base.type, base.charge, base.box, ff, 1.0, targets)
+        for fused in (0, 1):
+            e.set_launch(lanes=lanes, fm_fused=fused)
+            loss, g1, g2, gq = e.fm_loss_grad(ff.lj1, ff.lj2, 1.0)
+            say("  fused", fused, "loss", loss, lo)
+            assert abs(loss - lo) <= 1e-5 * lo
+            assert abs(gq - oq) <= 1e-5 * abs(oq)
+            np.testing.assert_allclose(g1, o1, rtol=1e-5, atol=1e-5 * np.abs(o1).max())
+            np.testing.assert_allclose(g2, o2, rtol=1e-5, atol=1e-5 * np.abs(o2).max())
+    e.close()
+
+
+def test_bonded_loss_follows_the_trial_table(orc):
+    """Flexible water, Lennard-Jones on the oxygens only, and a trial table with hydrogen terms
+    (bonded systems always take two passes): the loss is the oracle's."""
+    import ctypes as C
+    import dataclasses
+    from md_gpu_amd import engine as E, systems as S
+    say("fm flexible water, trial table with hydrogen terms")
+    base = S.water(nmol=343)
+    base = dataclasses.replace(base, ff=dataclasses.replace(base.ff, rc=8.0))
+    assert (base.ff.lj1[1] == 0).all()
+    eps, sig = np.array([[0.65, 0.2], [0.2, 0.1]]), np.array([[3.166, 1.5], [1.5, 1.0]])
+    trial = dataclasses.replace(base.ff, lj1=48.0 * eps * sig ** 12, lj2=24.0 * eps * sig ** 6)
+    rng = np.random.default_rng(7)
+    frame = S.wrap_centered(base.pos + np.clip(rng.normal(0.0, 0.05, (base.n, 3)), -0.1, 0.1),
+                            base.box.astype(np.float64)).astype(np.float32)
+    target = rng.normal(0.0, 50.0, (1, base.n, 3)).astype(np.float32)
+    e = E.Engine.from_system(base)
+    e.fm_set_frames(frame[None], target)
+    bonds, angles = (np.ascontiguousarray(x, np.int32) for x in (base.bonds, base.angles))
+    E._check(E.lib().md_set_topology(e._h, len(bonds), bonds.ctypes.data_as(C.c_void_p), len(angles),
+                                     angles.ctypes.data_as(C.c_void_p)))
+    for ff in (trial, base.ff):
+        so = dataclasses.replace(base.copy(), ff=ff, pos=frame)
+        lo = ((orc.forces(so)[0] - target[0]) ** 2).mean()
+        loss = e.fm_loss_grad(ff.lj1, ff.lj2, 1.0)[0]
+        say("  loss", loss, lo)
+        assert abs(loss - lo) <= 1e-5 * lo
+    e.close()
