@@ -468,10 +468,11 @@ __global__ __launch_bounds__(NTH) void k_persist(const PersistArgs a) {
                 }
                 double lam = 1.0;
                 if (a.leapfrog && a.thermostat == 1) lam = sqrt(1.0 + dtd / taud * ((double)p.T0 / T - 1.0));
-                if (a.leapfrog) a.th[0].S = lam;
-                RepState& st = a.st[0];
-                st.step = step0 + nsteps;
-                st.nb = s0.nb + nbuild;
+                // Not into the state itself: a workgroup that starts late may not have read it yet (a
+                // leapfrog run of one step without sums exchanges nothing).
+                a.end[0] = 1;
+                a.end[1] = (uint64_t)(s0.nb + nbuild);
+                a.end[2] = (uint64_t)__double_as_longlong(lam);
             }
         }
         if (active && sub == 0) {
@@ -480,6 +481,33 @@ __global__ __launch_bounds__(NTH) void k_persist(const PersistArgs a) {
             a.force[slot] = f;
         }
     }
+}
+
+// The end of a run, after every workgroup: step count, list builds and Berendsen factor into
+// the replica's state, the error word to pinned host memory and, after a run without errors,
+// the tile path's lists (built for earlier positions) stale.
+__global__ __launch_bounds__(64) void k_persist_end(const PersistArgs a, RepState* st, ThState* th, Gate* g, int* err_out) {
+    if (threadIdx.x != 0) return;
+    const int err = *a.err;
+    const uint64_t done = a.end[0], nb = a.end[1], lam = a.end[2];
+    loads_issued();
+    *err_out = err;
+    if (done) {
+        st->step += a.nsteps;
+        st->nb = (int)nb;
+        if (a.leapfrog) th->S = __longlong_as_double((long long)lam);
+    }
+    if (err) return;
+    st->trip[(done ? (int)nb : st->nb) & 1] = 1;
+    g->n_stale = 1;
+    g->n_run = 0;
+    g->n_force = 0;
+}
+
+extern "C" hipError_t md_launch_persist_end(const PersistArgs& a, RepState* s, ThState* th, Gate* g, int* err_out,
+                                            hipStream_t st) {
+    hipLaunchKernelGGL(k_persist_end, dim3(1), dim3(64), 0, st, a, s, th, g, err_out);
+    return hipGetLastError();
 }
 
 extern "C" hipError_t md_launch_persist(const PersistArgs& a, int lanes, size_t shmem, hipStream_t st, hipEvent_t ev0,

@@ -261,3 +261,30 @@ def test_persist_engines_side_by_side(E):
     for k in beside:
         for a, b in zip(alone[0], beside[k]):
             assert np.isfinite(a).all() and np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("thermostat", ["none", "berendsen"])
+@pytest.mark.parametrize("stats", [False, True])
+def test_persist_one_step_runs(E, thermostat, stats):
+    """Leapfrog runs of a single step (without sums nothing is exchanged between the workgroups),
+    from even and odd steps, between two longer ones: the tile path's trajectory.  Ten steps
+    differ by the rounding of FP32 force sums (some 1e-6 of a force) and of the positions
+    (1e-6 A each)."""
+    s = dataclasses.replace(perturbed(S.argon(), 0.1), integrator="leapfrog", thermostat=thermostat, tau=100.0, T0=120.0)
+    say("persist one-step runs", s.n, thermostat, "stats", stats)
+    out = []
+    for persist in (0, 1):
+        e = E.Engine.from_system(s)
+        e.set_launch(persist=persist, lanes=16)
+        frames = []
+        for n in (1, 1, 1, 2, 1, 1, 3):
+            e.run(n, stats=stats)
+            frames.append(e.download())
+        assert e.info()["steps"] == 10 and e.persist_info()["runs"] == 7 * persist
+        out.append(frames)
+        e.close()
+    for (p0, v0, f0), (p1, v1, f1) in zip(*out):
+        d = p1.astype(np.float64) - p0
+        d -= s.box * np.rint(d / s.box)
+        assert np.abs(d).max() < 2e-5
+        assert rel_rms(v1, v0) < 1e-5 and rel_rms(f1, f0) < 1e-5
