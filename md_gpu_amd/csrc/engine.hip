@@ -34,7 +34,7 @@
 
 extern "C" hipError_t md_launch_rebuild(const BuildArgs& a, int commit, hipStream_t st);
 extern "C" hipError_t md_launch_force_trip(RepState* s, Gate* g, int nrep, int force, int* tmax, int ntmax,
-                                           hipStream_t st);
+                                           const int* err, int* err_out, hipStream_t st);
 extern "C" hipError_t md_launch_step(const StepArgs& a, int lanes, int coul, hipStream_t st, hipEvent_t ev0,
                                      hipEvent_t ev1);
 extern "C" hipError_t md_launch_step_finalize(const StepArgs& a, int lanes, hipStream_t st);
@@ -53,8 +53,6 @@ extern "C" hipError_t md_launch_state_sums(const float4* vel, const float4* forc
                                            hipStream_t st);
 extern "C" hipError_t md_launch_persist(const PersistArgs& a, int lanes, size_t shmem, hipStream_t st, hipEvent_t ev0,
                                         hipEvent_t ev1);
-extern "C" hipError_t md_launch_persist_end(const PersistArgs& a, RepState* s, ThState* th, Gate* g, int* err_out,
-                                            hipStream_t st);
 extern "C" hipError_t md_launch_settle(const SettleArgs& a, hipStream_t st);
 extern "C" int md_launch_pme(const PmeArgs& a, const PmeFftArgs* f, hipfftHandle r2c, hipfftHandle c2r, int energy,
                              hipStream_t st);
@@ -945,13 +943,13 @@ int run_rollback(md_engine* e) {
 // Every list stale (force) and the builds' longest rows and largest sets per tile, which
 // accumulate in tmax, cleared.
 int list_begin(md_engine* e, bool force) {
-    HIPCHECK(md_launch_force_trip(e->rst.p, e->gate.p, e->R, force ? 1 : 0, e->tmax.p, 2 * e->ntiles(), e->st));
+    HIPCHECK(md_launch_force_trip(e->rst.p, e->gate.p, e->R, force ? 1 : 0, e->tmax.p, 2 * e->ntiles(), nullptr, nullptr, e->st));
     return MD_OK;
 }
 
 // Every list stale: rebuilt when next needed.
 int force_trip(md_engine* e) {
-    HIPCHECK(md_launch_force_trip(e->rst.p, e->gate.p, e->R, 1, nullptr, 0, e->st));
+    HIPCHECK(md_launch_force_trip(e->rst.p, e->gate.p, e->R, 1, nullptr, 0, nullptr, nullptr, e->st));
     return MD_OK;
 }
 
@@ -1617,8 +1615,7 @@ int run_persist(md_engine* e, int nsteps, int energy_every, bool want_stats, int
         a.pos[0] = e->pos[0].p; a.pos[1] = e->pos[1].p; a.vel = e->vel.p; a.force = e->force.p;
         a.ids = e->ids.p; a.typ = e->typ.p; a.ljtab = e->ljtab.p;
         a.st = e->rst.p; a.th = e->th.p; a.rep = e->rep.p;
-        a.pub = e->pk_xch.p; a.hint = e->pk_xch.p + 2 * MD_PK_WG * 6; a.end = e->pk_xch.p + 2 * MD_PK_WG * 7;
-        a.xch = e->pk_xch.p + MD_PK_PUB; a.err = e->err.p;
+        a.pub = e->pk_xch.p; a.hint = e->pk_xch.p + 2 * MD_PK_WG * 6; a.xch = e->pk_xch.p + MD_PK_PUB; a.err = e->err.p;
         a.stats = want_stats ? e->stats.p : nullptr; a.stat_cap = e->stat_cap;
         a.nslot = e->S; a.natom = e->N; a.nth = nth; a.nwg = nwg;
         // on one XCD where they fit: workgroups are dealt to the XCDs in turn
@@ -1635,7 +1632,8 @@ int run_persist(md_engine* e, int nsteps, int energy_every, bool want_stats, int
             if (!ev0 || !ev1) return fail(MD_E_HIP, "hipEventCreate failed");
         }
         HIPCHECK(md_launch_persist(a, G, persist_lds(e, cap_l), e->st, ev0, ev1));
-        HIPCHECK(md_launch_persist_end(a, e->rst.p, e->th.p, e->gate.p, &e->report->err, e->st));
+        // the tile path's lists were built for earlier positions: stale after a run without errors
+        HIPCHECK(md_launch_force_trip(e->rst.p, e->gate.p, e->R, 1, nullptr, 0, e->err.p, &e->report->err, e->st));
         HIPCHECK(hipStreamSynchronize(e->st));
         const int err = e->report->err;
         if ((err & MD_PK_ERR_WAIT) && a.spread > 1) {   // the XCD is taken: replay on any CU from now on

@@ -374,7 +374,7 @@ struct SettleArgs {
 // in one launch of at most MD_PK_WG workgroups of MD_PK_THREADS threads.
 #define MD_PK_SLOTS 4096          // largest system (slots): the staged positions fill at most 64 KB of LDS
 #define MD_PK_WG 64               // most workgroups (a lane of one wavefront reads each one's sums)
-#define MD_PK_PUB (2 * MD_PK_WG * 7 + 4)   // words of the exchange buffer for sums, hints and the run's end (positions follow)
+#define MD_PK_PUB (2 * MD_PK_WG * 7)   // words of the exchange buffer for sums and hints (positions follow)
 #define MD_PK_THREADS 1024
 #define MD_PK_TIMEOUT 50000000ull // wait limit, 100 MHz wall-clock ticks (0.5 s)
 #define MD_PK_TIMEOUT_FIRST 200000ull   // the same for the first exchange of workgroups placed on one XCD (2 ms)
@@ -388,13 +388,12 @@ struct PersistArgs {
     const int* ids;
     const int* typ;
     const float4* ljtab;  // [8*8] (lj1, lj2, LJ energy shift, 0)
-    const RepState* st;   // replica 0 (read by every workgroup: the run's end is stored by k_persist_end)
-    const ThState* th;
+    RepState* st;         // replica 0
+    ThState* th;
     const RepParam* rep;
     uint64_t* xch;        // [2][natom][2] published positions, zero at launch
     uint64_t* hint;       // [2][MD_PK_WG] step numbers a workgroup has published, zero at launch
     uint64_t* pub;        // [2][MD_PK_WG][6] published partial sums (2 KE, LJ, virial), zero at launch
-    uint64_t* end;        // [3] of a run that came to its end: 1, list builds so far, bits of the next factor S; zero at launch
     int* err;             // 1: an atom left the box; MD_PK_ERR_*
     StatRec* stats;       // [stat_cap] or null
     int stat_cap;

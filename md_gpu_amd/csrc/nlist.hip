@@ -825,10 +825,18 @@ __global__ __launch_bounds__(256) void k_nl_commit(BuildArgs a) {
 }
 
 // Mark the lists of all replicas stale (host-requested full rebuild; force = 0: leave
-// them) and clear the builds' maxima (ntmax of them).
-__global__ __launch_bounds__(256) void k_force_trip(RepState* st, Gate* g, int nrep, int force, int* tmax, int ntmax) {
+// them) and clear the builds' maxima (ntmax of them).  The persistent kernel's run end
+// passes its error word: the lists go stale only after a run without errors, and the
+// word goes to pinned host memory.
+__global__ __launch_bounds__(256) void k_force_trip(RepState* st, Gate* g, int nrep, int force, int* tmax, int ntmax,
+                                                    const int* err, int* err_out) {
     for (int i = blockIdx.x * 256 + threadIdx.x; i < ntmax; i += (int)gridDim.x * 256) tmax[i] = 0;
     if (blockIdx.x != 0) return;
+    if (err) {
+        const int v = *err;
+        if (threadIdx.x == 0) *err_out = v;
+        if (v) return;
+    }
     if (!force) return;
     for (int r = threadIdx.x; r < nrep; r += 256) st[r].trip[st[r].nb & 1] = 1;
     if (threadIdx.x == 0) {
@@ -925,9 +933,9 @@ extern "C" hipError_t md_launch_rebuild(const BuildArgs& a, int commit, hipStrea
 }
 
 extern "C" hipError_t md_launch_force_trip(RepState* s, Gate* g, int nrep, int force, int* tmax, int ntmax,
-                                           hipStream_t st) {
+                                           const int* err, int* err_out, hipStream_t st) {
     const int grid = std::max(1, std::min(256, (ntmax + 1023) / 1024));
-    hipLaunchKernelGGL(k_force_trip, dim3(grid), dim3(256), 0, st, s, g, nrep, force, tmax, ntmax);
+    hipLaunchKernelGGL(k_force_trip, dim3(grid), dim3(256), 0, st, s, g, nrep, force, tmax, ntmax, err, err_out);
     return hipGetLastError();
 }
 

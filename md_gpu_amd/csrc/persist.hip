@@ -121,7 +121,11 @@ __global__ __launch_bounds__(NTH) void k_persist(const PersistArgs a) {
     const double dtd = a.dt, taud = a.tau;
     double lamd = a.leapfrog ? a.th[0].S : 1.0;   // leapfrog: the factor of the run's first step
     const bool need_lam = a.leapfrog && a.thermostat == 1;
-    const bool need_ke = need_lam || a.stats != nullptr;   // the published sums have a reader
+    // The published sums have a reader.  A leapfrog run of one step exchanges no positions: it
+    // publishes them so that workgroup 0 stores the new state after everyone has read the old one
+    // (with the state stored by a launch of its own instead, which asks for nothing here, 100
+    // steps took 1 to 4 % longer: other registers throughout).
+    const bool need_ke = need_lam || a.stats != nullptr || (a.leapfrog && a.nsteps == 1);
     // the atom's position, published as step number n (into bank n & 1)
     auto publish = [&](unsigned n, float4 y, unsigned fl) {
         uint64_t* q = a.xch + ((size_t)(n & 1) * a.natom + slot) * 2;
@@ -441,7 +445,7 @@ __global__ __launch_bounds__(NTH) void k_persist(const PersistArgs a) {
     if (done == nsteps && nsteps > 0) {
         if (wave == 0 && bid == 0) {
             double t0 = 0.0, t1 = 0.0, t2 = 0.0;
-            if (need_ke) sums_of((unsigned)(nsteps + 1), t0, t1, t2);
+            if (need_ke) sums_of((unsigned)(nsteps + 1), t0, t1, t2);   // every workgroup has read st and th
             t0 = wave_sum_d(t0);
             t1 = wave_sum_d(t1);
             t2 = wave_sum_d(t2);
@@ -468,11 +472,10 @@ __global__ __launch_bounds__(NTH) void k_persist(const PersistArgs a) {
                 }
                 double lam = 1.0;
                 if (a.leapfrog && a.thermostat == 1) lam = sqrt(1.0 + dtd / taud * ((double)p.T0 / T - 1.0));
-                // Not into the state itself: a workgroup that starts late may not have read it yet (a
-                // leapfrog run of one step without sums exchanges nothing).
-                a.end[0] = 1;
-                a.end[1] = (uint64_t)(s0.nb + nbuild);
-                a.end[2] = (uint64_t)__double_as_longlong(lam);
+                if (a.leapfrog) a.th[0].S = lam;
+                RepState& st = a.st[0];
+                st.step = step0 + nsteps;
+                st.nb = s0.nb + nbuild;
             }
         }
         if (active && sub == 0) {
@@ -481,33 +484,6 @@ __global__ __launch_bounds__(NTH) void k_persist(const PersistArgs a) {
             a.force[slot] = f;
         }
     }
-}
-
-// The end of a run, after every workgroup: step count, list builds and Berendsen factor into
-// the replica's state, the error word to pinned host memory and, after a run without errors,
-// the tile path's lists (built for earlier positions) stale.
-__global__ __launch_bounds__(64) void k_persist_end(const PersistArgs a, RepState* st, ThState* th, Gate* g, int* err_out) {
-    if (threadIdx.x != 0) return;
-    const int err = *a.err;
-    const uint64_t done = a.end[0], nb = a.end[1], lam = a.end[2];
-    loads_issued();
-    *err_out = err;
-    if (done) {
-        st->step += a.nsteps;
-        st->nb = (int)nb;
-        if (a.leapfrog) th->S = __longlong_as_double((long long)lam);
-    }
-    if (err) return;
-    st->trip[(done ? (int)nb : st->nb) & 1] = 1;
-    g->n_stale = 1;
-    g->n_run = 0;
-    g->n_force = 0;
-}
-
-extern "C" hipError_t md_launch_persist_end(const PersistArgs& a, RepState* s, ThState* th, Gate* g, int* err_out,
-                                            hipStream_t st) {
-    hipLaunchKernelGGL(k_persist_end, dim3(1), dim3(64), 0, st, a, s, th, g, err_out);
-    return hipGetLastError();
 }
 
 extern "C" hipError_t md_launch_persist(const PersistArgs& a, int lanes, size_t shmem, hipStream_t st, hipEvent_t ev0,
