@@ -232,9 +232,9 @@ typedef struct md_launch_config {
                           gradient sums; 0 = a force pass, then the adjoint pass */
     int persist;       /* small single systems (one replica of at most 4,096 atoms, Lennard-Jones only,
                           no bonded terms, leapfrog or NVE velocity Verlet, no pressure coupling):
-                          1 = every step of a run in one launch of a few workgroups that meet at a
-                          grid barrier each step (1024 threads each, `lanes` per atom); other systems
-                          ignore it */
+                          1 = every step of a run in one launch of a few workgroups that exchange their
+                          positions each step (512 or 1024 threads each, `lanes` per atom); other
+                          systems ignore it */
 } md_launch_config;
 int md_set_launch(md_engine* e, const md_launch_config* cfg);
 int md_get_launch(md_engine* e, md_launch_config* cfg);
@@ -251,6 +251,18 @@ int md_autotune(md_engine* e, int nsteps, double* best_ms_per_step);
  * length (the run restarts from its first step with rows twice as long), and
  * the current row length per lane. */
 int md_persist_info(md_engine* e, long long* runs, long long* replays, int* row_len);
+/* Where its workgroups run: on one XCD while they fit.  fallbacks: runs that found
+ * the XCD taken (2 ms) and were replayed on any CU, with the same bits; hold:
+ * runs left before the XCD is tried again (md_set_launch and md_set_system try
+ * it at once).  Either pointer may be NULL. */
+int md_persist_placement(md_engine* e, long long* fallbacks, int* hold);
+
+/* Test support (like md_check_lists): conditions that a run does not meet by itself.
+ * MD_TEST_LATE_WORKGROUP: the next `value` runs of two steps or more that the
+ * persistent kernel would place on one XCD are launched without their last
+ * workgroup, so the others' first (bounded) wait ends and the run is replayed. */
+#define MD_TEST_LATE_WORKGROUP 1
+int md_test_control(md_engine* e, int what, int value);
 
 /* Kernel timing with HIP events recorded on the engine's stream around every
  * launch of the pair/step kernel during md_run (the persistent kernel, which

@@ -51,8 +51,8 @@ extern "C" hipError_t md_launch_copies(int npair, const void* const* src, void* 
 extern "C" hipError_t md_launch_check_lists(const BuildArgs& a, int row_g, int* bad, hipStream_t st);
 extern "C" hipError_t md_launch_state_sums(const float4* vel, const float4* force, const int* ids, int nslot, double* out,
                                            hipStream_t st);
-extern "C" hipError_t md_launch_persist(const PersistArgs& a, int lanes, size_t shmem, hipStream_t st, hipEvent_t ev0,
-                                        hipEvent_t ev1);
+extern "C" hipError_t md_launch_persist(const PersistArgs& a, int lanes, int nwg, size_t shmem, hipStream_t st,
+                                        hipEvent_t ev0, hipEvent_t ev1);
 extern "C" hipError_t md_launch_settle(const SettleArgs& a, hipStream_t st);
 extern "C" int md_launch_pme(const PmeArgs& a, const PmeFftArgs* f, hipfftHandle r2c, hipfftHandle c2r, int energy,
                              hipStream_t st);
@@ -277,8 +277,12 @@ struct md_engine {
     int pk_req = 0;                // list capacity the caller set (entries per atom): bounds the lane rows
     long long pk_runs = 0, pk_replays = 0;   // runs on the persistent kernel, replays after a row overflow
     size_t lds_max = 65536;        // LDS per workgroup on this device
-    bool pk_placed = true;         // persistent kernel: all workgroups on XCD pk_xcd while they fit
-    int pk_xcd = 0;
+    int pk_xcd = 0;                // persistent kernel: all workgroups on this XCD while they fit
+    int pk_hold = 0;               // runs left on any CU before the XCD is tried again
+    int pk_back = kPkBack;         // the next hold
+    static constexpr int kPkBack = 16;
+    long long pk_fallbacks = 0;    // runs replayed on any CU because the XCD was taken
+    int test_late = 0;             // md_test_control
     DBuf<uint64_t> pk_xch;         // published positions and sums (persistent kernel)
     static constexpr double kQueueRatio0 = 1.15;
     double queue_ratio = kQueueRatio0;   // launched / completed steps, learned per launch configuration
@@ -1255,6 +1259,8 @@ int md_set_system(md_engine* e, int nrep, const int* natom, const float* box, co
     CHECK(e->ang_list.alloc(4 * (size_t)N));
     CHECK(e->nbond.alloc(N));
     CHECK(e->nang.alloc(N));
+    e->pk_hold = 0;
+    e->pk_back = md_engine::kPkBack;
     e->has_sys = true;
     e->has_state = false;
     e->fm_nframes = 0;
@@ -1562,11 +1568,13 @@ bool persist_eligible(const md_engine* e) {
 bool persist_ok(const md_engine* e) { return e->persist && persist_eligible(e); }
 
 // Threads per workgroup: half of MD_PK_THREADS while the workgroups still fit one XCD
-// (a CU each), which shares the work of a step among twice the CUs.
+// (a CU each), which shares the work of a step among twice the CUs.  By the size alone: the
+// split of the FP64 sums over the workgroups, and so every bit of a run, does not depend on
+// whether the XCD was free.
 int persist_xcd(const md_engine* e) { return std::min(e->ncu / 8, MD_PK_WG); }
 int persist_wgs(const md_engine* e, int nth) { return (e->N + nth / e->lanes - 1) / (nth / e->lanes); }
 int persist_threads(const md_engine* e) {
-    return e->pk_placed && persist_wgs(e, MD_PK_THREADS / 2) <= persist_xcd(e) ? MD_PK_THREADS / 2 : MD_PK_THREADS;
+    return persist_wgs(e, MD_PK_THREADS / 2) <= persist_xcd(e) ? MD_PK_THREADS / 2 : MD_PK_THREADS;
 }
 
 // Dynamic LDS of a launch: staged positions and types (20 B per slot) and the
@@ -1596,7 +1604,7 @@ int persist_cap(const md_engine* e) {
 int run_persist(md_engine* e, int nsteps, int energy_every, bool want_stats, int* use_tiles) {
     *use_tiles = 0;
     const int G = e->lanes;
-    int nth = persist_threads(e), nwg = persist_wgs(e, nth);
+    const int nth = persist_threads(e), nwg = persist_wgs(e, nth);
     if (nwg > MD_PK_WG) {   // (S <= MD_PK_SLOTS and 64 atoms or more per workgroup keep nwg <= 64)
         *use_tiles = 1;
         return MD_OK;
@@ -1618,11 +1626,15 @@ int run_persist(md_engine* e, int nsteps, int energy_every, bool want_stats, int
         a.pub = e->pk_xch.p; a.hint = e->pk_xch.p + 2 * MD_PK_WG * 6; a.xch = e->pk_xch.p + MD_PK_PUB; a.err = e->err.p;
         a.stats = want_stats ? e->stats.p : nullptr; a.stat_cap = e->stat_cap;
         a.nslot = e->S; a.natom = e->N; a.nth = nth; a.nwg = nwg;
-        // on one XCD where they fit: workgroups are dealt to the XCDs in turn
-        a.spread = e->pk_placed && nwg <= persist_xcd(e) ? 8 : 1;
-        a.xcd = a.spread > 1 ? e->pk_xcd : 0;
-        a.nsteps = nsteps; a.energy_every = energy_every;
         a.leapfrog = e->in.integrator == MD_LEAPFROG ? 1 : 0;
+        // On one XCD where they fit: workgroups are dealt to the XCDs in turn.  (A leapfrog run of one
+        // step has no exchange of positions, whose short first limit tells early that the XCD is taken.)
+        const bool placed = e->pk_hold == 0 && nwg <= persist_xcd(e) && (nsteps > 1 || a.leapfrog == 0);
+        a.spread = placed ? 8 : 1;
+        a.xcd = placed ? e->pk_xcd : 0;
+        const bool late = placed && e->test_late > 0 && nsteps > 1 && nwg > 1;
+        e->test_late -= late;
+        a.nsteps = nsteps; a.energy_every = energy_every;
         a.thermostat = e->in.thermostat; a.ntype = e->ff.ntype; a.cap_l = cap_l;
         a.dt = e->in.dt; a.tau = e->in.tau; a.rc2 = e->rc2; a.rl2 = e->rl2; a.skin2q = e->skin2q;
         hipEvent_t ev0 = nullptr, ev1 = nullptr;
@@ -1631,18 +1643,17 @@ int run_persist(md_engine* e, int nsteps, int energy_every, bool want_stats, int
             ev1 = ev_get(e, 3);
             if (!ev0 || !ev1) return fail(MD_E_HIP, "hipEventCreate failed");
         }
-        HIPCHECK(md_launch_persist(a, G, persist_lds(e, cap_l), e->st, ev0, ev1));
+        HIPCHECK(md_launch_persist(a, G, late ? nwg - 1 : nwg, persist_lds(e, cap_l), e->st, ev0, ev1));
         // the tile path's lists were built for earlier positions: stale after a run without errors
         HIPCHECK(md_launch_force_trip(e->rst.p, e->gate.p, e->R, 1, nullptr, 0, e->err.p, &e->report->err, e->st));
         HIPCHECK(hipStreamSynchronize(e->st));
         const int err = e->report->err;
-        if ((err & MD_PK_ERR_WAIT) && a.spread > 1) {   // the XCD is taken: replay on any CU from now on
+        if ((err & MD_PK_ERR_WAIT) && placed) {   // the XCD is taken: replay on any CU, and the next runs there too
             CHECK(run_rollback(e));
             HIPCHECK(hipStreamSynchronize(e->st));
-            e->pk_placed = false;
-            nth = persist_threads(e);
-            nwg = persist_wgs(e, nth);
-            e->pk_replays++;
+            e->pk_hold = e->pk_back;   // 16 runs, twice as many each time it is found taken again
+            e->pk_back = std::min(2 * e->pk_back, 4096);
+            e->pk_fallbacks++;
             continue;
         }
         if (err & MD_PK_ERR_WAIT) return fail(MD_E_HIP, "persistent kernel: a wait for another workgroup timed out");
@@ -1661,6 +1672,8 @@ int run_persist(md_engine* e, int nsteps, int energy_every, bool want_stats, int
             e->t_step_ms += ms;
             e->n_step += nsteps;
         }
+        if (placed) e->pk_back = md_engine::kPkBack;
+        else if (e->pk_hold > 0) e->pk_hold--;
         e->pk_runs++;
         break;
     }
@@ -1926,6 +1939,8 @@ int md_set_launch(md_engine* e, const md_launch_config* c) {
         e->pk_cap = 0;
     }
     e->persist = c->persist;
+    e->pk_hold = 0;
+    e->pk_back = md_engine::kPkBack;
     e->queue_ratio = md_engine::kQueueRatio0;   // what a step costs in launches depends on the configuration
     e->drop_graphs();
     if (c->cell_div != e->cell_div) {
@@ -1955,6 +1970,22 @@ int md_get_launch(md_engine* e, md_launch_config* c) {
     c->fm_fused = e->fm_fused;
     c->persist = e->persist;
     return MD_OK;
+}
+
+int md_persist_placement(md_engine* e, long long* fallbacks, int* hold) {
+    if (!e) return fail(MD_E_INVALID, "null engine");
+    if (fallbacks) *fallbacks = e->pk_fallbacks;
+    if (hold) *hold = e->pk_hold;
+    return MD_OK;
+}
+
+int md_test_control(md_engine* e, int what, int value) {
+    if (!e) return fail(MD_E_INVALID, "null engine");
+    if (what == MD_TEST_LATE_WORKGROUP && value >= 0) {
+        e->test_late = value;
+        return MD_OK;
+    }
+    return fail(MD_E_INVALID, "unknown test control %d = %d", what, value);
 }
 
 int md_persist_info(md_engine* e, long long* runs, long long* replays, int* row_len) {

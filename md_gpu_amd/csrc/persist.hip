@@ -39,8 +39,8 @@
 // Bound by that latency (about 1.8 of 3.3 us a step at 864 atoms) and the walk's VALU
 // work on few CUs.  While they fit, the workgroups are placed on one XCD (the others are
 // launched for every one that works and leave: workgroups are dealt to the XCDs in turn;
-// engines take the XCDs in turn, and one that finds its XCD taken goes back to 1024 threads
-// on any CU)
+// engines take the XCDs in turn, and one that finds its XCD taken replays the run on any CU
+// and tries the XCD again after some runs)
 // and have 512 threads, twice as many CUs.  100 steps with a download, 864 atoms: 497
 // us with a grid barrier of release and acquire fences per step, 447 with agent-scope
 // words instead on one XCD, 428 with 512 threads, 377 without the barrier; 256 atoms, 10
@@ -486,9 +486,10 @@ __global__ __launch_bounds__(NTH) void k_persist(const PersistArgs a) {
     }
 }
 
-extern "C" hipError_t md_launch_persist(const PersistArgs& a, int lanes, size_t shmem, hipStream_t st, hipEvent_t ev0,
-                                        hipEvent_t ev1) {
-    const dim3 grid(a.nwg * a.spread), block(a.nth);
+// nwg: working workgroups launched (a.nwg, or fewer in a test of the bounded waits)
+extern "C" hipError_t md_launch_persist(const PersistArgs& a, int lanes, int nwg, size_t shmem, hipStream_t st,
+                                        hipEvent_t ev0, hipEvent_t ev1) {
+    const dim3 grid(nwg * a.spread), block(a.nth);
     const bool nt1 = a.ntype == 1;
     hipError_t rc = hipSuccess;
     auto go = [&](auto kern) {

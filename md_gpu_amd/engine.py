@@ -23,6 +23,9 @@ ERRORS = {-1: "invalid argument", -2: "HIP error", -3: "call out of order", -4: 
           -5: "unstable trajectory"}
 
 
+TEST_LATE_WORKGROUP = 1   # md_test_control
+
+
 class LaunchConfig(C.Structure):
     """md_launch_config (md_api.h)."""
     _fields_ = [("lanes", C.c_int), ("grid", C.c_int), ("cell_div", C.c_int), ("check_every", C.c_int),
@@ -91,6 +94,7 @@ def lib():
             "md_autotune": ([P, C.c_int, P], C.c_int), "md_timing_enable": ([P, C.c_int], C.c_int),
             "md_timing_get": ([P, P, P, P, P], C.c_int), "md_copy_bench": ([P, C.c_longlong, C.c_int, P], C.c_int),
             "md_rebuild_bench": ([P, C.c_int, P], C.c_int), "md_persist_info": ([P, P, P, P], C.c_int),
+            "md_persist_placement": ([P, P, P], C.c_int), "md_test_control": ([P, C.c_int, C.c_int], C.c_int),
             "md_fm_set_frames": ([P, C.c_int, P, P], C.c_int),
             "md_fm_loss_grad": ([P, P, P, C.c_float, P, P, P, P], C.c_int),
             "md_fm_loss_grad_noalloc": ([P, P, P, C.c_float, P, P, P, P], C.c_int),
@@ -110,7 +114,7 @@ def exported_symbols() -> List[str]:
             "md_get_launch", "md_autotune",
             "md_timing_enable", "md_timing_get", "md_copy_bench", "md_rebuild_bench", "md_fm_set_frames", "md_fm_loss_grad",
             "md_set_list_capacity", "md_fm_loss_grad_noalloc", "md_get_box", "md_get_sums", "md_persist_info",
-            "md_set_rigid", "md_set_pme"]
+            "md_persist_placement", "md_test_control", "md_set_rigid", "md_set_pme"]
 
 
 def _check(rc: int):
@@ -324,6 +328,17 @@ class Engine:
         runs = C.c_longlong(); rep = C.c_longlong(); rl = C.c_int()
         _check(lib().md_persist_info(self._h, C.byref(runs), C.byref(rep), C.byref(rl)))
         return dict(runs=runs.value, replays=rep.value, row_len=rl.value)
+
+    def persist_placement(self):
+        """Runs of the persistent kernel that found their XCD taken and were replayed on any CU,
+        and the runs left before it is tried again (md_persist_placement)."""
+        n = C.c_longlong(); hold = C.c_int()
+        _check(lib().md_persist_placement(self._h, C.byref(n), C.byref(hold)))
+        return dict(fallbacks=n.value, hold=hold.value)
+
+    def test_control(self, what: int, value: int):
+        """Test support (md_test_control, MD_TEST_*)."""
+        _check(lib().md_test_control(self._h, int(what), int(value)))
 
     def timing(self, enable: bool):
         _check(lib().md_timing_enable(self._h, 1 if enable else 0))

@@ -288,3 +288,67 @@ def test_persist_one_step_runs(E, thermostat, stats):
         d -= s.box * np.rint(d / s.box)
         assert np.abs(d).max() < 2e-5
         assert rel_rms(v1, v0) < 1e-5 and rel_rms(f1, f0) < 1e-5
+
+
+def sampled(s):
+    """The bits of a few runs of an engine: statistics and the frame they end in."""
+    def bits(e, runs):
+        out = [e.run(n, energy_every=3) for n in runs]
+        return [x.tobytes() for x in out] + [x.tobytes() for x in e.download()]
+    return bits
+
+
+@pytest.mark.parametrize("integrator,thermostat", [("vverlet", "none"), ("leapfrog", "berendsen")])
+def test_persist_falls_back_when_its_xcd_is_taken(E, integrator, thermostat):
+    """A placed run that misses a workgroup ends by its bounded wait and is replayed on any CU with
+    the same bits (frames, kinetic energies, temperatures); the XCD is tried again after 16 runs,
+    after 32 when it is found taken once more, and at once after a placed run or set_launch."""
+    s = dataclasses.replace(perturbed(S.argon(), 0.1), integrator=integrator, thermostat=thermostat, tau=100.0, T0=120.0)
+    say("persist fallback", s.n, integrator, thermostat)
+    bits = sampled(s)
+    runs = [20, 1, 30]
+    e = persist_engine(E, s, 16)
+    want = bits(e, runs)
+    assert e.persist_placement() == dict(fallbacks=0, hold=0)
+    e.close()
+    e = persist_engine(E, s, 16)
+    e.test_control(E.TEST_LATE_WORKGROUP, 1)
+    assert bits(e, runs) == want
+    assert e.persist_placement() == dict(fallbacks=1, hold=13)
+    assert e.persist_info()["runs"] == 3 and e.persist_info()["replays"] == 0
+    for _ in range(13):
+        e.run(1, stats=False)
+    e.test_control(E.TEST_LATE_WORKGROUP, 1)
+    e.run(2, stats=False)
+    assert e.persist_placement() == dict(fallbacks=2, hold=31)
+    e.set_launch(persist=1)
+    assert e.persist_placement()["hold"] == 0
+    e.run(2, stats=False)
+    assert e.persist_placement() == dict(fallbacks=2, hold=0)
+    e.close()
+
+
+def test_persist_engines_side_by_side_record_the_same(E):
+    """Engines side by side record the statistics of one alone, whatever their placement."""
+    import threading
+    s = dataclasses.replace(perturbed(S.argon(), 0.1), integrator="leapfrog", thermostat="berendsen", tau=100.0, T0=120.0)
+    say("persist side by side, berendsen")
+    bits = sampled(s)
+
+    def work(out, k):
+        e = persist_engine(E, s, 16)
+        if k % 2:
+            e.test_control(E.TEST_LATE_WORKGROUP, 1)
+        out[k] = bits(e, [50] * 6)
+        e.close()
+
+    out = {}
+    work(out, 0)
+    threads = [threading.Thread(target=work, args=(out, k)) for k in range(1, 5)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert len(out) == 5
+    for k in out:
+        assert out[k] == out[0], k
