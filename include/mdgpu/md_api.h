@@ -251,9 +251,9 @@ int md_autotune(md_engine* e, int nsteps, double* best_ms_per_step);
  * length (the run restarts from its first step with rows twice as long), and
  * the current row length per lane. */
 int md_persist_info(md_engine* e, long long* runs, long long* replays, int* row_len);
-/* Where its workgroups run: on one XCD while they fit.  fallbacks: runs that found
+/* Where its workgroups run: on one XCD while four of its CUs stay free.  fallbacks: runs that found
  * the XCD taken (2 ms) and were replayed on any CU, with the same bits; hold:
- * runs left before the XCD is tried again (md_set_launch and md_set_system try
+ * runs left before the next XCD is tried (md_set_launch and md_set_system try
  * it at once).  Either pointer may be NULL. */
 int md_persist_placement(md_engine* e, long long* fallbacks, int* hold);
 

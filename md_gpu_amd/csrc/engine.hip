@@ -278,7 +278,7 @@ struct md_engine {
     long long pk_runs = 0, pk_replays = 0;   // runs on the persistent kernel, replays after a row overflow
     size_t lds_max = 65536;        // LDS per workgroup on this device
     int pk_xcd = 0;                // persistent kernel: all workgroups on this XCD while they fit
-    int pk_hold = 0;               // runs left on any CU before the XCD is tried again
+    int pk_hold = 0;               // runs left on any CU before an XCD is tried again
     int pk_back = kPkBack;         // the next hold
     static constexpr int kPkBack = 16;
     long long pk_fallbacks = 0;    // runs replayed on any CU because the XCD was taken
@@ -1068,6 +1068,8 @@ int md_create(md_engine** out, int device) {
         md_destroy(e);
         return fail(MD_E_HIP, "hipHostMalloc failed");
     }
+    // the engines of a process take the XCDs in turn; one that finds its XCD taken (by another
+    // process's, say) moves on to the next
     static std::atomic<unsigned> engines{0};
     e->pk_xcd = (int)(engines++ % 8);
     if (!ev_get(e, 1)) {   // events 0 and 1 exist from here on: timing allocates no events later
@@ -1627,9 +1629,14 @@ int run_persist(md_engine* e, int nsteps, int energy_every, bool want_stats, int
         a.stats = want_stats ? e->stats.p : nullptr; a.stat_cap = e->stat_cap;
         a.nslot = e->S; a.natom = e->N; a.nth = nth; a.nwg = nwg;
         a.leapfrog = e->in.integrator == MD_LEAPFROG ? 1 : 0;
-        // On one XCD where they fit: workgroups are dealt to the XCDs in turn.  (A leapfrog run of one
-        // step has no exchange of positions, whose short first limit tells early that the XCD is taken.)
-        const bool placed = e->pk_hold == 0 && nwg <= persist_xcd(e) && (nsteps > 1 || a.leapfrog == 0);
+        // On one XCD while at least four of its CUs stay free: workgroups are dealt to the XCDs in
+        // turn, and a run is over when those that only mark the place have had a CU too, so an
+        // engine that filled its XCD held back every other engine's runs until its own ended.  (Nor
+        // does a full XCD pay: 100 steps of 2,048 atoms with 16 lanes 487 us spread, 515 on one; of
+        // 4,000 with 8 lanes 768 and 838, with 4 lanes 929 and 944; of 2,048 with 8 lanes 532 and 519.)
+        // A leapfrog run of one step has no exchange of positions, whose short first limit tells
+        // early that the XCD is taken.
+        const bool placed = e->pk_hold == 0 && nwg <= persist_xcd(e) - 4 && (nsteps > 1 || a.leapfrog == 0);
         a.spread = placed ? 8 : 1;
         a.xcd = placed ? e->pk_xcd : 0;
         const bool late = placed && e->test_late > 0 && nsteps > 1 && nwg > 1;
@@ -1653,6 +1660,7 @@ int run_persist(md_engine* e, int nsteps, int energy_every, bool want_stats, int
             HIPCHECK(hipStreamSynchronize(e->st));
             e->pk_hold = e->pk_back;   // 16 runs, twice as many each time it is found taken again
             e->pk_back = std::min(2 * e->pk_back, 4096);
+            e->pk_xcd = (e->pk_xcd + 1) % 8;
             e->pk_fallbacks++;
             continue;
         }

@@ -37,10 +37,10 @@
 // the host reports the error.
 //
 // Bound by that latency (about 1.8 of 3.3 us a step at 864 atoms) and the walk's VALU
-// work on few CUs.  While they fit, the workgroups are placed on one XCD (the others are
+// work on few CUs.  While four of its CUs stay free, the workgroups are placed on one XCD (the others are
 // launched for every one that works and leave: workgroups are dealt to the XCDs in turn;
 // engines take the XCDs in turn, and one that finds its XCD taken replays the run on any CU
-// and tries the XCD again after some runs)
+// and tries the next XCD after some runs)
 // and have 512 threads, twice as many CUs.  100 steps with a download, 864 atoms: 497
 // us with a grid barrier of release and acquire fences per step, 447 with agent-scope
 // words instead on one XCD, 428 with 512 threads, 377 without the barrier; 256 atoms, 10

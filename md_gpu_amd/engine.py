@@ -331,7 +331,7 @@ class Engine:
 
     def persist_placement(self):
         """Runs of the persistent kernel that found their XCD taken and were replayed on any CU,
-        and the runs left before it is tried again (md_persist_placement)."""
+        and the runs left before the next XCD is tried (md_persist_placement)."""
         n = C.c_longlong(); hold = C.c_int()
         _check(lib().md_persist_placement(self._h, C.byref(n), C.byref(hold)))
         return dict(fallbacks=n.value, hold=hold.value)

@@ -352,3 +352,35 @@ def test_persist_engines_side_by_side_record_the_same(E):
     assert len(out) == 5
     for k in out:
         assert out[k] == out[0], k
+
+
+def test_persist_long_run_does_not_hold_back_others(E):
+    """Short runs of other engines end while an engine with as many workgroups as an XCD has CUs is
+    in the middle of a long run (three engines, since two streams may share a hardware queue)."""
+    import threading
+    import time
+    s = S.argon(ncell=7).copy()   # 1,024 of its 1,372 atoms: 32 workgroups of 512 threads with 16 lanes
+    s.pos, s.vel, s.type, s.charge = s.pos[:1024], s.vel[:1024], s.type[:1024], s.charge[:1024]
+    say("persist long run beside short ones")
+    big = persist_engine(E, s, 16)
+    small = [persist_engine(E, perturbed(S.argon(ncell=4), 0.1), 16) for _ in range(3)]
+    for e in [big] + small:
+        e.run(10, stats=False)
+    ended = {}
+
+    def work(k, e, n):
+        e.run(n, stats=False)
+        ended[k] = time.perf_counter()
+
+    threads = [threading.Thread(target=work, args=("big", big, 40000))]
+    threads[0].start()
+    time.sleep(0.02)
+    assert "big" not in ended
+    for k, e in enumerate(small):
+        threads.append(threading.Thread(target=work, args=(k, e, 100)))
+        threads[-1].start()
+    for t in threads:
+        t.join()
+    assert min(ended[k] for k in range(3)) < ended["big"] - 0.02
+    for e in [big] + small:
+        e.close()
