@@ -1051,9 +1051,10 @@ int md_create(md_engine** out, int device) {
         lds = prop.sharedMemPerBlock;
     }
     e->lds_max = lds;
-    // the step and force-matching kernels hold the staged set and the dummy
-    // (16 bytes each) next to at most 8 KB of static LDS
-    e->jcap_max = (int)std::min<size_t>(MD_JMAX, (lds - 8192) / 16 - 1) / 64 * 64;
+    // the step and force-matching kernels hold the staged set and the dummy (16 bytes each)
+    // and at most 16 KB more: 7.5 KB of tables and sums and 8 KB of bonded terms in the step
+    // kernel, 9.7 KB of tables and sums in force matching
+    e->jcap_max = (int)std::min<size_t>(MD_JMAX, (lds - 16384) / 16 - 1) / 64 * 64;
     if (hipStreamCreateWithFlags(&e->st, hipStreamNonBlocking) != hipSuccess) {
         delete e;
         return fail(MD_E_HIP, "hipStreamCreate failed");

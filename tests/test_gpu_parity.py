@@ -562,3 +562,30 @@ def test_sort_edges(E, orc, n, cell_div, L):
         assert np.abs(F[off:off + s.n] - Fo).max() <= 1e-5 * max(np.abs(Fo).max(), 1.0)
         off += s.n
     e.close()
+
+
+@pytest.mark.parametrize("lanes", [4, 8, 16])
+def test_bonded_largest_sets(E, orc, lanes):
+    """Flexible water whose tile sets have the largest capacity (4,032 entries: with the bonded
+    terms 71 KB of LDS beside the tables): forces, energies and a few steps, through captured
+    segments and with direct launches."""
+    s = perturbed(S.water(nmol=1000), 0.05)
+    s = dataclasses.replace(s, ff=dataclasses.replace(s.ff, rc=13.0))
+    say("bonded largest sets", s.n, "lanes", lanes)
+    e = E.Engine.from_system(s)
+    e.set_launch(lanes=lanes)
+    so = s.copy()
+    so.pos = e.download()[0]
+    F, En, W = e.compute_forces()
+    Fo, Eo, Wo = orc.forces(so)
+    assert rel_rms(F, Fo) < FORCE_TOL
+    assert np.all(np.abs(En[0] - Eo) <= 1e-5 * max(np.abs(Eo).sum(), 1.0))
+    out = []
+    for submit in (0, 1):
+        e.set_launch(submit=submit)
+        e.upload(s.pos, s.vel)
+        e.run(4, energy_every=2)
+        out.append(e.download())
+    for a, b in zip(*out):
+        assert np.isfinite(a).all() and np.array_equal(a, b)
+    e.close()
