@@ -219,8 +219,9 @@ typedef struct md_launch_config {
     int grid;          /* unused (0): the step kernel runs one workgroup per 64-atom tile */
     int cell_div;      /* cell edge >= r_list / cell_div, 1..3 */
     int check_every;   /* steps queued between two (device-gated) list-rebuild chains */
-    int build_lanes;   /* 4 or 8; no effect (the list build runs 8 wavefronts per 64-atom
-                          tile; kept so that callers' settings stay valid) */
+    int build_lanes;   /* 4 or 8; no effect (the list build runs 16 wavefronts per 64-atom tile
+                          while every tile has a CU of its own, else 8; the same lists; kept so
+                          that callers' settings stay valid) */
     int submit;        /* 0: replayed HIP graph segments, 1: direct kernel launches */
     int refresh;       /* 1: also rebuild a list after check_every steps, ahead of the skin trip */
     int build_kernel;  /* 0: the tile neighbor-set build (the only list build) */
@@ -260,8 +261,11 @@ int md_persist_placement(md_engine* e, long long* fallbacks, int* hold);
 /* Test support (like md_check_lists): conditions that a run does not meet by itself.
  * MD_TEST_LATE_WORKGROUP: the next `value` runs of two steps or more that the
  * persistent kernel would place on one XCD are launched without their last
- * workgroup, so the others' first (bounded) wait ends and the run is replayed. */
+ * workgroup, so the others' first (bounded) wait ends and the run is replayed.
+ * MD_TEST_BUILD_WAVEFRONTS: list builds run 8 or 16 wavefronts per tile whatever
+ * the number of tiles (0: by the engine's rule); the lists are rebuilt. */
 #define MD_TEST_LATE_WORKGROUP 1
+#define MD_TEST_BUILD_WAVEFRONTS 2
 int md_test_control(md_engine* e, int what, int value);
 
 /* Kernel timing with HIP events recorded on the engine's stream around every

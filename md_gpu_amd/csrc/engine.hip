@@ -282,7 +282,7 @@ struct md_engine {
     int pk_back = kPkBack;         // the next hold
     static constexpr int kPkBack = 16;
     long long pk_fallbacks = 0;    // runs replayed on any CU because the XCD was taken
-    int test_late = 0;             // md_test_control
+    int test_late = 0, test_build = 0;   // md_test_control
     DBuf<uint64_t> pk_xch;         // published positions and sums (persistent kernel)
     static constexpr double kQueueRatio0 = 1.15;
     double queue_ratio = kQueueRatio0;   // launched / completed steps, learned per launch configuration
@@ -592,7 +592,7 @@ BuildArgs build_args(md_engine* e) {
     b.key = e->key.p; b.rank = e->rank.p; b.tmp = e->tmp.p; b.tmpid = e->tmpid.p;
     b.cell_count = e->cell_count.p; b.cell_start = e->cell_start.p; b.cell_rank = e->cell_rank.p;
     b.slot_of = e->slot_of.p; b.nl16 = e->nl16.p; b.ncount = e->ncount.p; b.rperm = e->rperm.p; b.ljfree = ljfree(e);
-    b.wide = e->ntiles() <= e->ncu ? 1 : 0;
+    b.wide = e->test_build ? e->test_build == 16 : e->ntiles() <= e->ncu;
     b.sort_lds = e->sort_lds; b.sort_na = e->sort_na;
     b.jset = e->jset.p; b.jcount = e->jcount.p;
     b.tilemax = e->tmax.p; b.jmax = e->tmax.p + e->ntiles();
@@ -1992,6 +1992,14 @@ int md_test_control(md_engine* e, int what, int value) {
     if (!e) return fail(MD_E_INVALID, "null engine");
     if (what == MD_TEST_LATE_WORKGROUP && value >= 0) {
         e->test_late = value;
+        return MD_OK;
+    }
+    if (what == MD_TEST_BUILD_WAVEFRONTS && (value == 0 || value == 8 || value == 16)) {
+        HIPCHECK(hipSetDevice(e->dev));
+        HIPCHECK(hipStreamSynchronize(e->st));
+        e->test_build = value;
+        e->drop_graphs();
+        if (e->has_sys && e->has_state) CHECK(full_rebuild(e));
         return MD_OK;
     }
     return fail(MD_E_INVALID, "unknown test control %d = %d", what, value);

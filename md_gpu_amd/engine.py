@@ -23,7 +23,7 @@ ERRORS = {-1: "invalid argument", -2: "HIP error", -3: "call out of order", -4: 
           -5: "unstable trajectory"}
 
 
-TEST_LATE_WORKGROUP = 1   # md_test_control
+TEST_LATE_WORKGROUP, TEST_BUILD_WAVEFRONTS = 1, 2   # md_test_control
 
 
 class LaunchConfig(C.Structure):

@@ -589,3 +589,45 @@ def test_bonded_largest_sets(E, orc, lanes):
     for a, b in zip(*out):
         assert np.isfinite(a).all() and np.array_equal(a, b)
     e.close()
+
+
+BUILDS = {"argon864": lambda: CASES["argon864"], "nacl4096_wolf": lambda: CASES["nacl4096_wolf"],
+          "water1536": lambda: CASES["water1536"], "atoms72": lambda: EDGES["atoms72"],
+          "dense1728": lambda: EDGES["dense1728"],
+          "arxe24": lambda: S.arxe_replicas(nrep=24, seed=3, nmin=256, nmax=1500),
+          "water17001": lambda: perturbed(S.water(nmol=5667), 0.05)}
+
+
+@pytest.mark.parametrize("name", list(BUILDS))
+def test_build_widths_same_lists(E, name):
+    """The tile build on 8 and on 16 wavefronts per tile writes the same sets and rows (candidate
+    order, not scheduling, fixes them): identical neighbor arrays and forces, and identical
+    100-step trajectories through in-run rebuilds; fewer tiles than CUs and more."""
+    s = BUILDS[name]()
+    say("build widths", name)
+    out = []
+    for nw in (8, 16):
+        e = E.Engine.from_system(s)
+        e.set_launch(persist=0)
+        e.test_control(E.TEST_BUILD_WAVEFRONTS, nw)
+        assert all(v == 0 for v in e.check_lists().values())
+        counts, nbrs = e.neighbors()
+        F, En, W = e.compute_forces()
+        st = e.run(100, energy_every=10) if name != "dense1728" else np.zeros(0)
+        out.append([x.tobytes() for x in (counts, nbrs, F, En, W, st, *e.download())] + [e.info()["rebuilds"]])
+        e.close()
+    assert out[0] == out[1]
+
+
+def test_build_width_control(E):
+    """Any other width is refused and leaves the engine as it was."""
+    e = E.Engine.from_system(CASES["argon864"])
+    a = e.neighbors()
+    for v in (4, -1, 32):
+        with pytest.raises(E.MDError):
+            e.test_control(E.TEST_BUILD_WAVEFRONTS, v)
+    with pytest.raises(E.MDError):
+        e.test_control(99, 1)
+    for x, y in zip(a, e.neighbors()):
+        assert np.array_equal(x, y)
+    e.close()
