@@ -134,6 +134,27 @@ def test_forces_brick_edges(E, orc, grid, order, cell_div):
     assert rel_rms(F, Fo) < FORCE_TOL
 
 
+# the bricks are 16 x 8 x 16 points: exact multiples, one point over on each axis and on all, one short
+@pytest.mark.parametrize("cell_div", [1, 3])
+@pytest.mark.parametrize("grid,order", [((32, 16, 32), 4), ((16, 8, 16), 8), ((33, 16, 32), 4), ((17, 8, 16), 6),
+                                        ((32, 17, 32), 6), ((32, 16, 33), 8), ((33, 17, 33), 4), ((31, 15, 31), 6)])
+def test_forces_brick_multiples(E, orc, grid, order, cell_div):
+    """Grids of whole bricks and of bricks with one point over or short on each axis (a brick of
+    one plane, whose atoms all reach it through the spline's support), after steps that move the
+    atoms away from their cells."""
+    s = nacl_pme(grid=grid, order=order)
+    say("pme forces brick multiples", s.pme, "cell_div", cell_div)
+    e = E.Engine.from_system(s)
+    e.set_launch(cell_div=cell_div)
+    e.run(5, stats=False)
+    so = s.copy()
+    so.pos = e.download()[0]
+    F, _, _ = e.compute_forces()
+    Fo, _, _ = orc.forces(so)
+    e.close()
+    assert rel_rms(F, Fo) < FORCE_TOL
+
+
 def test_forces_large_charges(E, orc):
     """Charges beyond 2^18 e take the spread's full-range fixed point: the forces of NaCl with
     charges of 3e5 e (the pair law scaled back by qfac) equal the oracle's."""
