@@ -613,9 +613,11 @@ StepArgs step_args(md_engine* e, int mode, int energy_every) {
     a.tile_rep = e->tile_rep.p; a.rep = e->rep.p; a.st = e->rst.p; a.gate = e->gate.p; a.th = e->th.p; a.part = e->part.p;
     a.lst = e->lst.p; a.lagmode = 0; a.lag = 0; a.par = 0; a.open = 0;
     // Cleared for deferred-finalize blocks (every tile takes part).  A single system's tiles look
-    // first once they no longer start all together (an idle launch of 196,608 water atoms
-    // 15.7 us without, 40 steps of them 7.09 -> 6.82 ms); below, the look only delays them.
-    a.prefilter = e->R > 1 || e->ntiles() >= 8 * e->ncu ? 1 : 0;
+    // first from a tile per CU on, where an idle launch's loads cost more than the look: 40 steps of
+    // flexible water 2,319 -> 2,290 us (516 tiles), 2,805 -> 2,742 (1,024), 4,709 -> 4,552 (2,048),
+    // 6,542 -> 6,354 (3,072), 32,768 ions with smooth PME 3,722 -> 3,700, argon of 256 to 1,688 tiles the
+    // same; below, argon of 8 to 63 tiles would take 0.8 % longer (631 -> 635 us), ions and water the same.
+    a.prefilter = e->R > 1 || e->ntiles() >= e->ncu ? 1 : 0;
     a.vvfused = vv_fused(e) ? 1 : 0;
     a.err = e->err.p; a.stats = e->stats.p; a.stat_cap = e->stat_cap;
     a.ljtab = e->ljtab.p;
