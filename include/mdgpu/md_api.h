@@ -141,7 +141,8 @@ int md_set_rigid(md_engine* e, int nmol, const int* mol, float d_oh, float d_hh)
  * splitting parameter beta = the force field's alpha.  The reference reads kmax
  * for it and computes no reciprocal part; its GROMACS PME (src/pme.c) is vendored,
  * not built.  With PME on, each step adds the reciprocal forces (order-p
- * B-splines on a grid[0] x grid[1] x grid[2] mesh, FFTs by hipFFT), removes
+ * B-splines on a grid[0] x grid[1] x grid[2] mesh; hipFFT transforms grids beyond
+ * the engine's own kernels), removes
  * -qfac qi qj erf(beta r)/r for every excluded pair, and adds the self and
  * neutralizing-background terms to the Coulomb energy and the virial.
  * order: 4, 6 or 8 (0 turns PME off); grid: points per box edge, >= order, at

@@ -914,7 +914,7 @@ Snapshot snapshot_arrays(md_engine* e) {
     return s;
 }
 
-// Queue the start of a run: snapshot, cleared maxima, error word and barrier flags, targets.
+// Queue the start of a run: snapshot, cleared maxima, error word and exchange buffer, targets.
 // nsteps < 0: the persistent kernel, which counts its steps itself.
 int run_begin(md_engine* e, long long nsteps) {
     const Snapshot s = snapshot_arrays(e);

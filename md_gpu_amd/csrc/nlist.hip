@@ -404,11 +404,11 @@ __global__ __launch_bounds__(SORT_NT) void k_nl_sort(BuildArgs a) {
 //     64 entries at a time to memory in one contiguous store.
 // So set and rows follow candidate order and do not depend on scheduling.
 //
-// Bound by VALU issue (72 % busy; 7 instructions per atom and 64 candidates for the test, 7
-// for the append, 4 to keep the mask in between), the rest barriers and load latency; at
-// 32,768 ions two tiles per CU leave it latency-bound.  A full build (us): 196,608 water
-// atoms 397 (660 before), 32,768 ions 77 (89), 512 Ar-Xe replicas 912 (1,065), 64 replicas
-// 151 (211).  Before, every wavefront tested every candidate of the tile (a barrier per 64
+// Bound by VALU issue (75 % busy with water, 78 % with Ar-Xe replicas; 7 instructions per
+// atom and 64 candidates for the test, 7 for the append, 4 to keep the mask in between),
+// the rest barriers and load latency; at 32,768 ions two tiles per CU leave it latency-bound
+// (40 %).  A full build (us): 196,608 water atoms 397 (660 before), 32,768 ions 77 (89), 512
+// Ar-Xe replicas 912 (1,065), 64 replicas 151 (211).  Before, every wavefront tested every candidate of the tile (a barrier per 64
 // of them), tested self and exclusions per atom and stored hits to memory 2 bytes at a
 // time; a group's own candidates are under half of the tile's.  Groups by bounding sphere
 // instead of box: 480 us (water).  80 registers keep three workgroups per CU (unbounded,

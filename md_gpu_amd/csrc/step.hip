@@ -22,7 +22,8 @@
 // moves; the tile's last wavefront (the shortest rows) then integrates all 64
 // atoms, a lane each, and with bonded terms it computes the bonds before its
 // rows, the wavefront before it the angles: the kernel is bound by VALU issue
-// (196,608 water atoms: 100 % busy, Ar-Xe replicas 84 %), and with 64 / G active
+// (95 to 98 % busy with 196,608 water atoms, 83 % with 512 Ar-Xe replicas, 46 % with
+// 32,768 ions, whose 512 tiles start together), and with 64 / G active
 // lanes these ends cost every wavefront as much as full ones (40 steps of water
 // 7.94 -> 7.63 ms with them on one wavefront, 60 steps of 512 Ar-Xe replicas
 // 15.3 -> 14.8 ms, the same bits).  KE / energies / virial and the skin-check flag

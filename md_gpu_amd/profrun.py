@@ -7,12 +7,14 @@ grid: 96^3 and 128^3), the 512 batched Ar-Xe replicas, force matching (NaCl 4,09
 calibration of the HBM byte counters).
 
     python -m md_gpu_amd.profrun [--system nacl|argon|water|arxe|nacl_pme|water_rigid_pme|fm|copy]
-                                 [--launch k=v,...] [--steps N] [--timed]
+                                 [--launch k=v,...] [--steps N] [--timed] [--rebuilds N]
 
 Counter collection serialises every dispatch, so this driver keeps the run
 short, needs no autotuning and reports (rather than raises) a failed run.
 With --timed every step is launched directly with HIP events around it (the
-same timing path bench.py uses for kernel durations).
+same timing path bench.py uses for kernel durations).  With --rebuilds N the run is
+followed by N full list builds (every launch of the build kernels a working one;
+--steps 0: no steps before them).
 
 The JSON line ends with a checksum of the final state (FP64 sums of the
 downloaded positions and velocities, and their hex digest) and the device
@@ -38,6 +40,7 @@ def main() -> int:
     ap.add_argument("--steps", type=int, default=60)
     ap.add_argument("--warmup", type=int, default=0)
     ap.add_argument("--timed", action="store_true")
+    ap.add_argument("--rebuilds", type=int, default=0)
     args = ap.parse_args()
     from md_gpu_amd import engine as E, systems as S
     cfg = dict((k, int(v)) for k, v in (kv.split("=") for kv in args.launch.split(",") if kv))
@@ -65,9 +68,11 @@ def main() -> int:
         wall = time.perf_counter() - t0
         out = dict(ok=True, system=args.system, launch=e.get_launch(), steps=args.steps,
                    rebuilds=e.info()["rebuilds"], run_rebuilds=e.info()["rebuilds"] - reb0,
-                   wall_ms_per_step=1e3 * wall / args.steps)
+                   wall_ms_per_step=1e3 * wall / max(args.steps, 1))
         if args.timed:
             out["timing"] = e.timing_get()
+        if args.rebuilds:
+            out["ms_per_rebuild"] = e.rebuild_bench(args.rebuilds)
     except E.MDError as x:
         out = dict(ok=False, error=str(x))
     try:
