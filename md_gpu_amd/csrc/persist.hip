@@ -51,22 +51,20 @@
 #include <type_traits>
 
 #include "md_device.h"
+#include "md_pk_words.h"
 #include "md_reduce.h"
 
 namespace {
 
 constexpr unsigned FL_TRIP = 1u, FL_ROWS = 2u, FL_STOP = 4u;   // flag bits below the step number
 
-// A published word: 32 bits of data and above them the step number << 3 (sums), or 48 bits
-// of data and above them the step number's low 13 bits and the atom's flag bits (positions).
-__device__ __forceinline__ void put(uint64_t* p, uint32_t v, unsigned tag) {
-    __hip_atomic_store(p, (uint64_t)v | ((uint64_t)tag << 32), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+// A published word (md_pk_words.h) is stored and loaded whole.
+__device__ __forceinline__ void put(uint64_t* p, uint32_t v, uint32_t tag) {
+    __hip_atomic_store(p, pk::word(v, tag), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 __device__ __forceinline__ uint64_t get(const uint64_t* p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-__device__ __forceinline__ bool of_step(uint64_t w, unsigned n) { return (unsigned)(w >> 51) == (n & 0x1fffu); }   // position
-__device__ __forceinline__ bool is_step(uint64_t w, unsigned n) { return (unsigned)(w >> 35) == n; }
 
 // The limit of a wait: looked at every 64 tries.
 struct Wait {
@@ -129,9 +127,9 @@ __global__ __launch_bounds__(NTH) void k_persist(const PersistArgs a) {
     // the atom's position, published as step number n (into bank n & 1)
     auto publish = [&](unsigned n, float4 y, unsigned fl) {
         uint64_t* q = a.xch + ((size_t)(n & 1) * a.natom + slot) * 2;
-        const unsigned tag = ((n << 3) | fl) << 16, iy = __float_as_uint(y.y);
-        put(q, __float_as_uint(y.x), tag | (iy >> 16));
-        put(q + 1, __float_as_uint(y.z), tag | (iy & 0xffffu));
+        const unsigned iy = __float_as_uint(y.y);
+        put(q, __float_as_uint(y.x), pk::pos_tag(n, fl, iy >> 16));
+        put(q + 1, __float_as_uint(y.z), pk::pos_tag(n, fl, iy & 0xffffu));
     };
     // every workgroup's sums of step number n (lane w: workgroup w's); false: the wait timed out
     auto sums_of = [&](unsigned n, double& t0, double& t1, double& t2) {
@@ -145,7 +143,7 @@ __global__ __launch_bounds__(NTH) void k_persist(const PersistArgs a) {
 #pragma unroll
                 for (int c = 0; c < 6; c++) w[c] = get(q + c);
 #pragma unroll
-                for (int c = 0; c < 6; c++) all = all && is_step(w[c], n);
+                for (int c = 0; c < 6; c++) all = all && pk::sum_of_step(w[c], n);
                 if (all) break;
                 if (wait.late(MD_PK_TIMEOUT)) {
                     ok = false;
@@ -230,7 +228,7 @@ __global__ __launch_bounds__(NTH) void k_persist(const PersistArgs a) {
                     }
 #pragma unroll
                 for (int u = 0; u < SPT; u++)
-                    if (((miss >> u) & 1u) && of_step(w[u][0], n) && of_step(w[u][1], n)) {
+                    if (((miss >> u) & 1u) && pk::pos_of_step(w[u][0], n) && pk::pos_of_step(w[u][1], n)) {
                         const int q = tid + u * NTH;
                         const unsigned iy = ((unsigned)(w[u][0] >> 32) << 16) | ((unsigned)(w[u][1] >> 32) & 0xffffu);
                         s_pos[q] = make_float4(__uint_as_float((uint32_t)w[u][0]), __uint_as_float(iy),
@@ -431,8 +429,8 @@ __global__ __launch_bounds__(NTH) void k_persist(const PersistArgs a) {
                 const uint64_t d = (uint64_t)__double_as_longlong(t);
                 const unsigned n = (unsigned)(k + 2);
                 uint64_t* q = a.pub + ((size_t)(n & 1) * MD_PK_WG + bid) * 6 + 2 * tid;
-                put(q, (uint32_t)d, n << 3);
-                put(q + 1, (uint32_t)(d >> 32), n << 3);
+                put(q, (uint32_t)d, pk::sum_tag(n));
+                put(q + 1, (uint32_t)(d >> 32), pk::sum_tag(n));
             }
         }
         if (!last) {
