@@ -1,6 +1,8 @@
 // state_out.h -- the state in the caller's atom order, from the device into the caller's
 // (pageable) arrays through an engine's own pinned ring (state_out.hip).
 #pragma once
+#include <mutex>
+
 #include "md_device.h"
 
 struct StateOutArgs {
@@ -15,13 +17,15 @@ struct StateOutArgs {
 };
 
 // Pinned memory of one engine, made by its first download (as much as that needs, at most
-// NS slots of SLOT bytes) and freed with it.
+// NS slots of SLOT bytes) and freed with it.  A download holds it until its arrays are filled:
+// downloads of one engine from several threads take turns.
 struct HostRing {
     static constexpr int NS = 16;
     static constexpr size_t SLOT = 512 << 10;
     char* p = nullptr;
     size_t bytes = 0;
     hipEvent_t ev[NS] = {};
+    std::mutex use;
     ~HostRing() { release(); }
     void release();
     hipError_t open(size_t want, bool events);

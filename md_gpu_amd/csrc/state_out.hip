@@ -126,6 +126,7 @@ hipError_t md_state_out(const StateOutArgs& a, float* const outs[3], HostRing& r
         p.narr += outs[k] != nullptr;
     }
     if (p.narr == 0 || a.natom < 1) return hipStreamSynchronize(st);
+    std::lock_guard<std::mutex> hold(ring.use);
     const size_t bytes = (size_t)a.natom * 12 * p.narr;
     const int most = (int)(HostRing::SLOT / (12 * p.narr)) & ~15;   // atoms of a chunk
     int slots = 1;

@@ -444,6 +444,33 @@ def test_download_edges(n, one_cpu):
     assert np.array_equal(only[0], pos) and np.array_equal(only[1], vel) and np.array_equal(only[2], f)
 
 
+@pytest.mark.parametrize("n", [3000, 60000])
+def test_downloads_from_several_threads(n):
+    """Threads that download one engine at the same time, one array, two or three (plans of different
+    sizes, on copying threads and without), each get the bits of a download alone."""
+    import threading
+    from md_gpu_amd.engine import Engine, _check, _ptr, lib
+    say("downloads from several threads", n)
+    e = Engine.from_system(lattice(n, 5))
+    want = e.download()
+    bad = []
+
+    def work(asked):
+        for _ in range(20):
+            out = [np.full((n, 3), np.nan, np.float32) if k in asked else None for k in range(3)]
+            _check(lib().md_download_state(e._h, *[None if x is None else _ptr(x) for x in out]))
+            if not all(np.array_equal(out[k], want[k]) for k in asked):
+                bad.append(asked)
+
+    threads = [threading.Thread(target=work, args=(a,)) for a in ((0, 1, 2), (0,), (1, 2), (2,))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    e.close()
+    assert not bad
+
+
 def stars(n, seed=3):
     """n molecules of a center with four bonds and four angles (the most an atom can have)."""
     m = max(6, int(np.ceil(n ** (1 / 3))))
